@@ -31,11 +31,15 @@ HBM_PEAK_GBS = 8000.0
 
 # kernel family behind each timed phase, and the algorithmic bytes per unit the
 # library's phase timers count (the per-launch figure is that times the units)
-PHASE_KERNEL = {"stage1": "owm::k_stage1", "leaf_aggs": "owm::k_leaf_aggs",
+PHASE_KERNEL = {"grid_partition": "owm::k_grid_part", "grid_bins": "owm::k_grid_bin",
+                "grid_windows": "owm::k_grid_windows", "stage1": "owm::k_stage1", "leaf_aggs": "owm::k_leaf_aggs",
                 "sort_tree_pass": "owm::k_sort_records", "morton": "owm::k_morton",
                 "bbox": "owm::k_bbox", "agg_levels": "owm::k_agg_levels",
                 "stage1_join": "owm::k_s1_bin+k_scan_excl"}
-PHASE_BYTES = {"stage1": "24 B x N x Wsize/Displace + 4 B x windows",
+PHASE_BYTES = {"grid_partition": "36 B x N (x, y, z read; a z key and a cell word written)",
+               "grid_bins": "12 B x N + 16 B x grid cells",
+               "grid_windows": "16 B x grid cells + 8 B x windows",
+               "stage1": "24 B x N x Wsize/Displace + 4 B x windows",
                "leaf_aggs": "32 B x N + 48 B x leaves",
                "sort_tree_pass": "56 B x N for the first pass (x, y, z read; a 32-byte point written), 64 B x N for later passes (a 32-byte point read and written)",
                "morton": "16 B x N", "bbox": "16 B x N", "agg_levels": "48 B x (leaves + level entries)",
@@ -174,7 +178,8 @@ def cpu_window_split(x, y, z, gpu_phases, factors=(0.02, 0.05, 0.1), reps=3):
     t0 = time.perf_counter()
     tree = pyoracle.Tree(x, y, z, p)
     t_tree = time.perf_counter() - t0
-    gpu_ms = sum(gpu_phases[k]["ms_per_step"] for k in ("stage1", "stage1_join") if k in gpu_phases)
+    gpu_ms = sum(gpu_phases[k]["ms_per_step"] for k in ("grid_bins", "grid_windows", "stage1", "stage1_join")
+                 if k in gpu_phases)
     rows = []
     for f in factors:
         cols = max(1, int(round(f * p.ncols)))
@@ -290,7 +295,9 @@ def run_headline(ctx, torch, synth, args):
     full = ctx.profile_read()
     ctx.profile(False)
     dname = max((k for k in full if full[k]["calls"]), key=lambda k: full[k]["ms"])
-    ev_phases = sorted({dname, "sort_tree_pass"})
+    # the pass that puts the points in spatial order, whichever chain ran
+    order = "grid_partition" if full["grid_partition"]["calls"] else "sort_tree_pass"
+    ev_phases = sorted({dname, order})
     ctx.profile(True, phases=ev_phases)
     log(f"timing {args.steps} batched steps (events on {', '.join(ev_phases)})")
     # a step ends with the seeds in host memory as the C ABI returns them (one
@@ -305,7 +312,7 @@ def run_headline(ctx, torch, synth, args):
     ctx.profile(False)
     ms = (t1 - t0) / args.steps * 1e3
     roofline = roofline_of(prof, dname, args.steps, n_total, TRAFFIC_BATCH)
-    roofline_sort = roofline_of(prof, "sort_tree_pass", args.steps, n_total, TRAFFIC_BATCH)
+    roofline_sort = roofline_of(prof, order, args.steps, n_total, TRAFFIC_BATCH)
     if args.save_tune_table:
         with open(args.save_tune_table, "w") as f:
             json.dump(table, f, indent=1)

@@ -86,6 +86,8 @@ owm_status owm_ctx_create(int device, uint64_t hbm_budget_bytes, owm_ctx **out)
         return OWM_E_DEVICE;
     if (hipSetDevice(device) != hipSuccess)
         return OWM_E_DEVICE;
+    if (owm::grid_kernels_init() != hipSuccess)
+        return OWM_E_DEVICE;
     owm_ctx *c = new owm_ctx();
     c->device = device;
     resolve_scratch(device);
@@ -705,11 +707,11 @@ owm_status owm_tree_run(owm_ctx *ctx, owm_tree *tree, const owm_params *params, 
     uint64_t need = 0;
     owm_status st = tree_query(ctx, tree, params, 1, 4, nullptr, 0, P, qo);
     if (st == OWM_OK)
-        st = read_seeds(ctx, qo, P, seeds, cap, off, &need);
+        st = read_seeds(ctx, qo, (uint32_t)P.td.size(), seeds, cap, off, &need);
     if (st == OWM_OK && need) {
         st = tree_query(ctx, tree, params, 1, 4, nullptr, 0, P, qo, need + need / 8 + 1024);
         if (st == OWM_OK)
-            st = read_seeds(ctx, qo, P, seeds, cap, off, &need);
+            st = read_seeds(ctx, qo, (uint32_t)P.td.size(), seeds, cap, off, &need);
         if (st == OWM_OK && need) {
             set_err(ctx, "stage-1 join list overflow persisted");
             st = OWM_E_INTERNAL;

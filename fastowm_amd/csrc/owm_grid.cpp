@@ -1,0 +1,432 @@
+// Host side of the column-grid chain (grid.hip): whole runs of tiles whose
+// trees nobody keeps.  Plans each tile's column grid (owm_axis.h), buckets and
+// work items, enqueues the chain and reads the seeds back.  Calls that it does
+// not take go on to the tree chain (run_batch), with the boxes it took.
+#include "owm_host.h"
+
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
+#include <cstring>
+
+namespace owm {
+
+static inline uint64_t up256(uint64_t v) { return (v + 255) / 256 * 256; }
+
+// The plan of one call: the device table and its totals.  Entries are ordered
+// by the size class of their buckets' cells, so that each class is one launch
+// of the bins with LDS for its own largest bucket.
+struct GridPlan {
+    std::vector<GridTile> t;
+    std::vector<uint32_t> st_off, item_off, blk_off, gcell_off;
+    std::vector<uint32_t> pt_off;  // caller's tile order
+    struct Class {
+        uint32_t t0, t1, cells;
+    };
+    std::vector<Class> cls;
+    uint64_t np = 0, cells = 0, tab = 0, nwin = 0, nleaf = 0, pool_cap = 0;
+    uint32_t max_nb = 1, rows_cap = 32;
+};
+
+// Bucket cells up to which tiles share a launch of the bins: the LDS of the
+// largest bucket of a launch bounds the workgroups per CU for all of them.
+static int cell_class(uint32_t cells) { return cells <= 1024 ? 0 : cells <= 4096 ? 1 : 2; }
+
+// Fills one tile's grid; false when the chain does not take it.
+static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64_t n)
+{
+    memset(&T, 0, sizeof T);
+    T.n = (uint32_t)n;
+    // the integer products of stage 3's centres must not wrap
+    if (D.width >= 1e9 || D.height >= 1e9 || !D.ncols || !D.nrows)
+        return false;
+    const double hd = (double)(float)D.h, hb = (double)(float)D.hb;
+    const double init[2] = {D.initx, D.inity}, initg[2] = {D.initxg, D.inityg};
+    const uint32_t nw[2] = {D.ncols, D.nrows}, ng[2] = {D.ncolsg, D.nrowsg};
+    for (int a = 0; a < 2; ++a) {
+        grid_edges(T.ax[a].w, init[a], D.displace, hd, nw[a], false, 64);
+        grid_edges(T.ax[a].g, initg[a], P.bsize ? (double)P.bsize : 1.0, hb, ng[a], true, 1);
+        grid_axis(T.ax[a]);
+    }
+    T.min_num_points = D.min_num_points;
+    T.stage2_need = P.overlap != 0.0 ? 2u : 1u;
+    // buckets: the smallest power-of-two rectangle of cells that leaves at
+    // most this many of them (about two sort tiles of points each)
+    const uint32_t cx = T.ax[0].ncol, cy = T.ax[1].ncol;
+    auto buckets = [&](uint32_t lw, uint32_t lh) {
+        return ((uint64_t)(cx - 1) / (1u << lw) + 1) * ((uint64_t)(cy - 1) / (1u << lh) + 1);
+    };
+    const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(n / 8192, 16), 1024);
+    uint32_t lw = 3, lh = 3;
+    while (buckets(lw, lh) > want && lw + lh < 12)
+        (lw <= lh ? lw : lh) += 1;
+    if (buckets(lw, lh) > GRID_MAX_BUCKETS)
+        ++lw;
+    if (buckets(lw, lh) > GRID_MAX_BUCKETS)
+        return false;
+    T.lw = lw;
+    T.lh = lh;
+    T.nbx = (cx - 1) / (1u << lw) + 1;
+    T.nby = (cy - 1) / (1u << lh) + 1;
+    T.nb = T.nbx * T.nby;
+    T.nst = (uint32_t)((n + GRID_PTS - 1) / GRID_PTS);
+    const uint64_t mean = n / T.nb;
+    T.split = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(mean / 32768, 1), 16);
+    const double run = T.nst ? (double)n / ((double)T.nst * T.nb) : 1.0;
+    T.lpr = run <= 8 ? 2 : run <= 20 ? 3 : run <= 48 ? 4 : run <= 128 ? 5 : 6;
+    // window blocks, and the rows of cells that one spans
+    T.lbw = T.ax[0].w.pair && T.ax[1].w.pair ? 5 : 4;
+    return true;
+}
+
+// An upper bound on the rows of cells under bw windows.
+static double rows_of(const GridAxis &A, uint32_t bw)
+{
+    const double len = (bw - 1) * A.w.step + 2.0 * A.w.half;
+    double r = (len * A.w.inv + 1.0) * (A.w.pair ? 1.0 : 2.0);
+    if (A.g.n)
+        r += (len * A.g.inv + 1.0) * (A.g.pair ? 1.0 : 2.0);
+    return r + 4.0;
+}
+
+// An upper bound on the tree chain's device memory for the same call: a call
+// that might not fit the budget there keeps that chain's answer.
+static uint64_t tree_chain_bound(const GridPlan &P)
+{
+    return P.np * 112 + P.nleaf * 1000 + P.nwin * 32 + (64ull << 20);
+}
+
+static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
+                      const std::vector<std::array<double, 4>> &box, GridPlan &P)
+{
+    std::vector<GridTile> raw(n_tiles);
+    P.pt_off.assign(n_tiles + 1, 0);
+    for (uint32_t t = 0; t < n_tiles; ++t) {
+        Derived D;
+        std::string why;
+        if (derive_params(tiles[t].params, tiles[t].n, box[t].data(), D, why) != OWM_OK)
+            return false;  // the tree chain reports it
+        if (!plan_tile(raw[t], tiles[t].params, D, tiles[t].n))
+            return false;
+        raw[t].pt_off = P.pt_off[t];
+        P.pt_off[t + 1] = P.pt_off[t] + (uint32_t)tiles[t].n;
+        P.nwin += (uint64_t)D.ncols * D.nrows;
+        P.nleaf += tiles[t].n / std::max(pick_leaf(ctx, tiles[t].n, 0), 1u) + 1;
+    }
+    P.np = P.pt_off[n_tiles];
+    // 32x32-window blocks where there are enough of them to occupy the device
+    uint64_t big = 0;
+    for (const GridTile &T : raw)
+        big += ((T.ax[0].w.n + 31ull) / 32) * ((T.ax[1].w.n + 31ull) / 32);
+    double rows = 32.0;
+    for (GridTile &T : raw) {
+        if (big < 512)
+            T.lbw = 4;
+        double r = std::max(rows_of(T.ax[0], 1u << T.lbw), rows_of(T.ax[1], 1u << T.lbw));
+        if (T.lbw == 5 && r > 64.0) {
+            T.lbw = 4;
+            r = std::max(rows_of(T.ax[0], 16), rows_of(T.ax[1], 16));
+        }
+        rows = std::max(rows, std::ceil(r) * (double)(1u << T.lbw) / 32.0);
+    }
+    if (rows > 96.0)
+        return false;  // 48 KB of row sums; longer windows stay with the tree chain
+    P.rows_cap = (uint32_t)std::ceil(rows);
+    for (int c = 0; c < 3; ++c) {
+        const uint32_t t0 = (uint32_t)P.t.size();
+        uint32_t cells = 0;
+        for (const GridTile &T : raw)
+            if (cell_class(1u << (T.lw + T.lh)) == c) {
+                P.t.push_back(T);
+                cells = std::max(cells, 1u << (T.lw + T.lh));
+            }
+        if (P.t.size() > t0)
+            P.cls.push_back({t0, (uint32_t)P.t.size(), cells});
+    }
+    P.st_off.assign(n_tiles + 1, 0);
+    P.item_off.assign(n_tiles + 1, 0);
+    P.blk_off.assign(n_tiles + 1, 0);
+    P.gcell_off.assign(n_tiles + 1, 0);
+    uint64_t st = 0, items = 0, blk = 0, gc = 0;
+    for (uint32_t t = 0; t < n_tiles; ++t) {
+        GridTile &T = P.t[t];
+        T.st_off = (uint32_t)st;
+        T.item_off = (uint32_t)items;
+        T.blk_off = (uint32_t)blk;
+        T.gcell_off = (uint32_t)gc;
+        T.tab_off = P.tab;
+        T.cell_off = P.cells;
+        T.nblkx = ((T.ax[0].w.n - 1) >> T.lbw) + 1;
+        st += T.nst;
+        items += (uint64_t)T.nb * T.split;
+        blk += (uint64_t)T.nblkx * (((T.ax[1].w.n - 1) >> T.lbw) + 1);
+        gc += (uint64_t)T.ax[0].g.n * T.ax[1].g.n;
+        P.tab += (uint64_t)T.nst * (T.nb + 1);
+        P.cells += (uint64_t)T.nb * T.split << (T.lw + T.lh);
+        if (items >= (1ull << 30) || blk >= (1ull << 30) || gc >= (1ull << 30))
+            return false;
+        P.st_off[t + 1] = (uint32_t)st;
+        P.item_off[t + 1] = (uint32_t)items;
+        P.blk_off[t + 1] = (uint32_t)blk;
+        P.gcell_off[t + 1] = (uint32_t)gc;
+        P.max_nb = std::max(P.max_nb, T.nb);
+    }
+    // a quarter of the points may lie on edges before the tree chain takes over
+    P.pool_cap = (P.np / 4 + 65536) / GRID_POOLS;
+    return true;
+}
+
+// Exact boxes of the tiles that come without one (device reduction).
+static owm_status take_boxes(owm_ctx *ctx, const double *dx, const double *dy,
+                             const owm_tile *tiles, uint32_t n_tiles,
+                             std::vector<std::array<double, 4>> &box)
+{
+    hipStream_t s = ctx->stream;
+    uint64_t np = 0;
+    for (uint32_t t = 0; t < n_tiles; ++t)
+        np += tiles[t].n;
+    const uint64_t bk_bytes = bbox_key_words(n_tiles) * 8, off_bytes = (n_tiles + 1) * 4ull;
+    owm_status st = ctx->small.ensure(ctx, up256(bk_bytes) + up256(off_bytes));
+    if (st != OWM_OK)
+        return st;
+    unsigned long long *bk = (unsigned long long *)ctx->small.take(bk_bytes);
+    uint32_t *ptoff = (uint32_t *)ctx->small.take(off_bytes);
+    uint8_t *h = ctx->pinned(ctx->h_io, ctx->h_io_cap, io_bytes(n_tiles));
+    if (!bk || !ptoff || !h) {
+        set_err(ctx, "pinned host allocation failed");
+        return OWM_E_NOMEM;
+    }
+    uint32_t *ho = (uint32_t *)h;
+    unsigned long long *hk = (unsigned long long *)(h + up256(off_bytes));
+    ho[0] = 0;
+    for (uint32_t t = 0; t < n_tiles; ++t)
+        ho[t + 1] = ho[t] + (uint32_t)tiles[t].n;
+    HIP_TRY(hipMemcpyAsync(ptoff, ho, off_bytes, hipMemcpyHostToDevice, s), "upload offsets");
+    BatchDev B{};
+    B.ntiles = n_tiles;
+    B.np = (uint32_t)np;
+    B.pt_off = ptoff;
+    launch_bbox_init(s, bk, n_tiles);
+    const int pi = ctx->prof.begin(s, PH_BBOX);
+    launch_bbox(s, B, dx, dy, bk);
+    ctx->prof.end(s, pi, 16ull * np, np);
+    HIP_TRY(hipMemcpyAsync(hk, bk, n_tiles * 32ull, hipMemcpyDeviceToHost, s), "bbox D2H");
+    HIP_TRY(hipStreamSynchronize(s), "bbox sync");
+    ctx->prof.collect();
+    auto dec = [](unsigned long long k) {
+        const uint64_t b = (k >> 63) ? (k & 0x7FFFFFFFFFFFFFFFull) : ~k;
+        double v;
+        memcpy(&v, &b, 8);
+        return v;
+    };
+    for (uint32_t t = 0; t < n_tiles; ++t) {
+        if (tiles[t].params.flags & OWM_F_HAVE_BBOX)
+            continue;
+        if (tiles[t].n == 0 || hk[4 * t] == ~0ull || hk[4 * t + 1] == ~0ull) {
+            set_err(ctx, "tile %u: no finite points to take a bbox from", t);
+            return OWM_E_ARG;
+        }
+        box[t] = {dec(hk[4 * t]), dec(hk[4 * t + 2]), dec(hk[4 * t + 1]), dec(hk[4 * t + 3])};
+    }
+    return OWM_OK;
+}
+
+// Everything the chain's launches depend on.
+static void plan_key(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
+                     const GridPlan &P, std::vector<uint8_t> &key)
+{
+    auto put = [&key](const void *p, size_t n) {
+        const uint8_t *b = (const uint8_t *)p;
+        key.insert(key.end(), b, b + n);
+    };
+    key.clear();
+    put("grid", 4);
+    const void *ptrs[4] = {dx, dy, dz, ctx->arena.buf.ptr};
+    put(ptrs, sizeof ptrs);
+    put(P.t.data(), P.t.size() * sizeof(GridTile));
+    put(P.pt_off.data(), P.pt_off.size() * 4);
+}
+
+owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
+                    const owm_tile *tiles, uint32_t n_tiles, uint32_t flags, uint32_t *seeds,
+                    uint64_t cap, uint64_t *seed_off_host, std::vector<owm_tile> &boxed,
+                    bool &handled)
+{
+    handled = false;
+    owm_status st = check_tiles(ctx, tiles, n_tiles);
+    if (st != OWM_OK)
+        return st;
+    uint64_t np = 0;
+    bool need_box = false;
+    std::vector<std::array<double, 4>> box(n_tiles);
+    for (uint32_t t = 0; t < n_tiles; ++t) {
+        if (tiles[t].params.leaf_size)
+            return OWM_OK;  // the caller asks for a tree with such leaves
+        if (tiles[t].offset != np)
+            return OWM_OK;  // the tree chain reports it
+        np += tiles[t].n;
+        if (tiles[t].params.flags & OWM_F_HAVE_BBOX)
+            memcpy(box[t].data(), tiles[t].params.bbox, sizeof(double) * 4);
+        else
+            need_box = true;
+    }
+    if (np == 0)
+        return OWM_OK;
+    if (need_box) {
+        st = take_boxes(ctx, dx, dy, tiles, n_tiles, box);
+        if (st != OWM_OK)
+            return st;
+    }
+    // what a call that is not taken hands on: its tiles with their boxes
+    auto hand_on = [&]() {
+        if (need_box) {
+            boxed.assign(tiles, tiles + n_tiles);
+            for (uint32_t t = 0; t < n_tiles; ++t) {
+                boxed[t].params.flags |= OWM_F_HAVE_BBOX;
+                memcpy(boxed[t].params.bbox, box[t].data(), sizeof(double) * 4);
+            }
+        }
+        return OWM_OK;
+    };
+    GridPlan P;
+    if (!make_plan(ctx, tiles, n_tiles, box, P))
+        return hand_on();
+    const uint32_t T = n_tiles;
+    const uint64_t nwords = (np + 31) / 32, items = P.item_off[T], gcells = P.gcell_off[T];
+    const uint64_t nseed = std::min<uint64_t>(np, P.nwin + gcells) + 1;
+    const uint64_t table = up256(T * sizeof(GridTile)) + 5 * up256((T + 1) * 4ull);
+    const uint64_t need = table + up256(np * 8) + up256(np * 4) + up256(P.tab * 2) +
+                          up256(P.cells * 16) + up256(items * 4) +
+                          up256(P.pool_cap * GRID_POOLS * sizeof(GridRare)) +
+                          up256(GRID_POOLS * 64) + 2 * up256((nwords + 4) * 4) +
+                          up256((gcells + 1) * 4) + up256((nwords / 4096 + 2) * 4) +
+                          up256(nseed * 4) + up256((T + 1) * 4ull) + 4096;
+    const uint64_t others = ctx->held_bytes() - ctx->arena.buf.bytes;
+    if (ctx->budget && others + std::max(need, tree_chain_bound(P)) > ctx->budget)
+        return hand_on();
+    void *old_arena = ctx->arena.buf.ptr;
+    st = ctx->arena.ensure(ctx, need);
+    if (st != OWM_OK)
+        return st;
+    if (ctx->arena.buf.ptr != old_arena)
+        ctx->graphs.clear();
+    handled = true;
+
+    Arena &A = ctx->arena;
+    hipStream_t s = ctx->stream;
+    bool graph = (flags & OWM_B_GRAPH) != 0;
+    std::vector<uint8_t> key;
+    if (graph || (flags & B_AUTO_GRAPH))
+        plan_key(ctx, dx, dy, dz, P, key);
+    if (!graph && (flags & B_AUTO_GRAPH)) {
+        graph = !ctx->prof.on && key == ctx->graphs.last_key;
+        ctx->graphs.last_key = key;
+    }
+    // table
+    uint8_t *d = A.take(table);
+    (void)hipStreamSynchronize(s);  // the previous upload from this buffer must have completed
+    uint8_t *h = ctx->pinned(ctx->h_tab, ctx->h_tab_cap, table);
+    if (!d || !h) {
+        set_err(ctx, "pinned host allocation failed");
+        return OWM_E_NOMEM;
+    }
+    GridDev G{};
+    G.ntiles = T;
+    G.ngcell = (uint32_t)gcells;
+    G.tiles = (const GridTile *)d;
+    memcpy(h, P.t.data(), T * sizeof(GridTile));
+    const std::vector<uint32_t> *src[5] = {&P.st_off, &P.item_off, &P.blk_off, &P.gcell_off,
+                                           &P.pt_off};
+    const uint32_t *off[5];
+    uint64_t o = up256(T * sizeof(GridTile));
+    for (int k = 0; k < 5; ++k, o += up256((T + 1) * 4ull)) {
+        memcpy(h + o, src[k]->data(), (T + 1) * 4ull);
+        off[k] = (const uint32_t *)(d + o);
+    }
+    G.st_off = off[0];
+    G.item_off = off[1];
+    G.blk_off = off[2];
+    G.gcell_off = off[3];
+    BatchDev B{};
+    B.ntiles = T;
+    B.np = (uint32_t)np;
+    B.pt_off = off[4];
+    HIP_TRY(hipMemcpyAsync(d, h, table, hipMemcpyHostToDevice, s), "upload table");
+
+    QueryOut qo;
+    auto body = [&]() -> owm_status {
+        G.zk = (unsigned long long *)A.take(np * 8);
+        G.cw = (uint32_t *)A.take(np * 4);
+        G.tab = (uint16_t *)A.take(P.tab * 2);
+        G.cells = (uint4 *)A.take(P.cells * 16);
+        G.heads = (uint32_t *)A.take(items * 4);
+        G.pool = (GridRare *)A.take(P.pool_cap * GRID_POOLS * sizeof(GridRare));
+        G.pool_cap = (uint32_t)P.pool_cap;
+        G.pool_used = (uint32_t *)A.take(GRID_POOLS * 64);
+        G.seen = (uint32_t *)A.take((nwords + 4) * 4);
+        G.llp = (uint32_t *)A.take((nwords + 4) * 4);
+        G.cell_flag = (uint32_t *)A.take((gcells + 1) * 4);
+        uint32_t *lookback = (uint32_t *)A.take((nwords / 4096 + 2) * 4);
+        uint32_t *out = (uint32_t *)A.take(nseed * 4);
+        uint32_t *seed_off = (uint32_t *)A.take((T + 1) * 4ull);
+        uint32_t *cnt = (uint32_t *)A.take(1024);
+        if (!cnt) {
+            set_err(ctx, "scratch arena exhausted (grid)");
+            return OWM_E_INTERNAL;
+        }
+        G.err = cnt + 3;
+        FillRanges z;
+        auto zero = [&](uint32_t *p, uint64_t words) {
+            z.ptr[z.count] = p;
+            z.len[z.count++] = words;
+        };
+        zero(cnt, 16);
+        zero(G.pool_used, GRID_POOLS * 16);
+        zero(G.seen, nwords + 4);
+        zero(G.llp, nwords + 4);
+        zero(G.cell_flag, gcells + 1);
+        zero(lookback, nwords / 4096 + 2);
+        launch_fill_ranges(s, z);
+        int pi = ctx->prof.begin(s, PH_GRID_PART);
+        launch_grid_part(s, G, dx, dy, dz, P.st_off[T], P.max_nb);
+        // x, y and z read; a z key and a word written
+        ctx->prof.end(s, pi, 36ull * np, np);
+        pi = ctx->prof.begin(s, PH_GRID_BIN);
+        for (const GridPlan::Class &c : P.cls)
+            launch_grid_bin(s, G, dx, dy, dz, c.t0, c.t1, P.item_off[c.t0],
+                            P.item_off[c.t1] - P.item_off[c.t0], c.cells);
+        ctx->prof.end(s, pi, 12ull * np + 16ull * P.cells, np, (uint32_t)P.cls.size());
+        pi = ctx->prof.begin(s, PH_GRID_WIN);
+        launch_grid_windows(s, G, dx, dy, P.blk_off[T], P.rows_cap);
+        ctx->prof.end(s, pi, 16ull * P.cells + 8ull * P.nwin, P.nwin);
+        if (gcells) {
+            pi = ctx->prof.begin(s, PH_STAGE3);
+            launch_grid_cells(s, G);
+            ctx->prof.end(s, pi, 12ull * gcells, gcells);
+        }
+        pi = ctx->prof.begin(s, PH_MERGE);
+        launch_bits_compact(s, G.llp, (uint32_t)nwords, out, cnt + 2, lookback, cnt + 7);
+        ctx->prof.end(s, pi, 4ull * nwords, nwords);
+        launch_seed_ranges(s, B, out, cnt + 2, seed_off);
+        launch_seeds_local(s, B, out, cnt + 2, (uint32_t)nseed);
+        HIP_TRY(hipGetLastError(), "grid chain launch");
+        qo.cnt = cnt;
+        qo.seed_off = seed_off;
+        qo.seeds = out;
+        return OWM_OK;
+    };
+    st = run_chain(ctx, graph, std::move(key), A, qo, body);
+    if (st != OWM_OK)
+        return st;
+    uint32_t err = 0;
+    st = read_seeds(ctx, qo, n_tiles, seeds, cap, seed_off_host, nullptr, &err);
+    if (st != OWM_OK)
+        return st;
+    if (err & GRID_ERR_POOL) {
+        handled = false;
+        return hand_on();
+    }
+    return OWM_OK;
+}
+
+}  // namespace owm

@@ -82,7 +82,7 @@ struct IoLayout {
 static const char *PHASE_NAMES[PH_COUNT] = {
     "bbox", "morton", "sort_tree_pass", "leaf_aggs", "karras", "agg_levels", "stage1",
     "stage2_mark", "stage2_compact", "stage3", "merge_seeds", "stage1_join",
-    "stage1_summaries", "xyz_parse", "qtree_stats"};
+    "stage1_summaries", "xyz_parse", "qtree_stats", "grid_partition", "grid_bins", "grid_windows"};
 
 const char *phase_name(int ph) { return PHASE_NAMES[ph]; }
 
@@ -869,7 +869,7 @@ owm_status Arena::ensure(owm_ctx *ctx, uint64_t bytes)
 
 // -------------------------------------------------------------- batches --
 
-static owm_status check_tiles(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles)
+owm_status check_tiles(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles)
 {
     if (n_tiles == 0) {
         set_err(ctx, "n_tiles must be > 0");
@@ -1203,12 +1203,11 @@ owm_status check_guards(owm_ctx *ctx, const uint32_t *hc, uint64_t *s1_needed)
     return OWM_OK;
 }
 
-owm_status read_seeds(owm_ctx *ctx, const QueryOut &qo, const Prepared &P, uint32_t *seeds,
+owm_status read_seeds(owm_ctx *ctx, const QueryOut &qo, uint32_t n_tiles, uint32_t *seeds,
                       uint64_t cap, uint64_t *seed_off_host, uint64_t *s1_needed,
-                      const RunMem *mem)
+                      uint32_t *pool_full, const RunMem *mem)
 {
     hipStream_t s = ctx->stream;
-    const uint32_t n_tiles = (uint32_t)P.td.size();
     const IoLayout io(n_tiles);
     uint8_t *h = mem ? mem->h_io : ctx->pinned(ctx->h_io, ctx->h_io_cap, io.bytes);
     if (!h) {
@@ -1222,8 +1221,17 @@ owm_status read_seeds(owm_ctx *ctx, const QueryOut &qo, const Prepared &P, uint3
             "ranges D2H");
     HIP_TRY(hipStreamSynchronize(s), "pipeline");
     ctx->prof.collect();
-    owm_status st = check_guards(ctx, hc, s1_needed);
-    if (st != OWM_OK || *s1_needed)
+    if (pool_full) {
+        // the column-grid chain: its only recoverable flag ends the read
+        *pool_full = hc[3] & GRID_ERR_POOL;
+        if (*pool_full)
+            return OWM_OK;
+    }
+    uint64_t need = 0;
+    owm_status st = check_guards(ctx, hc, &need);
+    if (s1_needed)
+        *s1_needed = need;
+    if (st != OWM_OK || need)
         return st;
     const uint64_t ns = hc[2];
     for (uint32_t t = 0; t <= n_tiles; ++t)
@@ -1270,35 +1278,14 @@ void GraphCache::clear()
     last_key.clear();
 }
 
-// Enqueues (or replays) the device chain of a batch: guard reset, tree build,
-// stages 1-3 and the merge.  With a graph, the chain is captured on first use
-// and replayed while its key matches.
-static owm_status enqueue_chain(owm_ctx *ctx, bool graph, const double *dx, const double *dy,
-                                const double *dz, Prepared &P, BatchDev &B, TreeOut &T,
-                                uint32_t *guard, QueryOut &qo, const RunMem *mem = nullptr)
+// Enqueues a chain (body), or replays it from the graph captured for its key.
+owm_status run_chain(owm_ctx *ctx, bool graph, std::vector<uint8_t> key, Arena &A, QueryOut &qo,
+                     const std::function<owm_status()> &body)
 {
     hipStream_t s = ctx->stream;
-    Arena &A = mem ? *mem->arena : ctx->arena;
-    auto body = [&]() -> owm_status {
-        // build_tree zeroes the guard with its own scratch
-        owm_status st = build_tree(ctx, s, P.L, B, dx, dy, dz, T, A, guard);
-        if (st != OWM_OK)
-            return st;
-        TreeDev TV = tree_view(T);
-        TV.X = dx;
-        TV.Y = dy;
-        st = enqueue_query(ctx, s, B, TV, P.Q, P.L.np, P.cfg, P.any_need1 ? 1u : 0u, A, qo, 1, 4,
-                           nullptr, 0, mem);
-        if (st != OWM_OK)
-            return st;
-        launch_add_u32(s, qo.cnt + 3, guard, qo.cnt + 3);
-        return OWM_OK;
-    };
     if (!graph)
         return body();
     GraphCache &G = ctx->graphs;
-    std::vector<uint8_t> key;
-    graph_key(ctx, dx, dy, dz, P, key);
     for (size_t i = 0; i < G.slots.size(); ++i)
         if (G.slots[i].key == key) {
             GraphCache::Slot hit = std::move(G.slots[i]);
@@ -1351,6 +1338,36 @@ static owm_status enqueue_chain(owm_ctx *ctx, bool graph, const double *dx, cons
     return OWM_OK;
 }
 
+// Enqueues (or replays) the device chain of a batch: guard reset, tree build,
+// stages 1-3 and the merge.  With a graph, the chain is captured on first use
+// and replayed while its key matches.
+static owm_status enqueue_chain(owm_ctx *ctx, bool graph, const double *dx, const double *dy,
+                                const double *dz, Prepared &P, BatchDev &B, TreeOut &T,
+                                uint32_t *guard, QueryOut &qo, const RunMem *mem = nullptr)
+{
+    hipStream_t s = ctx->stream;
+    Arena &A = mem ? *mem->arena : ctx->arena;
+    auto body = [&]() -> owm_status {
+        // build_tree zeroes the guard with its own scratch
+        owm_status st = build_tree(ctx, s, P.L, B, dx, dy, dz, T, A, guard);
+        if (st != OWM_OK)
+            return st;
+        TreeDev TV = tree_view(T);
+        TV.X = dx;
+        TV.Y = dy;
+        st = enqueue_query(ctx, s, B, TV, P.Q, P.L.np, P.cfg, P.any_need1 ? 1u : 0u, A, qo, 1, 4,
+                           nullptr, 0, mem);
+        if (st != OWM_OK)
+            return st;
+        launch_add_u32(s, qo.cnt + 3, guard, qo.cnt + 3);
+        return OWM_OK;
+    };
+    std::vector<uint8_t> key;
+    if (graph)
+        graph_key(ctx, dx, dy, dz, P, key);
+    return run_chain(ctx, graph, std::move(key), A, qo, body);
+}
+
 // Runs the whole pipeline on a batch whose points are in device memory
 // (concatenated SoA).  seeds/seed_off_host receive tile-local ids.  With
 // OWM_B_GRAPH the device chain is captured once per batch layout and replayed.
@@ -1358,8 +1375,19 @@ owm_status run_batch(owm_ctx *ctx, const double *dx, const double *dy, const dou
                      const owm_tile *tiles, uint32_t n_tiles, uint32_t flags, uint32_t *seeds,
                      uint64_t cap, uint64_t *seed_off_host)
 {
+    owm_status st;
+    std::vector<owm_tile> boxed;  // the tiles with the boxes the grid chain took
+    if (!ctx->tuner.forced && !getenv("OWM_NO_GRID")) {
+        bool done = false;
+        st = run_grid(ctx, dx, dy, dz, tiles, n_tiles, flags, seeds, cap, seed_off_host, boxed,
+                      done);
+        if (st != OWM_OK || done)
+            return st;
+        if (!boxed.empty())
+            tiles = boxed.data();
+    }
     Prepared P;
-    owm_status st = prepare_tree(ctx, dx, dy, tiles, n_tiles, P);
+    st = prepare_tree(ctx, dx, dy, tiles, n_tiles, P);
     if (st != OWM_OK)
         return st;
     st = prepare_query(ctx, &tiles[0].params, sizeof(owm_tile), P.box, P.L.np, P);
@@ -1403,7 +1431,7 @@ owm_status run_batch(owm_ctx *ctx, const double *dx, const double *dy, const dou
         if (st != OWM_OK)
             return st;
         uint64_t s1_need = 0;
-        st = read_seeds(ctx, qo, P, seeds, cap, seed_off_host, &s1_need);
+        st = read_seeds(ctx, qo, n_tiles, seeds, cap, seed_off_host, &s1_need);
         if (st != OWM_OK || s1_need == 0)
             return st;
         if (attempt > 0) {
@@ -1481,7 +1509,7 @@ owm_status run_tile_fixed(owm_ctx *ctx, const double *dx, const double *dy, cons
         if (st != OWM_OK)
             return st;
         uint64_t s1_need = 0, off[2] = {0, 0};
-        st = read_seeds(ctx, qo, P, seeds, cap, off, &s1_need, &mem);
+        st = read_seeds(ctx, qo, 1, seeds, cap, off, &s1_need, nullptr, &mem);
         *n_seeds = off[1];
         if (st != OWM_OK || s1_need == 0)
             return st;

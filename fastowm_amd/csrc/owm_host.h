@@ -4,6 +4,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <deque>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -195,9 +196,22 @@ owm_status prepare_query(owm_ctx *ctx, const owm_params *params, uint32_t stride
                          Prepared &P);
 owm_status upload_table(owm_ctx *ctx, Arena &A, const Prepared &P, BatchDev &B,
                         const RunMem *mem = nullptr);
-owm_status read_seeds(owm_ctx *ctx, const QueryOut &qo, const Prepared &P, uint32_t *seeds,
+// Reads the counts, checks the device guards, copies the seeds (tile-local).
+// pool_full (column-grid chain): set, with nothing copied, when the chain's pool
+// was full.
+owm_status read_seeds(owm_ctx *ctx, const QueryOut &qo, uint32_t n_tiles, uint32_t *seeds,
                       uint64_t cap, uint64_t *seed_off_host, uint64_t *s1_needed,
-                      const RunMem *mem = nullptr);
+                      uint32_t *pool_full = nullptr, const RunMem *mem = nullptr);
+owm_status check_tiles(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles);
+owm_status run_chain(owm_ctx *ctx, bool graph, std::vector<uint8_t> key, Arena &A, QueryOut &qo,
+                     const std::function<owm_status()> &body);
+// The whole pipeline by the column-grid chain (owm_grid.cpp).  handled: it
+// answered; else (with OWM_OK) the caller runs the tree chain, on `boxed` when
+// that is not empty.
+owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
+                    const owm_tile *tiles, uint32_t n_tiles, uint32_t flags, uint32_t *seeds,
+                    uint64_t cap, uint64_t *seed_off_host, std::vector<owm_tile> &boxed,
+                    bool &handled);
 // Host bytes of the readback and table staging of an n_tiles batch.
 uint64_t io_bytes(uint32_t n_tiles);
 // Writes the tile table (tiles, then the eight offset arrays, in the device
@@ -244,7 +258,8 @@ struct ServeState;
 
 enum Phase {
     PH_BBOX, PH_MORTON, PH_SORT_TREE, PH_LEAVES, PH_KARRAS, PH_LEVELS, PH_STAGE1,
-    PH_S2_MARK, PH_STAGE2, PH_STAGE3, PH_MERGE, PH_S1_JOIN, PH_LCS, PH_XYZ, PH_QSTATS, PH_COUNT
+    PH_S2_MARK, PH_STAGE2, PH_STAGE3, PH_MERGE, PH_S1_JOIN, PH_LCS, PH_XYZ, PH_QSTATS,
+    PH_GRID_PART, PH_GRID_BIN, PH_GRID_WIN, PH_COUNT
 };
 
 const char *phase_name(int ph);

@@ -1,6 +1,7 @@
 // Host-side launchers of the OWM kernels (one translation unit per kernel
 // family; every launcher enqueues on the given stream and never synchronises).
 #pragma once
+#include "owm_axis.h"
 #include "owm_dev.h"
 
 namespace owm {
@@ -114,6 +115,76 @@ void launch_agg_levels(hipStream_t s, const TreeOut &T, const AggLevels &V);
 // Karras tree over each tile's leaves; every node's aggregate is merged from
 // the levels' blocks that tile its leaf range (levels built first).
 void launch_karras(hipStream_t s, const BatchDev &B, const TreeOut &T, const AggLevels &V);
+
+// ---- column grid (grid.hip) ----
+// Points per sort tile of the partition, and the packed (cell, slot) word: a
+// point's cell within its bucket above its slot within the sort tile.
+constexpr uint32_t GRID_SLOT_BITS = 12, GRID_PTS = 1u << GRID_SLOT_BITS;
+constexpr uint32_t GRID_SLOT_MASK = GRID_PTS - 1u;
+constexpr uint32_t GRID_CELL_BITS = 13, GRID_MAX_CELLS = 1u << GRID_CELL_BITS;
+constexpr uint32_t GRID_CELL_MASK = GRID_MAX_CELLS - 1u;
+constexpr uint32_t GRID_MAX_BUCKETS = 8192;
+constexpr uint32_t GRID_POOLS = 64;  // shares of the pool, each with a cursor of its own
+// bits of *err: the pool of points without a column is full; a window block
+// has more rows than planned (cannot happen)
+constexpr uint32_t GRID_ERR_POOL = 32u, GRID_ERR_ROWS = 64u;
+
+// A point without a column (on an edge, or between the edges of a pair) with
+// the windows [wx0, wx1) x [wy0, wy1) and stage-3 cells [gx0, gx1) x [gy0, gy1)
+// that hold it.  The first entry of each block of the pool is its header: id
+// the entries that follow, next the bucket's next block.
+struct GridRare {
+    unsigned long long zk;
+    uint32_t id, next;
+    uint16_t wx0, wx1, wy0, wy1, gx0, gx1, gy0, gy1;
+};
+
+// Per-tile description of the column-grid chain (device table).
+struct GridTile {
+    GridAxis ax[2];
+    uint64_t tab_off;   // first run-start entry: [nst][nb + 1]
+    uint64_t cell_off;  // first grid cell: [nb][split][2^(lw + lh)]
+    uint32_t pt_off, n;
+    uint32_t st_off, nst;        // sort tiles
+    uint32_t lw, lh;             // a bucket is 2^lw columns x 2^lh rows
+    uint32_t nbx, nby, nb;       // buckets
+    uint32_t split, item_off;    // items: each bucket's sort tiles in `split` shares
+    uint32_t lpr;                // lanes per run segment (log2) of the bins
+    uint32_t lbw, nblkx, blk_off;  // window blocks of 2^lbw x 2^lbw
+    uint32_t gcell_off;          // first stage-3 cell
+    uint32_t min_num_points, stage2_need;
+};
+
+struct GridDev {
+    uint32_t ntiles, ngcell;
+    const GridTile *tiles;
+    const uint32_t *st_off, *item_off, *blk_off, *gcell_off;  // [ntiles + 1] each
+    unsigned long long *zk;  // [np] z keys, grouped by bucket within each sort tile
+    uint32_t *cw;            // [np] cell << GRID_SLOT_BITS | slot (bit 31: no column)
+    uint16_t *tab;           // run starts per sort tile and bucket
+    uint4 *cells;            // {z key, id, count} per grid cell
+    uint32_t *heads;         // [items] first pool block of the item's listed points
+    GridRare *pool;
+    uint32_t *pool_used;     // [GRID_POOLS * 16] entries used of each share (one per 64 bytes)
+    uint32_t pool_cap;       // entries per share
+    uint32_t *seen, *llp;    // point bitmaps: one window, two (LLPs, then seeds)
+    uint32_t *cell_flag;     // [ngcell] stage-3 cells that hold an LLP
+    uint32_t *err;
+};
+
+// Raises the kernels' LDS limits; once per device.
+hipError_t grid_kernels_init();
+void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const double *y,
+                      const double *z, uint32_t sort_tiles, uint32_t max_nb);
+// Items [item0, item0 + items) of the table entries [t0, t1); cells: the
+// largest bucket's.
+void launch_grid_bin(hipStream_t s, const GridDev &G, const double *x, const double *y,
+                     const double *z, uint32_t t0, uint32_t t1, uint32_t item0, uint32_t items,
+                     uint32_t cells);
+// rows_cap * 32 row sums of LDS (rows_cap >= 32)
+void launch_grid_windows(hipStream_t s, const GridDev &G, const double *x, const double *y,
+                         uint32_t blocks, uint32_t rows_cap);
+void launch_grid_cells(hipStream_t s, const GridDev &G);
 
 // ---- .xyz reader (xyz.hip) ----
 // The text buffer is zero-padded to a whole number of xyz_chunk_bytes() plus

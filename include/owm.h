@@ -46,7 +46,10 @@ typedef struct owm_params {
     uint32_t wsize;     /* sliding-window side in metres (u32, as the reference) */
     uint32_t bsize;     /* stage-3 grid cell side in metres; 0 skips stage 3 */
     double overlap;     /* window overlap ratio, 0 <= overlap < 1 */
-    uint32_t leaf_size; /* maxNumber points per tree leaf; 0 = autotuned */
+    /* maxNumber points per tree leaf; 0 = the library's choice: whole runs
+     * (owm_run_tile*, batches, unkeyed serving) then build no tree where the
+     * column-grid chain takes the call, and resident trees take the tuned size */
+    uint32_t leaf_size;
     uint32_t flags;     /* OWM_F_* */
     double bbox[4];     /* minx, maxx, miny, maxy when OWM_F_HAVE_BBOX */
 } owm_params;

@@ -1,0 +1,139 @@
+"""Whole runs by the column-grid chain (leaf_size 0) against the oracle, at the
+sizes where it can go wrong: the edges of sort tiles, buckets of one cell row,
+shares of large buckets, points on and within ulps of window and cell edges,
+more points without a column than the chain's pool holds, and parameters it
+hands to the tree chain.  Seeds are ids: equal or wrong."""
+import numpy as np
+import pytest
+
+import pyoracle as O
+from fastowm_amd import owm, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print("[case]", *a, flush=True)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with owm.Context(0) as c:
+        yield c
+
+
+def _run(ctx, x, y, z, ws, bs, ov, phase=True):
+    want, _, _ = O.run(x, y, z, ws, bs, ov, 32)
+    ctx.profile(True)
+    got = ctx.run_tile(x, y, z, ws, bs, ov)
+    calls = ctx.profile_read()
+    ctx.profile(False)
+    assert (calls["grid_partition"]["calls"] > 0) == phase
+    assert np.array_equal(got, want), (len(got), len(want))
+    assert np.array_equal(ctx.run_tile(x, y, z, ws, bs, ov), want)  # again: nothing left over
+    return want
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 4095, 4096, 4097, 8192, 12289, 70_001])
+@pytest.mark.parametrize("ws,bs,ov", [(10, 20, 0.8), (7, 13, 0.5), (12, 20, 0.7), (8, 0, 0.0)])
+def test_sizes(ctx, n, ws, bs, ov):
+    say("grid chain", n, ws, bs, ov)
+    t = synth.scaled(synth.config_c1(seed=n), max(n, 400))
+    x, y, z = t.generate()
+    x, y, z = x[:n].copy(), y[:n].copy(), z[:n].copy()
+    if n < 3:  # a box of one or two points needs an extent
+        x, y, z = np.append(x, x[0] + 30.0), np.append(y, y[0] + 25.0), np.append(z, z[0])
+    _run(ctx, x, y, z, ws, bs, ov)
+
+
+@pytest.mark.parametrize("ws,bs,ov", [(12, 20, 0.8), (20, 10, 0.5), (5, 30, 0.9), (15, 25, 0.6),
+                                      (9, 17, 0.63), (6, 14, 0.97), (3, 1, 0.0), (1, 2, 0.5)])
+@pytest.mark.parametrize("cm", [False, True])
+def test_parameters(ctx, ws, bs, ov, cm):
+    say("grid chain parameters", ws, bs, ov, cm)
+    t = synth.scaled(synth.config_c2(seed=ws), 150_000)
+    x, y, z = t.generate()
+    if cm:  # centimetre coordinates put about one point in a hundred on an edge
+        x, y, z = (np.round(a, 2) for a in (x, y, z))
+    _run(ctx, x, y, z, ws, bs, ov)
+
+
+@pytest.mark.parametrize("origin", [(0.0, 0.0), (612_345.0, 4_512_345.0), (-1234.56, 7.89)])
+@pytest.mark.parametrize("ws,bs,ov", [(8, 20, 0.5), (10, 20, 0.8), (12, 9, 0.7), (10, 6, 0.0)])
+def test_points_near_edges(ctx, origin, ws, bs, ov):
+    """Points 0 to 3 ulps, 1e-9 and 1e-6 either side of window and cell edges
+    and of their crossings, among random ones; z in whole steps (ties)."""
+    say("grid chain, points near edges", origin, ws, bs, ov)
+    rng = np.random.default_rng(int(ws * 100 + bs))
+    side, out = 180.0, []
+    for o in origin:
+        d = round(ws * (1 - ov), 2)
+        i = np.arange(int((side + 2 * ws * ov) / d) + 2)
+        c = (o - ws // 2 + d) + i * d
+        edges = np.concatenate([c - ws // 2, c + ws // 2])
+        k = np.arange(int(side / bs) + 1)
+        edges = np.concatenate([edges, (o + bs // 2 + k * bs) - bs // 2, (o + bs // 2 + k * bs) + bs // 2])
+        edges = edges[(edges > o) & (edges < o + side)]
+        v = rng.choice(edges, 9_000)
+        step = rng.integers(-3, 4, 9_000)
+        for _ in range(3):
+            v = np.where(step > 0, np.nextafter(v, np.inf), np.where(step < 0, np.nextafter(v, -np.inf), v))
+            step -= np.sign(step)
+        v[::7] += rng.choice([-1e-6, -1e-9, 1e-9, 1e-6], len(v[::7]))
+        out.append((v, o + side * rng.random(60_000)))
+    (ex, rx), (ey, ry) = out
+    x = np.concatenate([ex, ex, rx[:9_000], rx, [origin[0], origin[0] + side]])
+    y = np.concatenate([ey, ry[:9_000], ey, ry, [origin[1], origin[1] + side]])
+    z = np.round(rng.normal(50.0, 2.0, len(x)), 1)
+    p = rng.permutation(len(x))
+    _run(ctx, x[p], y[p], z[p], ws, bs, ov)
+
+
+def test_special_values(ctx):
+    """NaN and infinite coordinates and heights, the type's largest value, zeros of
+    both signs; coordinates far from every edge."""
+    say("grid chain, special values")
+    t = synth.scaled(synth.config_c1(seed=5), 40_000)
+    x, y, z = t.generate()
+    box = synth.bbox(x, y)
+    rng = np.random.default_rng(5)
+    for a in (x, y, z):
+        a[rng.integers(0, len(a), 300)] = np.nan
+    for a, v in ((x, np.inf), (y, -np.inf), (z, np.inf), (z, -np.inf), (z, 1.7976931348623157e308),
+                 (z, -0.0), (z, 0.0), (x, 1e300), (y, -1e300)):
+        a[rng.integers(0, len(a), 60)] = v
+    want = None
+    for leaf in (32, 0):
+        got = ctx.run_tile(x, y, z, 12, 20, 0.8, leaf, bbox=box)
+        want = got if want is None else want
+    assert np.array_equal(got, want) and len(want) > 50
+
+
+def test_lattice_falls_back(ctx):
+    """Every point on an edge: more than the pool holds, so the tree chain
+    answers; with the same points moved off the edges the grid chain does."""
+    say("grid chain, edge lattice")
+    rng = np.random.default_rng(9)
+    n = 400_000
+    x, y = (rng.integers(0, 801, n).astype(np.float64) for _ in range(2))
+    z = np.round(rng.normal(50.0, 3.0, n), 1)
+    _run(ctx, x, y, z, 8, 20, 0.5)
+    _run(ctx, x + 0.25, y + 0.25, z, 8, 20, 0.5)
+
+
+def test_shares_of_large_buckets(ctx):
+    """Few cells and many points: buckets read in shares, and cells beyond the
+    first class of buckets in one batch with small tiles."""
+    say("grid chain, shares")
+    big = synth.Tile(seed=3, n=3_000_000, width=150.0, height=140.0)
+    wide = synth.Tile(seed=4, n=300_000, width=1500.0, height=1300.0)
+    small = synth.scaled(synth.config_c1(seed=6), 20_011)
+    tiles = [(small, 10, 20, 0.8), (wide, 5, 12, 0.9), (big, 12, 20, 0.75), (small, 12, 20, 0.7)]
+    arrs = [t.generate() for t, *_ in tiles]
+    wants = [O.run(*a, ws, bs, ov, 32)[0] for a, (_, ws, bs, ov) in zip(arrs, tiles)]
+    desc = [(len(a[0]), dict(wsize=ws, bsize=bs, overlap=ov)) for a, (_, ws, bs, ov) in zip(arrs, tiles)]
+    xyz = [np.concatenate([a[k] for a in arrs]) for k in range(3)]
+    for graph in (False, True, True, False, True):
+        got = ctx.batch_run(*xyz, desc, graph=graph)
+        for i, (g, w) in enumerate(zip(got, wants)):
+            assert np.array_equal(g, w), f"tile {i}"
