@@ -18,14 +18,14 @@ static inline uint64_t up256(uint64_t v) { return (v + 255) / 256 * 256; }
 // of the bins with LDS for its own largest bucket.
 struct GridPlan {
     std::vector<GridTile> t;
-    std::vector<uint32_t> st_off, item_off, blk_off, gcell_off;
+    std::vector<uint32_t> st_off, item_off, blk_off, gcell_off, axis_off;
     std::vector<uint32_t> pt_off;  // caller's tile order
     struct Class {
         uint32_t t0, t1, cells;
     };
     std::vector<Class> cls;
-    uint64_t np = 0, cells = 0, tab = 0, nwin = 0, nleaf = 0, pool_cap = 0;
-    uint32_t max_nb = 1, rows_cap = 32;
+    uint64_t np = 0, recs = 0, cells = 0, tab = 0, nwin = 0, nleaf = 0, pool_cap = 0, list_cap = 0;
+    uint32_t max_nb = 1, win_cells = 1024;
 };
 
 // Bucket cells up to which tiles share a launch of the bins: the LDS of the
@@ -33,7 +33,8 @@ struct GridPlan {
 static int cell_class(uint32_t cells) { return cells <= 1024 ? 0 : cells <= 4096 ? 1 : 2; }
 
 // Fills one tile's grid; false when the chain does not take it.
-static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64_t n)
+static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64_t n,
+                      uint64_t launch_points)
 {
     memset(&T, 0, sizeof T);
     T.n = (uint32_t)n;
@@ -50,13 +51,18 @@ static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64
     }
     T.min_num_points = D.min_num_points;
     T.stage2_need = P.overlap != 0.0 ? 2u : 1u;
-    // buckets: the smallest power-of-two rectangle of cells that leaves at
-    // most this many of them (about two sort tiles of points each)
+    // Buckets: the smallest power-of-two rectangle of cells that leaves at most
+    // this many of them.  More buckets give a small launch more workgroups (1M
+    // points: bins 21 us with 8192 points a bucket, 11 us with 2048); fewer give
+    // a large one longer runs, which cost fewer loads (20M points: 129 us with
+    // 900 buckets, 102 us with 450) and fewer items (512 tiles, 329M points: 1.05
+    // ms with 4096 points a bucket, 0.99 ms with 8192).
     const uint32_t cx = T.ax[0].ncol, cy = T.ax[1].ncol;
     auto buckets = [&](uint32_t lw, uint32_t lh) {
         return ((uint64_t)(cx - 1) / (1u << lw) + 1) * ((uint64_t)(cy - 1) / (1u << lh) + 1);
     };
-    const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(n / 8192, 16), 1024);
+    const uint64_t per = launch_points <= (2u << 20) ? 2048 : launch_points <= (16u << 20) ? 4096 : 8192;
+    const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(n / per, 16), 512);
     uint32_t lw = 3, lh = 3;
     while (buckets(lw, lh) > want && lw + lh < 12)
         (lw <= lh ? lw : lh) += 1;
@@ -71,22 +77,27 @@ static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64
     T.nb = T.nbx * T.nby;
     T.nst = (uint32_t)((n + GRID_PTS - 1) / GRID_PTS);
     const uint64_t mean = n / T.nb;
+    // A bucket's points beyond 32768 are shared out: more workgroups, more partial
+    // cells for the windows to add up (120M points: bins + windows 0.90 ms with
+    // 16384, 0.69 with 32768, 0.75 with 65536).
     T.split = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(mean / 32768, 1), 16);
+    // A lane reads four consecutive points of a run, a segment is 2^lpr lanes:
+    // small segments waste the fewest lanes at the ends of runs, larger ones cost
+    // fewer list entries (10k points in 16 buckets: 19 us with one lane, 13 with
+    // two; 96 mixed tiles: 0.67 ms with one, 0.69 with two, 0.72 with four).
     const double run = T.nst ? (double)n / ((double)T.nst * T.nb) : 1.0;
-    T.lpr = run <= 8 ? 2 : run <= 20 ? 3 : run <= 48 ? 4 : run <= 128 ? 5 : 6;
-    // window blocks, and the rows of cells that one spans
-    T.lbw = T.ax[0].w.pair && T.ax[1].w.pair ? 5 : 4;
+    T.lpr = run <= 6.0 ? 0 : run <= 64.0 ? 1 : run <= 128.0 ? 2 : 3;
     return true;
 }
 
-// An upper bound on the rows of cells under bw windows.
-static double rows_of(const GridAxis &A, uint32_t bw)
+// An upper bound on the columns under bw windows.
+static double cols_of(const GridAxis &A, uint32_t bw)
 {
     const double len = (bw - 1) * A.w.step + 2.0 * A.w.half;
     double r = (len * A.w.inv + 1.0) * (A.w.pair ? 1.0 : 2.0);
     if (A.g.n)
         r += (len * A.g.inv + 1.0) * (A.g.pair ? 1.0 : 2.0);
-    return r + 4.0;
+    return std::ceil(r) + 4.0;
 }
 
 // An upper bound on the tree chain's device memory for the same call: a call
@@ -100,13 +111,16 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
                       const std::vector<std::array<double, 4>> &box, GridPlan &P)
 {
     std::vector<GridTile> raw(n_tiles);
+    uint64_t launch_points = 0;
+    for (uint32_t t = 0; t < n_tiles; ++t)
+        launch_points += tiles[t].n;
     P.pt_off.assign(n_tiles + 1, 0);
     for (uint32_t t = 0; t < n_tiles; ++t) {
         Derived D;
         std::string why;
         if (derive_params(tiles[t].params, tiles[t].n, box[t].data(), D, why) != OWM_OK)
             return false;  // the tree chain reports it
-        if (!plan_tile(raw[t], tiles[t].params, D, tiles[t].n))
+        if (!plan_tile(raw[t], tiles[t].params, D, tiles[t].n, launch_points))
             return false;
         raw[t].pt_off = P.pt_off[t];
         P.pt_off[t + 1] = P.pt_off[t] + (uint32_t)tiles[t].n;
@@ -114,24 +128,24 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
         P.nleaf += tiles[t].n / std::max(pick_leaf(ctx, tiles[t].n, 0), 1u) + 1;
     }
     P.np = P.pt_off[n_tiles];
-    // 32x32-window blocks where there are enough of them to occupy the device
+    // blocks of 32x32 windows where there are enough of them to occupy the
+    // device and their cells fit (48 KB), else smaller
     uint64_t big = 0;
     for (const GridTile &T : raw)
         big += ((T.ax[0].w.n + 31ull) / 32) * ((T.ax[1].w.n + 31ull) / 32);
-    double rows = 32.0;
     for (GridTile &T : raw) {
-        if (big < 512)
-            T.lbw = 4;
-        double r = std::max(rows_of(T.ax[0], 1u << T.lbw), rows_of(T.ax[1], 1u << T.lbw));
-        if (T.lbw == 5 && r > 64.0) {
-            T.lbw = 4;
-            r = std::max(rows_of(T.ax[0], 16), rows_of(T.ax[1], 16));
+        T.lbw = big < 512 || !T.ax[0].w.pair || !T.ax[1].w.pair ? 4 : 5;
+        double cells;
+        for (;; --T.lbw) {
+            const uint32_t bw = 1u << T.lbw;
+            cells = cols_of(T.ax[1], bw) * std::max<double>(cols_of(T.ax[0], bw), bw);
+            if (cells <= 3072.0 || T.lbw == 3)
+                break;
         }
-        rows = std::max(rows, std::ceil(r) * (double)(1u << T.lbw) / 32.0);
+        if (cells > GRID_MAX_WIN_CELLS)
+            return false;  // window sides of very many steps
+        P.win_cells = std::max(P.win_cells, (uint32_t)cells);
     }
-    if (rows > 96.0)
-        return false;  // 48 KB of row sums; longer windows stay with the tree chain
-    P.rows_cap = (uint32_t)std::ceil(rows);
     for (int c = 0; c < 3; ++c) {
         const uint32_t t0 = (uint32_t)P.t.size();
         uint32_t cells = 0;
@@ -147,10 +161,13 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
     P.item_off.assign(n_tiles + 1, 0);
     P.blk_off.assign(n_tiles + 1, 0);
     P.gcell_off.assign(n_tiles + 1, 0);
+    P.axis_off.assign(n_tiles + 1, 0);
     uint64_t st = 0, items = 0, blk = 0, gc = 0;
     for (uint32_t t = 0; t < n_tiles; ++t) {
         GridTile &T = P.t[t];
         T.st_off = (uint32_t)st;
+        T.rec_off = (uint32_t)P.recs;
+        P.recs += (T.n + 3ull) / 4 * 4;
         T.item_off = (uint32_t)items;
         T.blk_off = (uint32_t)blk;
         T.gcell_off = (uint32_t)gc;
@@ -169,10 +186,12 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
         P.item_off[t + 1] = (uint32_t)items;
         P.blk_off[t + 1] = (uint32_t)blk;
         P.gcell_off[t + 1] = (uint32_t)gc;
+        P.axis_off[t + 1] = P.axis_off[t] + T.ax[0].w.n + T.ax[1].w.n;
         P.max_nb = std::max(P.max_nb, T.nb);
     }
     // a quarter of the points may lie on edges before the tree chain takes over
     P.pool_cap = (P.np / 4 + 65536) / GRID_POOLS;
+    P.list_cap = P.pool_cap + P.pool_cap / 64 + 2 * (items / GRID_POOLS + 1);
     return true;
 }
 
@@ -294,11 +313,11 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
     const uint32_t T = n_tiles;
     const uint64_t nwords = (np + 31) / 32, items = P.item_off[T], gcells = P.gcell_off[T];
     const uint64_t nseed = std::min<uint64_t>(np, P.nwin + gcells) + 1;
-    const uint64_t table = up256(T * sizeof(GridTile)) + 5 * up256((T + 1) * 4ull);
-    const uint64_t need = table + up256(np * 8) + up256(np * 4) + up256(P.tab * 2) +
-                          up256(P.cells * 16) + up256(items * 4) +
+    const uint64_t table = up256(T * sizeof(GridTile)) + 6 * up256((T + 1) * 4ull);
+    const uint64_t need = table + up256(P.recs * 12 + 64) + up256(P.tab * 2) +
+                          up256(P.cells * 16) + up256(items * 4) + up256(P.axis_off[T] * 8ull) +
                           up256(P.pool_cap * GRID_POOLS * sizeof(GridRare)) +
-                          up256(GRID_POOLS * 64) + 2 * up256((nwords + 4) * 4) +
+                          up256(P.list_cap * GRID_POOLS * 4) + up256(GRID_POOLS * 128) + 2 * up256((nwords + 4) * 4) +
                           up256((gcells + 1) * 4) + up256((nwords / 4096 + 2) * 4) +
                           up256(nseed * 4) + up256((T + 1) * 4ull) + 4096;
     const uint64_t others = ctx->held_bytes() - ctx->arena.buf.bytes;
@@ -335,11 +354,11 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
     G.ngcell = (uint32_t)gcells;
     G.tiles = (const GridTile *)d;
     memcpy(h, P.t.data(), T * sizeof(GridTile));
-    const std::vector<uint32_t> *src[5] = {&P.st_off, &P.item_off, &P.blk_off, &P.gcell_off,
-                                           &P.pt_off};
-    const uint32_t *off[5];
+    const std::vector<uint32_t> *src[6] = {&P.st_off,    &P.item_off, &P.blk_off,
+                                           &P.gcell_off, &P.axis_off, &P.pt_off};
+    const uint32_t *off[6];
     uint64_t o = up256(T * sizeof(GridTile));
-    for (int k = 0; k < 5; ++k, o += up256((T + 1) * 4ull)) {
+    for (int k = 0; k < 6; ++k, o += up256((T + 1) * 4ull)) {
         memcpy(h + o, src[k]->data(), (T + 1) * 4ull);
         off[k] = (const uint32_t *)(d + o);
     }
@@ -347,22 +366,26 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
     G.item_off = off[1];
     G.blk_off = off[2];
     G.gcell_off = off[3];
+    G.axis_off = off[4];
     BatchDev B{};
     B.ntiles = T;
     B.np = (uint32_t)np;
-    B.pt_off = off[4];
+    B.pt_off = off[5];
     HIP_TRY(hipMemcpyAsync(d, h, table, hipMemcpyHostToDevice, s), "upload table");
 
     QueryOut qo;
     auto body = [&]() -> owm_status {
-        G.zk = (unsigned long long *)A.take(np * 8);
-        G.cw = (uint32_t *)A.take(np * 4);
+        // (a lane's last load may reach 36 bytes past its run)
+        G.rec = (uint32_t *)A.take(P.recs * 12 + 64);
         G.tab = (uint16_t *)A.take(P.tab * 2);
         G.cells = (uint4 *)A.take(P.cells * 16);
         G.heads = (uint32_t *)A.take(items * 4);
+        G.wcols = (int2 *)A.take(P.axis_off[T] * 8ull);
         G.pool = (GridRare *)A.take(P.pool_cap * GRID_POOLS * sizeof(GridRare));
         G.pool_cap = (uint32_t)P.pool_cap;
-        G.pool_used = (uint32_t *)A.take(GRID_POOLS * 64);
+        G.list = (uint32_t *)A.take(P.list_cap * GRID_POOLS * 4);
+        G.list_cap = (uint32_t)P.list_cap;
+        G.pool_used = (uint32_t *)A.take(GRID_POOLS * 128);
         G.seen = (uint32_t *)A.take((nwords + 4) * 4);
         G.llp = (uint32_t *)A.take((nwords + 4) * 4);
         G.cell_flag = (uint32_t *)A.take((gcells + 1) * 4);
@@ -381,23 +404,23 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
             z.len[z.count++] = words;
         };
         zero(cnt, 16);
-        zero(G.pool_used, GRID_POOLS * 16);
+        zero(G.pool_used, GRID_POOLS * 32);
         zero(G.seen, nwords + 4);
         zero(G.llp, nwords + 4);
         zero(G.cell_flag, gcells + 1);
         zero(lookback, nwords / 4096 + 2);
-        launch_fill_ranges(s, z);
+        launch_grid_prep(s, G, z, P.axis_off[T]);
         int pi = ctx->prof.begin(s, PH_GRID_PART);
         launch_grid_part(s, G, dx, dy, dz, P.st_off[T], P.max_nb);
-        // x, y and z read; a z key and a word written
+        // x, y and z read; a record written
         ctx->prof.end(s, pi, 36ull * np, np);
         pi = ctx->prof.begin(s, PH_GRID_BIN);
         for (const GridPlan::Class &c : P.cls)
-            launch_grid_bin(s, G, dx, dy, dz, c.t0, c.t1, P.item_off[c.t0],
+            launch_grid_bin(s, G, c.t0, c.t1, P.item_off[c.t0],
                             P.item_off[c.t1] - P.item_off[c.t0], c.cells);
         ctx->prof.end(s, pi, 12ull * np + 16ull * P.cells, np, (uint32_t)P.cls.size());
         pi = ctx->prof.begin(s, PH_GRID_WIN);
-        launch_grid_windows(s, G, dx, dy, P.blk_off[T], P.rows_cap);
+        launch_grid_windows(s, G, dx, dy, P.blk_off[T], P.win_cells);
         ctx->prof.end(s, pi, 16ull * P.cells + 8ull * P.nwin, P.nwin);
         if (gcells) {
             pi = ctx->prof.begin(s, PH_STAGE3);

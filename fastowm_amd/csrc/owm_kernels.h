@@ -131,11 +131,10 @@ constexpr uint32_t GRID_ERR_POOL = 32u, GRID_ERR_ROWS = 64u;
 
 // A point without a column (on an edge, or between the edges of a pair) with
 // the windows [wx0, wx1) x [wy0, wy1) and stage-3 cells [gx0, gx1) x [gy0, gy1)
-// that hold it.  The first entry of each block of the pool is its header: id
-// the entries that follow, next the bucket's next block.
+// that hold it.
 struct GridRare {
     unsigned long long zk;
-    uint32_t id, next;
+    uint32_t id, pad;
     uint16_t wx0, wx1, wy0, wy1, gx0, gx1, gy0, gy1;
 };
 
@@ -145,6 +144,7 @@ struct GridTile {
     uint64_t tab_off;   // first run-start entry: [nst][nb + 1]
     uint64_t cell_off;  // first grid cell: [nb][split][2^(lw + lh)]
     uint32_t pt_off, n;
+    uint32_t rec_off;            // first record (a multiple of 4)
     uint32_t st_off, nst;        // sort tiles
     uint32_t lw, lh;             // a bucket is 2^lw columns x 2^lh rows
     uint32_t nbx, nby, nb;       // buckets
@@ -159,14 +159,18 @@ struct GridDev {
     uint32_t ntiles, ngcell;
     const GridTile *tiles;
     const uint32_t *st_off, *item_off, *blk_off, *gcell_off;  // [ntiles + 1] each
-    unsigned long long *zk;  // [np] z keys, grouped by bucket within each sort tile
-    uint32_t *cw;            // [np] cell << GRID_SLOT_BITS | slot (bit 31: no column)
+    const uint32_t *axis_off;  // [ntiles + 1] first entry of a tile in wcols (ncols + nrows each)
+    int2 *wcols;               // columns [first, last] of the windows of each axis
+    // 12-byte records, grouped by bucket within each sort tile: z key (2 words),
+    // cell << GRID_SLOT_BITS | slot (bit 31: no column, the key is its pool entry)
+    uint32_t *rec;
     uint16_t *tab;           // run starts per sort tile and bucket
     uint4 *cells;            // {z key, id, count} per grid cell
-    uint32_t *heads;         // [items] first pool block of the item's listed points
-    GridRare *pool;
-    uint32_t *pool_used;     // [GRID_POOLS * 16] entries used of each share (one per 64 bytes)
-    uint32_t pool_cap;       // entries per share
+    GridRare *pool;          // points without a column
+    uint32_t *heads;         // [items] the item's first block in list, or OWM_NONE
+    uint32_t *list;          // blocks {n, next block, n pool entries}
+    uint32_t *pool_used;     // [GRID_POOLS * 32] used of each share of pool (word 0) and list (16)
+    uint32_t pool_cap, list_cap;  // entries (words) per share
     uint32_t *seen, *llp;    // point bitmaps: one window, two (LLPs, then seeds)
     uint32_t *cell_flag;     // [ngcell] stage-3 cells that hold an LLP
     uint32_t *err;
@@ -174,16 +178,19 @@ struct GridDev {
 
 // Raises the kernels' LDS limits; once per device.
 hipError_t grid_kernels_init();
+// Zeroes the ranges and fills G.wcols (windows: its entries).
+void launch_grid_prep(hipStream_t s, const GridDev &G, const FillRanges &r, uint32_t windows);
 void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const double *y,
                       const double *z, uint32_t sort_tiles, uint32_t max_nb);
 // Items [item0, item0 + items) of the table entries [t0, t1); cells: the
 // largest bucket's.
-void launch_grid_bin(hipStream_t s, const GridDev &G, const double *x, const double *y,
-                     const double *z, uint32_t t0, uint32_t t1, uint32_t item0, uint32_t items,
-                     uint32_t cells);
-// rows_cap * 32 row sums of LDS (rows_cap >= 32)
+void launch_grid_bin(hipStream_t s, const GridDev &G, uint32_t t0, uint32_t t1, uint32_t item0,
+                     uint32_t items, uint32_t cells);
+// cells_cap: cells under a window block (at least the windows of a block), at
+// most GRID_MAX_WIN_CELLS
+constexpr uint32_t GRID_MAX_WIN_CELLS = 9216;
 void launch_grid_windows(hipStream_t s, const GridDev &G, const double *x, const double *y,
-                         uint32_t blocks, uint32_t rows_cap);
+                         uint32_t blocks, uint32_t cells_cap);
 void launch_grid_cells(hipStream_t s, const GridDev &G);
 
 // ---- .xyz reader (xyz.hip) ----
