@@ -80,7 +80,11 @@ __device__ __forceinline__ uint32_t grid_key(const GridTile &T, uint32_t cx, uin
 
 // Everything the chain starts from: ranges that must be zero (blockIdx.y below
 // their count), and the columns of every window of a tile, x then y.
-__global__ __launch_bounds__(256) void k_grid_prep(GridDev G, FillRanges r, uint32_t windows)
+// The table of a few tiles is read from host memory, and copied, here: an upload
+// of its own would cost more.
+__global__ __launch_bounds__(256) void k_grid_prep(GridDev G, FillRanges r, uint32_t windows,
+                                                    const uint32_t *__restrict__ host_table,
+                                                    uint32_t table_words)
 {
     const uint32_t i0 = blockIdx.x * 256u + threadIdx.x;
     if (blockIdx.y < r.count) {
@@ -90,10 +94,18 @@ __global__ __launch_bounds__(256) void k_grid_prep(GridDev G, FillRanges r, uint
             p[i] = 0;
         return;
     }
+    const uint32_t *own = (const uint32_t *)G.tiles;
+    if (blockIdx.y > r.count) {
+        for (uint32_t i = i0; i < table_words; i += gridDim.x * 256u)
+            const_cast<uint32_t *>(own)[i] = host_table[i];
+        return;
+    }
+    const uint32_t *table = host_table ? host_table : own;
+    const uint32_t *axis_off = table + (G.axis_off - own);
     for (uint32_t i = i0; i < windows; i += gridDim.x * 256u) {
-        const uint32_t t = owm_find_tile(G.axis_off, G.ntiles, i);
-        const GridTile &T = G.tiles[t];
-        const uint32_t q = i - G.axis_off[t], n = T.ax[0].w.n, a = q >= n ? 1u : 0u;
+        const uint32_t t = owm_find_tile(axis_off, G.ntiles, i);
+        const GridTile &T = ((const GridTile *)table)[t];
+        const uint32_t q = i - axis_off[t], n = T.ax[0].w.n, a = q >= n ? 1u : 0u;
         int first, last;
         axis_window_cols(T.ax[a], a ? q - n : q, first, last);
         G.wcols[i] = make_int2(first, last);
@@ -827,14 +839,17 @@ __global__ __launch_bounds__(256) void k_grid_cells(GridDev G)
 
 // ----------------------------------------------------------------- launch --
 
-void launch_grid_prep(hipStream_t s, const GridDev &G, const FillRanges &r, uint32_t windows)
+void launch_grid_prep(hipStream_t s, const GridDev &G, const FillRanges &r, uint32_t windows,
+                      const uint32_t *host_table, uint32_t table_words)
 {
     uint64_t most = windows;
     for (uint32_t k = 0; k < r.count; ++k)
         most = r.len[k] > most ? r.len[k] : most;
     const uint64_t g = (most + 1023) / 1024;  // four words a thread, up to 2048 blocks
-    hipLaunchKernelGGL(k_grid_prep, dim3((uint32_t)(g < 1 ? 1 : g > 2048 ? 2048 : g), r.count + 1),
-                       dim3(256), 0, s, G, r, windows);
+    hipLaunchKernelGGL(k_grid_prep,
+                       dim3((uint32_t)(g < 1 ? 1 : g > 2048 ? 2048 : g),
+                            r.count + (host_table ? 2 : 1)),
+                       dim3(256), 0, s, G, r, windows, host_table, table_words);
 }
 
 void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const double *y,

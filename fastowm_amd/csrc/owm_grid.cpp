@@ -195,6 +195,79 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
     return true;
 }
 
+// The chain's results in page-locked host memory: count and error flags, tile
+// ranges, the first indices (most calls' all: no copy follows the chain), and
+// before it the boxes.
+struct GridIo {
+    static constexpr uint32_t IDS = 65536;
+    uint32_t *head = nullptr, *off = nullptr, *ids = nullptr;
+    double *box = nullptr;
+    GridIo(owm_ctx *ctx, uint32_t n_tiles)
+    {
+        const uint64_t o = 256 + up256((n_tiles + 1) * 4ull), i = o + IDS * 4ull;
+        uint8_t *h = ctx->pinned(ctx->h_io, ctx->h_io_cap,
+                                 std::max<uint64_t>(i + n_tiles * 32ull, io_bytes(n_tiles)));
+        if (!h)
+            return;
+        head = (uint32_t *)h;
+        off = (uint32_t *)(h + 256);
+        ids = (uint32_t *)(h + o);
+        box = (double *)(h + i);
+    }
+};
+
+// Boxes of at most BOX_TILES tiles: one launch that leaves them in io.box.
+static owm_status take_few_boxes(owm_ctx *ctx, const double *dx, const double *dy,
+                                 const owm_tile *tiles, uint32_t n_tiles, const GridIo &io,
+                                 std::vector<std::array<double, 4>> &box)
+{
+    hipStream_t s = ctx->stream;
+    if (!ctx->box_work.ptr) {
+        HIP_TRY(ctx->box_work.reserve(box_work_bytes()), "box work");
+        launch_fill_u32(s, (uint32_t *)ctx->box_work.ptr, BOX_TILES, 0u);
+    }
+    BoxArgs a{};
+    a.ntiles = n_tiles;
+    uint64_t np = 0, want = 0;
+    auto needed = [&](uint32_t t) {
+        return tiles[t].n && !(tiles[t].params.flags & OWM_F_HAVE_BBOX);
+    };
+    for (uint32_t t = 0; t < n_tiles; ++t)
+        if (needed(t)) {
+            np += tiles[t].n;
+            want += (tiles[t].n + BOX_POINTS - 1) / BOX_POINTS;
+        }
+    // a workgroup per BOX_POINTS points, and no more than four to a CU (their
+    // tickets are atomics on one word)
+    const double scale = want > 1024 ? 1024.0 / (double)want : 1.0;
+    for (uint32_t t = 0; t < n_tiles; ++t) {
+        uint32_t g = 0;
+        if (needed(t))
+            g = std::max(1u, (uint32_t)((double)((tiles[t].n + BOX_POINTS - 1) / BOX_POINTS) * scale));
+        a.pt[t + 1] = a.pt[t] + (uint32_t)tiles[t].n;
+        a.blk[t + 1] = a.blk[t] + g;
+    }
+    if (a.blk[n_tiles]) {
+        const int pi = ctx->prof.begin(s, PH_BBOX);
+        launch_boxes(s, a, dx, dy, ctx->box_work.ptr, io.box);
+        ctx->prof.end(s, pi, 16ull * np, np);
+        HIP_TRY(hipGetLastError(), "box launch");
+        HIP_TRY(hipStreamSynchronize(s), "bbox sync");
+        ctx->prof.collect();
+    }
+    for (uint32_t t = 0; t < n_tiles; ++t) {
+        if (tiles[t].params.flags & OWM_F_HAVE_BBOX)
+            continue;
+        const double *b = io.box + 4 * t;  // min x, min y, max x, max y
+        if (tiles[t].n == 0 || !(b[0] <= b[2]) || !(b[1] <= b[3])) {
+            set_err(ctx, "tile %u: no finite points to take a bbox from", t);
+            return OWM_E_ARG;
+        }
+        box[t] = {b[0], b[2], b[1], b[3]};
+    }
+    return OWM_OK;
+}
+
 // Exact boxes of the tiles that come without one (device reduction).
 static owm_status take_boxes(owm_ctx *ctx, const double *dx, const double *dy,
                              const owm_tile *tiles, uint32_t n_tiles,
@@ -252,7 +325,7 @@ static owm_status take_boxes(owm_ctx *ctx, const double *dx, const double *dy,
 
 // Everything the chain's launches depend on.
 static void plan_key(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
-                     const GridPlan &P, std::vector<uint8_t> &key)
+                     const GridPlan &P, const GridIo &io, std::vector<uint8_t> &key)
 {
     auto put = [&key](const void *p, size_t n) {
         const uint8_t *b = (const uint8_t *)p;
@@ -260,7 +333,7 @@ static void plan_key(owm_ctx *ctx, const double *dx, const double *dy, const dou
     };
     key.clear();
     put("grid", 4);
-    const void *ptrs[4] = {dx, dy, dz, ctx->arena.buf.ptr};
+    const void *ptrs[6] = {dx, dy, dz, ctx->arena.buf.ptr, io.head, ctx->h_tab};
     put(ptrs, sizeof ptrs);
     put(P.t.data(), P.t.size() * sizeof(GridTile));
     put(P.pt_off.data(), P.pt_off.size() * 4);
@@ -291,8 +364,14 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
     }
     if (np == 0)
         return OWM_OK;
+    const GridIo io(ctx, n_tiles);
+    if (!io.head) {
+        set_err(ctx, "pinned host allocation failed");
+        return OWM_E_NOMEM;
+    }
     if (need_box) {
-        st = take_boxes(ctx, dx, dy, tiles, n_tiles, box);
+        st = n_tiles <= BOX_TILES ? take_few_boxes(ctx, dx, dy, tiles, n_tiles, io, box)
+                                  : take_boxes(ctx, dx, dy, tiles, n_tiles, box);
         if (st != OWM_OK)
             return st;
     }
@@ -333,21 +412,21 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
 
     Arena &A = ctx->arena;
     hipStream_t s = ctx->stream;
-    bool graph = (flags & OWM_B_GRAPH) != 0;
-    std::vector<uint8_t> key;
-    if (graph || (flags & B_AUTO_GRAPH))
-        plan_key(ctx, dx, dy, dz, P, key);
-    if (!graph && (flags & B_AUTO_GRAPH)) {
-        graph = !ctx->prof.on && key == ctx->graphs.last_key;
-        ctx->graphs.last_key = key;
-    }
     // table
     uint8_t *d = A.take(table);
-    (void)hipStreamSynchronize(s);  // the previous upload from this buffer must have completed
+    (void)hipStreamSynchronize(s);  // the previous reads of this buffer must have completed
     uint8_t *h = ctx->pinned(ctx->h_tab, ctx->h_tab_cap, table);
     if (!d || !h) {
         set_err(ctx, "pinned host allocation failed");
         return OWM_E_NOMEM;
+    }
+    bool graph = (flags & OWM_B_GRAPH) != 0;
+    std::vector<uint8_t> key;
+    if (graph || (flags & B_AUTO_GRAPH))
+        plan_key(ctx, dx, dy, dz, P, io, key);
+    if (!graph && (flags & B_AUTO_GRAPH)) {
+        graph = !ctx->prof.on && key == ctx->graphs.last_key;
+        ctx->graphs.last_key = key;
     }
     GridDev G{};
     G.ntiles = T;
@@ -371,7 +450,10 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
     B.ntiles = T;
     B.np = (uint32_t)np;
     B.pt_off = off[5];
-    HIP_TRY(hipMemcpyAsync(d, h, table, hipMemcpyHostToDevice, s), "upload table");
+    // a few tiles' table is fetched by the chain's first launch
+    const bool fetch = T <= 8;
+    if (!fetch)
+        HIP_TRY(hipMemcpyAsync(d, h, table, hipMemcpyHostToDevice, s), "upload table");
 
     QueryOut qo;
     auto body = [&]() -> owm_status {
@@ -409,7 +491,8 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
         zero(G.llp, nwords + 4);
         zero(G.cell_flag, gcells + 1);
         zero(lookback, nwords / 4096 + 2);
-        launch_grid_prep(s, G, z, P.axis_off[T]);
+        launch_grid_prep(s, G, z, P.axis_off[T], fetch ? (const uint32_t *)h : nullptr,
+                         (uint32_t)(table / 4));
         int pi = ctx->prof.begin(s, PH_GRID_PART);
         launch_grid_part(s, G, dx, dy, dz, P.st_off[T], P.max_nb);
         // x, y and z read; a record written
@@ -428,27 +511,48 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
             ctx->prof.end(s, pi, 12ull * gcells, gcells);
         }
         pi = ctx->prof.begin(s, PH_MERGE);
-        launch_bits_compact(s, G.llp, (uint32_t)nwords, out, cnt + 2, lookback, cnt + 7);
+        SeedOut S;
+        S.ntiles = T;
+        S.pt_off = B.pt_off;
+        S.err = cnt + 3;
+        S.host = io.head;
+        S.host_off = io.off;
+        S.host_ids = io.ids;
+        S.host_cap = GridIo::IDS;
+        launch_seeds(s, B, G.llp, (uint32_t)nwords, out, (uint32_t)nseed, seed_off, cnt + 2,
+                     lookback, cnt + 7, S);
         ctx->prof.end(s, pi, 4ull * nwords, nwords);
-        launch_seed_ranges(s, B, out, cnt + 2, seed_off);
-        launch_seeds_local(s, B, out, cnt + 2, (uint32_t)nseed);
         HIP_TRY(hipGetLastError(), "grid chain launch");
         qo.cnt = cnt;
-        qo.seed_off = seed_off;
         qo.seeds = out;
         return OWM_OK;
     };
     st = run_chain(ctx, graph, std::move(key), A, qo, body);
     if (st != OWM_OK)
         return st;
-    uint32_t err = 0;
-    st = read_seeds(ctx, qo, n_tiles, seeds, cap, seed_off_host, nullptr, &err);
-    if (st != OWM_OK)
-        return st;
+    HIP_TRY(hipStreamSynchronize(s), "pipeline");
+    ctx->prof.collect();
+    const uint32_t err = io.head[1];
+    if (err & ~GRID_ERR_POOL) {
+        set_err(ctx, "device capacity guard tripped (flags %u)", err);
+        return OWM_E_INTERNAL;
+    }
     if (err & GRID_ERR_POOL) {
         handled = false;
         return hand_on();
     }
+    const uint64_t ns = io.head[0];
+    for (uint32_t t = 0; t <= n_tiles; ++t)
+        seed_off_host[t] = io.off[t];
+    if (ns > cap) {
+        set_err(ctx, "seed buffer holds %llu, %llu needed", (unsigned long long)cap,
+                (unsigned long long)ns);
+        return OWM_E_CAPACITY;
+    }
+    if (ns <= GridIo::IDS)
+        memcpy(seeds, io.ids, ns * 4);
+    else
+        HIP_TRY(hipMemcpy(seeds, qo.seeds, ns * 4, hipMemcpyDeviceToHost), "seeds D2H");
     return OWM_OK;
 }
 

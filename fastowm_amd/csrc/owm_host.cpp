@@ -1205,7 +1205,7 @@ owm_status check_guards(owm_ctx *ctx, const uint32_t *hc, uint64_t *s1_needed)
 
 owm_status read_seeds(owm_ctx *ctx, const QueryOut &qo, uint32_t n_tiles, uint32_t *seeds,
                       uint64_t cap, uint64_t *seed_off_host, uint64_t *s1_needed,
-                      uint32_t *pool_full, const RunMem *mem)
+                      const RunMem *mem)
 {
     hipStream_t s = ctx->stream;
     const IoLayout io(n_tiles);
@@ -1221,17 +1221,8 @@ owm_status read_seeds(owm_ctx *ctx, const QueryOut &qo, uint32_t n_tiles, uint32
             "ranges D2H");
     HIP_TRY(hipStreamSynchronize(s), "pipeline");
     ctx->prof.collect();
-    if (pool_full) {
-        // the column-grid chain: its only recoverable flag ends the read
-        *pool_full = hc[3] & GRID_ERR_POOL;
-        if (*pool_full)
-            return OWM_OK;
-    }
-    uint64_t need = 0;
-    owm_status st = check_guards(ctx, hc, &need);
-    if (s1_needed)
-        *s1_needed = need;
-    if (st != OWM_OK || need)
+    owm_status st = check_guards(ctx, hc, s1_needed);
+    if (st != OWM_OK || *s1_needed)
         return st;
     const uint64_t ns = hc[2];
     for (uint32_t t = 0; t <= n_tiles; ++t)
@@ -1509,7 +1500,7 @@ owm_status run_tile_fixed(owm_ctx *ctx, const double *dx, const double *dy, cons
         if (st != OWM_OK)
             return st;
         uint64_t s1_need = 0, off[2] = {0, 0};
-        st = read_seeds(ctx, qo, 1, seeds, cap, off, &s1_need, nullptr, &mem);
+        st = read_seeds(ctx, qo, 1, seeds, cap, off, &s1_need, &mem);
         *n_seeds = off[1];
         if (st != OWM_OK || s1_need == 0)
             return st;
@@ -1582,7 +1573,7 @@ uint64_t owm_ctx::room_for(const owm::DevBuf &b) const
 uint64_t owm_ctx::held_bytes() const
 {
     uint64_t b = arena.buf.bytes + small.buf.bytes + upload.bytes + s1_list.bytes;
-    b += xyz_text.bytes + xyz_work.bytes + xyz_cloud.bytes + qs_work.bytes;
+    b += box_work.bytes + xyz_text.bytes + xyz_work.bytes + xyz_cloud.bytes + qs_work.bytes;
     b += trees_bytes.load();
     return b;
 }

@@ -197,11 +197,9 @@ owm_status prepare_query(owm_ctx *ctx, const owm_params *params, uint32_t stride
 owm_status upload_table(owm_ctx *ctx, Arena &A, const Prepared &P, BatchDev &B,
                         const RunMem *mem = nullptr);
 // Reads the counts, checks the device guards, copies the seeds (tile-local).
-// pool_full (column-grid chain): set, with nothing copied, when the chain's pool
-// was full.
 owm_status read_seeds(owm_ctx *ctx, const QueryOut &qo, uint32_t n_tiles, uint32_t *seeds,
                       uint64_t cap, uint64_t *seed_off_host, uint64_t *s1_needed,
-                      uint32_t *pool_full = nullptr, const RunMem *mem = nullptr);
+                      const RunMem *mem = nullptr);
 owm_status check_tiles(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles);
 owm_status run_chain(owm_ctx *ctx, bool graph, std::vector<uint8_t> key, Arena &A, QueryOut &qo,
                      const std::function<owm_status()> &body);
@@ -312,6 +310,7 @@ struct owm_ctx {
     std::string err;
     owm::Arena arena;   // tree + scratch of the current run
     owm::Arena small;   // bbox pass
+    owm::DevBuf box_work;  // partial boxes of launch_boxes
     owm::DevBuf upload; // host inputs staged to the device
     owm::DevBuf s1_list; // stage-1 leaf/block join list (grows on demand)
     // .xyz reader: the text and index, parse work (and the cloud when no line

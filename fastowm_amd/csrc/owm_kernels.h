@@ -77,6 +77,20 @@ struct TreeOut {
     uint2 *nd_child;  // children (OWM_LEAF_BIT | leaf, or node)
 };
 
+// Exact boxes (NaNs ignored) of up to BOX_TILES tiles in one launch, straight
+// to host memory: box[4 t ..] = min x, min y, max x, max y (min > max: the tile
+// has no such coordinate).  Tile t is [pt[t], pt[t+1]) and takes the workgroups
+// [blk[t], blk[t+1]), blk[ntiles] <= BOX_BLOCKS.  work: box_work_bytes(), its first
+// BOX_TILES words zero before the first launch that uses it (each launch leaves
+// them zero); launches on one work are ordered by their stream.
+constexpr uint32_t BOX_TILES = 64, BOX_BLOCKS = 4096, BOX_POINTS = 4096;
+struct BoxArgs {
+    uint32_t ntiles;
+    uint32_t pt[BOX_TILES + 1], blk[BOX_TILES + 1];
+};
+uint64_t box_work_bytes();
+void launch_boxes(hipStream_t s, const BoxArgs &a, const double *x, const double *y, void *work,
+                  double *box);
 // bbox per tile as order-preserving u64 keys [minx, miny, maxx(inv), maxy(inv)]
 void launch_bbox(hipStream_t s, const BatchDev &B, const double *x, const double *y,
                  unsigned long long *bbox_keys);
@@ -178,8 +192,11 @@ struct GridDev {
 
 // Raises the kernels' LDS limits; once per device.
 hipError_t grid_kernels_init();
-// Zeroes the ranges and fills G.wcols (windows: its entries).
-void launch_grid_prep(hipStream_t s, const GridDev &G, const FillRanges &r, uint32_t windows);
+// Zeroes the ranges and fills G.wcols (windows: its entries).  host_table (may
+// be null: G.tiles is in place): the table in host memory, table_words long, which
+// the launch reads from there and copies to G.tiles.
+void launch_grid_prep(hipStream_t s, const GridDev &G, const FillRanges &r, uint32_t windows,
+                      const uint32_t *host_table, uint32_t table_words);
 void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const double *y,
                       const double *z, uint32_t sort_tiles, uint32_t max_nb);
 // Items [item0, item0 + items) of the table entries [t0, t1); cells: the
@@ -308,6 +325,18 @@ void launch_bits_set(hipStream_t s, const uint32_t *ids, const uint32_t *d_off, 
 // set bits of words[0..nwords) -> ascending indices + count
 void launch_bits_compact(hipStream_t s, const uint32_t *words, uint32_t nwords, uint32_t *out,
                          uint32_t *d_count, uint32_t *lookback, uint32_t *tile_counter);
+// The seeds of a batch from their bitmap: indices within their tiles in out (at
+// most n_max), and the results in host memory (page-locked, mapped): host[0] the
+// count, host[1] *err, host_off[ntiles + 1] each tile's first, host_ids the first
+// host_cap indices.  seed_off: ntiles + 1 words of scratch.
+struct SeedOut {
+    uint32_t ntiles = 0, host_cap = 0;
+    const uint32_t *pt_off = nullptr, *err = nullptr;  // device
+    uint32_t *host = nullptr, *host_off = nullptr, *host_ids = nullptr;
+};
+void launch_seeds(hipStream_t s, const BatchDev &B, const uint32_t *words, uint32_t nwords,
+                  uint32_t *out, uint32_t n_max, uint32_t *seed_off, uint32_t *d_count,
+                  uint32_t *lookback, uint32_t *tile_counter, const SeedOut &S);
 void launch_stage3(hipStream_t s, const BatchDev &B, const TreeDev &T, const uint32_t *llp,
                    const uint32_t *n_llp, uint32_t n_llp_max, uint32_t *cell_flag,
                    uint32_t *cell_res, uint32_t *err);

@@ -201,15 +201,21 @@ __global__ __launch_bounds__(256) void k_bits_set(const uint32_t *__restrict__ i
 // compaction with one look-back per tile of CP_BLOCK x 4 x BC_VEC words (BC_VEC
 // uint4 loads per lane).  The look-back chain is serial, so a large bitmap
 // takes large tiles (few links) and a small one small tiles (enough
-// workgroups).
-template <int BC_VEC>
+// workgroups).  With SEEDS the indices written are those within the tiles, and
+// the tiles' ranges, the count, the error flags and the first S.host_cap indices
+// also go to host memory, where the caller finds them without a copy.
+template <int BC_VEC, bool SEEDS>
 __global__ __launch_bounds__(CP_BLOCK) void k_bits_compact(const uint32_t *__restrict__ words,
                                                            uint32_t nwords,
                                                            uint32_t *__restrict__ out,
                                                            uint32_t *d_count, uint32_t *lookback,
-                                                           uint32_t *tile_counter)
+                                                           uint32_t *tile_counter, SeedOut S)
 {
     constexpr uint32_t BC_TILE = CP_BLOCK * BC_VEC * 4;
+    // a tile's indices on their way out: linear writes reach host memory at the
+    // link's rate (each lane writing its own run took 60 us for 64K of them)
+    constexpr uint32_t BC_STAGE = SEEDS ? 4096 : 1;
+    __shared__ uint32_t s_out[BC_STAGE], s_last;
     __shared__ uint32_t s_tile, s_tmp[CP_BLOCK / 64], s_prefix;
     const uint32_t ntiles = (nwords + BC_TILE - 1) / BC_TILE;
     if (nwords == 0) {
@@ -242,15 +248,89 @@ __global__ __launch_bounds__(CP_BLOCK) void k_bits_compact(const uint32_t *__res
         }
         uint32_t total;
         const uint32_t excl = block_excl_scan_cp(cnt, s_tmp, total);
+        // the tiles of the batch whose points this tile of words holds, found while
+        // the prefix is on its way
+        const uint32_t p0 = tile * BC_TILE << 5, p1 = (tile + 1) * BC_TILE << 5;
+        uint32_t b0 = 0, b1 = 0;
+        if (SEEDS && S.ntiles > 1) {
+            b0 = owm_find_tile(S.pt_off, S.ntiles, p0);
+            b1 = owm_find_tile(S.pt_off, S.ntiles, p1);
+        }
         if (threadIdx.x == 0) {
             const uint32_t prefix = tile_prefix(lookback, tile, total);
             s_prefix = prefix;
-            if (tile == ntiles - 1)
+            if (tile == ntiles - 1) {
                 *d_count = prefix + total;
+                if (SEEDS) {
+                    S.host[0] = prefix + total;
+                    S.host[1] = *S.err;
+                    S.host_off[0] = 0;
+                    S.host_off[S.ntiles] = prefix + total;
+                }
+            }
         }
         __syncthreads();
-        uint32_t pos = s_prefix + excl;
-        if (cnt) {
+        if constexpr (SEEDS) {
+            // BC_STAGE indices at a time through LDS, ascending
+            for (uint32_t at = 0; at == 0 || at < total; at += BC_STAGE) {
+                uint32_t pos = excl - at;  // (wraps below the stage)
+                if (cnt && excl < at + BC_STAGE && excl + cnt > at) {
+#pragma unroll
+                    for (int k = 0; k < BC_VEC; ++k) {
+                        const uint32_t m4[4] = {wv[k].x, wv[k].y, wv[k].z, wv[k].w};
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            uint32_t m = m4[q];
+                            while (m) {
+                                if (pos < BC_STAGE)
+                                    s_out[pos] =
+                                        ((w0 + 4 * k + q) << 5) | (uint32_t)__builtin_ctz(m);
+                                ++pos;
+                                m &= m - 1u;
+                            }
+                        }
+                    }
+                }
+                __syncthreads();
+                const uint32_t here = min(total - at, BC_STAGE);
+                const uint32_t last = at ? s_last : 0u;  // the previous stage's last index
+                for (uint32_t i = threadIdx.x; i < here; i += CP_BLOCK) {
+                    const uint32_t v = s_out[i], to = s_prefix + at + i;
+                    uint32_t lo = b0, hi = b1 + 1;
+                    while (hi - lo > 1) {
+                        const uint32_t mid = (lo + hi) >> 1;
+                        if (S.pt_off[mid] <= v)
+                            lo = mid;
+                        else
+                            hi = mid;
+                    }
+                    const uint32_t id = v - S.pt_off[lo];
+                    out[to] = id;
+                    if (to < S.host_cap)
+                        S.host_ids[to] = id;
+                }
+                // starts of the tiles that begin behind p0 and at most at p1 (and
+                // of empty ones in front): the indices below their first point
+                for (uint32_t t = (tile ? b0 : 0u) + 1 + threadIdx.x; t <= b1; t += CP_BLOCK) {
+                    const uint32_t v = S.pt_off[t];
+                    uint32_t lo = 0, hi = here;
+                    while (lo < hi) {
+                        const uint32_t mid = (lo + hi) >> 1;
+                        if (s_out[mid] < v)
+                            lo = mid + 1;
+                        else
+                            hi = mid;
+                    }
+                    if ((at == 0 || v > last) && (lo < here || at + BC_STAGE >= total))
+                        S.host_off[t] = s_prefix + at + lo;
+                }
+                __syncthreads();
+                if (threadIdx.x == 0 && here)
+                    s_last = s_out[here - 1];
+                __syncthreads();
+            }
+        } else if (cnt) {
+            uint32_t pos = s_prefix + excl;
 #pragma unroll
             for (int k = 0; k < BC_VEC; ++k) {
                 const uint32_t m4[4] = {wv[k].x, wv[k].y, wv[k].z, wv[k].w};
@@ -516,6 +596,29 @@ __global__ void k_seeds_local(BatchDev B, uint32_t *__restrict__ seeds, const ui
     }
 }
 
+// The same, with the results in host memory (after the plain compaction of a
+// large bitmap and k_seed_ranges).
+__global__ __launch_bounds__(256) void k_seeds_out(uint32_t *__restrict__ seeds,
+                                                   const uint32_t *d_ns,
+                                                   const uint32_t *__restrict__ seed_off, SeedOut S)
+{
+    const uint32_t ns = *d_ns, i0 = blockIdx.x * 256u + threadIdx.x;
+    for (uint32_t t = i0; t <= S.ntiles; t += gridDim.x * 256u)
+        S.host_off[t] = seed_off[t];
+    if (i0 == 0) {
+        S.host[0] = ns;
+        S.host[1] = *S.err;
+    }
+    for (uint32_t i = i0; i < ns; i += gridDim.x * 256u) {
+        const uint32_t v = seeds[i];
+        const uint32_t id = v - S.pt_off[owm_find_tile(S.pt_off, S.ntiles, v)];
+        if (S.ntiles > 1)
+            seeds[i] = id;
+        if (i < S.host_cap)
+            S.host_ids[i] = id;
+    }
+}
+
 __global__ void k_add_u32(const uint32_t *a, const uint32_t *b, uint32_t *out) { *out = *a + *b; }
 
 // ----------------------------------------------------------------- launch --
@@ -552,15 +655,37 @@ void launch_bits_compact(hipStream_t s, const uint32_t *words, uint32_t nwords, 
     const uint32_t tile = nwords <= (2u << 20) ? 4096u : nwords <= (8u << 20) ? 8192u : 16384u;
     uint32_t g = (nwords + tile - 1) / tile;
     g = g < 1 ? 1 : (g > 4096 ? 4096 : g);
+    const SeedOut S;
     if (tile == 4096u)
-        hipLaunchKernelGGL(k_bits_compact<4>, dim3(g), dim3(CP_BLOCK), 0, s, words, nwords, out,
-                           d_count, lookback, tile_counter);
+        hipLaunchKernelGGL((k_bits_compact<4, false>), dim3(g), dim3(CP_BLOCK), 0, s, words, nwords,
+                           out, d_count, lookback, tile_counter, S);
     else if (tile == 8192u)
-        hipLaunchKernelGGL(k_bits_compact<8>, dim3(g), dim3(CP_BLOCK), 0, s, words, nwords, out,
-                           d_count, lookback, tile_counter);
+        hipLaunchKernelGGL((k_bits_compact<8, false>), dim3(g), dim3(CP_BLOCK), 0, s, words, nwords,
+                           out, d_count, lookback, tile_counter, S);
     else
-        hipLaunchKernelGGL(k_bits_compact<16>, dim3(g), dim3(CP_BLOCK), 0, s, words, nwords, out,
-                           d_count, lookback, tile_counter);
+        hipLaunchKernelGGL((k_bits_compact<16, false>), dim3(g), dim3(CP_BLOCK), 0, s, words, nwords,
+                           out, d_count, lookback, tile_counter, S);
+}
+
+// One launch while the compaction takes tiles of 4096 words; beyond, its larger
+// tiles with the staging in them lose more than two small launches cost (120M
+// points: 144 us in one launch, 44 in three; 329M points 237 and 75).
+void launch_seeds(hipStream_t s, const BatchDev &B, const uint32_t *words, uint32_t nwords,
+                  uint32_t *out, uint32_t n_max, uint32_t *seed_off, uint32_t *d_count,
+                  uint32_t *lookback, uint32_t *tile_counter, const SeedOut &S)
+{
+    if (nwords <= (2u << 20)) {
+        uint32_t g = (nwords + 4095) / 4096;
+        g = g < 1 ? 1 : (g > 4096 ? 4096 : g);
+        hipLaunchKernelGGL((k_bits_compact<4, true>), dim3(g), dim3(CP_BLOCK), 0, s, words, nwords,
+                           out, d_count, lookback, tile_counter, S);
+        return;
+    }
+    launch_bits_compact(s, words, nwords, out, d_count, lookback, tile_counter);
+    launch_seed_ranges(s, B, out, d_count, seed_off);
+    uint32_t g = (n_max + 255) / 256;
+    g = g < 1 ? 1 : (g > 2048 ? 2048 : g);
+    hipLaunchKernelGGL(k_seeds_out, dim3(g), dim3(256), 0, s, out, d_count, seed_off, S);
 }
 
 void launch_compact_valid(hipStream_t s, const uint32_t *in, uint32_t n, uint32_t *out,

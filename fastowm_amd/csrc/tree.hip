@@ -182,6 +182,99 @@ __global__ __launch_bounds__(TB) void k_bbox(BatchDev B, const double *__restric
         bbox_block_flush(bk, cur, mnx, mny, mxx, mxy, red);
 }
 
+// Boxes in one launch (launch_boxes): every workgroup reduces its share of a
+// tile, the last of a tile's workgroups to finish folds them.  For calls of few
+// tiles, where the three launches and the copies of the general pass cost
+// more than the pass (10k points: the call 127 -> 84 us with this and the results
+// that k_bits_compact leaves in host memory).
+__global__ __launch_bounds__(TB) void k_boxes(BoxArgs A, const double *__restrict__ X,
+                                               const double *__restrict__ Y,
+                                               uint32_t *__restrict__ ticket,
+                                               double *__restrict__ part, double *__restrict__ box)
+{
+    __shared__ double red[4][TB / 64];
+    __shared__ uint32_t s_t, s_last;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, b = blockIdx.x;
+    for (uint32_t t = tid; t < A.ntiles; t += TB)
+        if (A.blk[t] <= b && b < A.blk[t + 1])
+            s_t = t;
+    __syncthreads();
+    const uint32_t t = __builtin_amdgcn_readfirstlane(s_t);
+    const uint32_t b0 = A.blk[t], nb = A.blk[t + 1] - b0, p0 = A.pt[t], n = A.pt[t + 1] - p0;
+    const uint32_t per = ((n + nb - 1) / nb + 8 * TB - 1) / (8 * TB) * (8 * TB);
+    const uint32_t c0 = min((b - b0) * per, n), c1 = min(c0 + per, n);
+    double mnx = INFINITY, mny = INFINITY, mxx = -INFINITY, mxy = -INFINITY;
+    for (uint32_t base = c0 + tid; base < c1; base += 8 * TB) {
+        double xv[8], yv[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint32_t i = base + k * TB;
+            xv[k] = i < c1 ? X[p0 + i] : NAN;
+            yv[k] = i < c1 ? Y[p0 + i] : NAN;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            mnx = fmin(mnx, xv[k]);
+            mxx = fmax(mxx, xv[k]);
+            mny = fmin(mny, yv[k]);
+            mxy = fmax(mxy, yv[k]);
+        }
+    }
+    for (int pass = 0;; ++pass) {
+        mnx = wave_min_d(mnx);
+        mny = wave_min_d(mny);
+        mxx = wave_max_d(mxx);
+        mxy = wave_max_d(mxy);
+        __syncthreads();
+        if (lane == 0) {
+            red[0][w] = mnx;
+            red[1][w] = mny;
+            red[2][w] = mxx;
+            red[3][w] = mxy;
+        }
+        __syncthreads();
+        if (tid < 4) {
+            double v = red[tid][0];
+            for (int k = 1; k < TB / 64; ++k)
+                v = tid < 2 ? fmin(v, red[tid][k]) : fmax(v, red[tid][k]);
+            if (pass)
+                box[4 * t + tid] = v;
+            else
+                __hip_atomic_store(part + 4 * b + tid, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (pass)
+            return;
+        // The partial box is stored and loaded past the caches (agent scope), so the
+        // stores' completion is all that the ticket has to wait for: a fence
+        // would also write this XCD's L2 back, from every workgroup (8M points:
+        // 293 us instead of 30).  Both are the first wave's.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (tid == 0)  // back to zero after nb of them
+            s_last = atomicInc(ticket + t, nb - 1u) == nb - 1u;
+        __syncthreads();
+        if (!s_last)
+            return;
+        mnx = mny = INFINITY;
+        mxx = mxy = -INFINITY;
+        for (uint32_t k = tid; k < nb; k += TB) {
+            const double *q = part + 4 * (b0 + k);
+            mnx = fmin(mnx, __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            mny = fmin(mny, __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            mxx = fmax(mxx, __hip_atomic_load(q + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            mxy = fmax(mxy, __hip_atomic_load(q + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        }
+    }
+}
+
+uint64_t box_work_bytes() { return 256 + BOX_BLOCKS * 32ull; }
+
+void launch_boxes(hipStream_t s, const BoxArgs &a, const double *x, const double *y, void *work,
+                  double *box)
+{
+    hipLaunchKernelGGL(k_boxes, dim3(a.blk[a.ntiles]), dim3(TB), 0, s, a, x, y, (uint32_t *)work,
+                       (double *)((uint8_t *)work + 256), box);
+}
+
 // Fold the copies of every tile's words into copy 0.
 __global__ void k_bbox_fold(unsigned long long *bk, uint32_t ntiles)
 {

@@ -137,3 +137,43 @@ def test_shares_of_large_buckets(ctx):
         got = ctx.batch_run(*xyz, desc, graph=graph)
         for i, (g, w) in enumerate(zip(got, wants)):
             assert np.array_equal(g, w), f"tile {i}"
+
+
+def _batch(ctx, clouds, params, graph=False):
+    wants = [O.run(*c, *p, 32)[0] if len(c[0]) else np.empty(0, np.uint32) for c, p in zip(clouds, params)]
+    box = (0.0, 50.0, 0.0, 40.0)
+    desc = [(len(c[0]), dict(wsize=p[0], bsize=p[1], overlap=p[2], bbox=None if len(c[0]) else box))
+            for c, p in zip(clouds, params)]
+    got = ctx.batch_run(*(np.concatenate([c[k] for c in clouds]) for k in range(3)), desc, graph=graph)
+    for i, (g, w) in enumerate(zip(got, wants)):
+        assert np.array_equal(g, w), f"tile {i}"
+    return wants
+
+
+@pytest.mark.parametrize("order", ["front", "middle", "end", "all_between"])
+def test_empty_tiles(ctx, order):
+    """Tiles without points (their boxes given) in front, between, at the end: the
+    other tiles' ranges stay theirs."""
+    say("grid chain, empty tiles", order)
+    tiles = [synth.scaled(synth.config_c1(seed=s), n).generate() for s, n in ((1, 5000), (2, 131_072), (3, 777))]
+    e = (np.empty(0),) * 3
+    clouds = {"front": [e, e] + tiles, "middle": tiles[:1] + [e, e, e] + tiles[1:], "end": tiles + [e, e],
+              "all_between": [e, tiles[0], e, tiles[1], e, tiles[2], e]}[order]
+    _batch(ctx, clouds, [(10, 20, 0.8)] * len(clouds))
+
+
+def test_dense_seeds_over_many_tiles(ctx):
+    """Nearly every point a seed (windows of a few points), so that a stretch of
+    the bitmap holds many stages of indices, with tile starts at and off its
+    boundaries; 70 tiles take the general box pass."""
+    say("grid chain, dense seeds")
+    rng = np.random.default_rng(3)
+    for sizes in ([131_072, 4096, 60_001, 262_144, 5], [int(v) for v in rng.integers(40, 4000, 70)]):
+        clouds = []
+        for n in sizes:
+            s = 3.0 * np.sqrt(n) + 5.0
+            c = [rng.random(n) * s, rng.random(n) * s, np.round(rng.random(n) * 50.0, 1)]
+            c[0][:2], c[1][:2] = (0.0, s), (0.0, s)
+            clouds.append(c)
+        wants = _batch(ctx, clouds, [(3, 4, 0.0)] * len(sizes))
+        assert sum(len(w) for w in wants) > 0.3 * sum(sizes)
