@@ -86,7 +86,7 @@ owm_status owm_ctx_create(int device, uint64_t hbm_budget_bytes, owm_ctx **out)
         return OWM_E_DEVICE;
     if (hipSetDevice(device) != hipSuccess)
         return OWM_E_DEVICE;
-    if (owm::grid_kernels_init() != hipSuccess)
+    if (owm::grid_kernels_init() != hipSuccess || owm::qs_kernels_init() != hipSuccess)
         return OWM_E_DEVICE;
     owm_ctx *c = new owm_ctx();
     c->device = device;

@@ -323,6 +323,23 @@ static owm_status take_boxes(owm_ctx *ctx, const double *dx, const double *dy,
     return OWM_OK;
 }
 
+owm_status one_box(owm_ctx *ctx, const double *dx, const double *dy, uint64_t n, double *box,
+                   bool &any)
+{
+    const GridIo io(ctx, 1);
+    if (!io.head) {
+        set_err(ctx, "pinned host allocation failed");
+        return OWM_E_NOMEM;
+    }
+    owm_tile t{};
+    t.n = n;
+    std::vector<std::array<double, 4>> b(1);
+    const owm_status st = take_few_boxes(ctx, dx, dy, &t, 1, io, b);
+    any = st != OWM_E_ARG;
+    memcpy(box, b[0].data(), sizeof b[0]);
+    return any ? st : OWM_OK;
+}
+
 // Everything the chain's launches depend on.
 static void plan_key(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
                      const GridPlan &P, const GridIo &io, std::vector<uint8_t> &key)

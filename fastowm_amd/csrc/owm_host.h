@@ -248,6 +248,10 @@ constexpr uint32_t B_AUTO_GRAPH = 1u << 31;
 owm_status run_batch(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
                      const owm_tile *tiles, uint32_t n_tiles, uint32_t flags, uint32_t *seeds,
                      uint64_t cap, uint64_t *seed_off_host);
+// Exact box (min x, max x, min y, max y) of a cloud of fewer than 2^32 points in
+// device memory; any: it has finite points.
+owm_status one_box(owm_ctx *ctx, const double *dx, const double *dy, uint64_t n, double *box,
+                   bool &any);
 uint64_t tree_bytes(const TreeLayout &L);
 uint64_t query_bytes(const QueryLayout &Q, uint64_t np, uint64_t n_in);
 TreeDev tree_view(const TreeOut &T);

@@ -285,6 +285,38 @@ void launch_qs_path(hipStream_t s, const double *x, const double *y, uint64_t n,
 // offset of createQuadrants at depth d-1).
 void launch_qs_level(hipStream_t s, const QsDev &D, int d, float rd, double off);
 
+// The leaves down to depth QF_DEPTH without sorting (k_qs_part, k_qs_bins,
+// k_qs_out), and of few and small nodes that stay open there (k_qs_deep).
+constexpr int QF_TOP = 5, QF_DEPTH = 12;  // buckets are the depth-5 nodes
+constexpr uint32_t QF_BUCKETS = 1u << (2 * QF_TOP);
+constexpr uint32_t QF_BIN_BITS = 2 * (QF_DEPTH - QF_TOP), QF_BINS = 1u << QF_BIN_BITS;
+constexpr uint32_t QF_SLOT_BITS = 14, QF_PTS = 1u << QF_SLOT_BITS;  // points per sort tile
+constexpr uint32_t QF_NODE_PTS = 1023;  // points of a node that k_qs_deep takes
+constexpr uint32_t QF_OUT = 8192;       // leaf classes that fit the host buffer
+// bits of *flags beyond D.flags': one bucket holds too many points for one
+// workgroup; too many points, or too many in one node, below depth QF_DEPTH
+constexpr uint32_t QF_SKEW = 4, QF_DEEP = 8;
+struct QsFast {
+    QsDev D;
+    QsPath P;
+    double inv, tol;  // 1 / cell side at depth QF_DEPTH; estimates this close to a boundary are not trusted
+    float r0;
+    uint64_t radius_split;  // bit d: minRadius splits occupied nodes of depth d
+    uint32_t nst, bucket_cap;
+    uint32_t *rec;   // [nst * QF_PTS] bin << QF_SLOT_BITS | slot, by bucket within each sort tile
+    uint16_t *tab;   // [nst][QF_BUCKETS + 1] run starts
+    uint32_t *tot;   // [QF_BUCKETS] points per bucket
+    uint32_t *ids;   // points of the nodes open at depth QF_DEPTH, by node
+    uint4 *node;     // {path key, first in ids, points, 0}
+    uint32_t *used;  // [0] ids, [16] nodes
+    uint32_t ids_cap, node_cap;
+    // host memory (page-locked): [0] classes, [1] *novf, [2] *flags, [4 ..] open
+    // nodes per depth, then from word 128 {depth, points, leaves (2 words)}
+    uint32_t *host;
+};
+hipError_t qs_kernels_init();
+void launch_qs_fast(hipStream_t s, const QsFast &F);
+
 // ---- stages (stages.hip) ----
 struct Stage1Cfg {
     uint32_t bx, by;  // window block shape

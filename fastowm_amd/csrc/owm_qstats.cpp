@@ -74,17 +74,16 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
         const uint64_t ovf_cap = n / QS_HB + 1;
         const uint64_t hist_words = (uint64_t)(QS_MAX_DEPTH + 1) * QS_HB;
         const bool need_bbox = !(p->flags & OWM_F_HAVE_BBOX);
-        // layout: [x y] | st | cnt | remap | cen0 | cen1 | nopen | hist | ovf | novf flags | bbox
+        // layout: [x y] | st | cnt | remap | cen0 | cen1 | nopen | hist | ovf | novf flags | sort
         const uint64_t w_xy = device_ptrs ? 0 : al256(n * 8);
         const uint64_t w_st = al256(std::max<uint64_t>(n, 1) * 4), w_sl = al256(slots * 4);
         const uint64_t w_cen = al256(open_cap * 16), w_rng = al256(open_cap * 8);
         const uint64_t w_nopen = al256((QS_MAX_DEPTH + 1) * 4);
         const uint64_t w_hist = al256(hist_words * 8), w_ovf = al256(ovf_cap * 8);
-        const uint64_t w_bb = need_bbox ? al256(bbox_key_words(1) * 8) + 256 : 0;
         // sort scratch for up to 16 sorted depths (4 passes of one key byte)
         const uint64_t w_sort = al256(sort_scratch_bytes(std::max<uint64_t>(n, 1), 4, 1, 0));
         const uint64_t total = 2 * w_xy + w_st + 2 * w_sl + 2 * w_cen + 2 * w_rng + w_nopen +
-                               w_hist + w_ovf + 256 + w_sort + w_bb;
+                               w_hist + w_ovf + 256 + w_sort;
         HIP_TRY(hipStreamSynchronize(s), "sync before the statistics");
         if (ctx->qs_work.bytes < total) {
             if (ctx->budget && ctx->held_bytes() - ctx->qs_work.bytes + total > ctx->budget) {
@@ -139,39 +138,14 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
                 set_err(ctx, "no points to take a bbox from");
                 return OWM_E_ARG;
             }
-            unsigned long long *bk = (unsigned long long *)take(al256(bbox_key_words(1) * 8));
-            uint32_t *ptoff = (uint32_t *)take(256);
-            uint8_t *h = ctx->pinned(ctx->h_io, ctx->h_io_cap, 256);
-            if (!h) {
-                set_err(ctx, "pinned host allocation failed");
-                return OWM_E_NOMEM;
-            }
-            const uint32_t po[2] = {0, (uint32_t)n};
-            memcpy(h, po, 8);
-            HIP_TRY(hipMemcpyAsync(ptoff, h, 8, hipMemcpyHostToDevice, s), "bbox offsets");
-            BatchDev B0{};
-            B0.ntiles = 1;
-            B0.np = (uint32_t)n;
-            B0.pt_off = ptoff;
-            launch_bbox_init(s, bk, 1);
-            launch_bbox(s, B0, dx, dy, bk);
-            HIP_TRY(hipMemcpyAsync(h + 64, bk, 32, hipMemcpyDeviceToHost, s), "bbox D2H");
-            HIP_TRY(hipStreamSynchronize(s), "bbox");
-            const unsigned long long *hk = (const unsigned long long *)(h + 64);
-            if (hk[0] == ~0ull || hk[1] == ~0ull) {
+            bool any = false;
+            const owm_status st = one_box(ctx, dx, dy, n, box, any);
+            if (st != OWM_OK)
+                return st;
+            if (!any) {
                 set_err(ctx, "no finite points to take a bbox from");
                 return OWM_E_ARG;
             }
-            auto dec = [](unsigned long long k) {
-                uint64_t b = (k >> 63) ? (k & 0x7FFFFFFFFFFFFFFFull) : ~k;
-                double v;
-                memcpy(&v, &b, 8);
-                return v;
-            };
-            box[0] = dec(hk[0]);
-            box[1] = dec(hk[2]);
-            box[2] = dec(hk[1]);
-            box[3] = dec(hk[3]);
         } else {
             memcpy(box, p->bbox, sizeof box);
         }
@@ -205,7 +179,110 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
         }
         D.sort_levels = sl;
         const int passes = sl / 4;
-
+        std::vector<owm_leaf_bin> cls;
+        std::vector<uint32_t> nopen;
+        std::vector<uint2> ovf;
+        int last = 0;
+        auto too_deep = [&]() {
+            if (p->policy == OWM_QT_MAXNUMBER)
+                set_err(ctx, "a node holds more than %u points below depth %d: the "
+                             "reference quadtree never stops splitting there",
+                        p->max_number, QS_MAX_DEPTH);
+            else
+                set_err(ctx, "minRadius %g: occupied nodes split below depth %d",
+                        (double)p->min_radius, QS_MAX_DEPTH);
+            return OWM_E_ARG;
+        };
+        bool done = false;
+        // Without sorting where leaves are expected down to depth 12: from 32768
+        // points on (100k points: 230 us instead of 560), and up to 2^28 (one
+        // workgroup reads a bucket's runs of every sort tile).  A cloud most of
+        // whose points share one bucket, or with many points below depth 12, is
+        // sorted after all.
+        if (sl == QF_DEPTH && n >= 32768 && n < (1ull << 28)) {
+            QsFast F{};
+            F.D = D;
+            F.P.cx = cx;
+            F.P.cy = cy;
+            for (int k = 0; k < QS_KEY_LEVELS; ++k)
+                F.P.off[k] = (double)(depth_radius(r0, k) * 0.5f);
+            // the depth-12 cell's side is the depth-10 offset; below 2^-100 the
+            // float radii would not halve exactly
+            const double side = F.P.off[QF_DEPTH - 2];
+            const double bound = std::max(std::fabs(cx), std::fabs(cy)) + 2.0 * (double)r0;
+            F.inv = 1.0 / side;
+            F.tol = side > 0x1p-100 ? std::ldexp(bound, -45) * F.inv : 1.0;
+            F.r0 = r0;
+            for (int k = 0; k <= QF_DEPTH; ++k)
+                if ((double)depth_radius(r0, k) * 0.5 > (double)p->min_radius)
+                    F.radius_split |= 1ull << k;
+            F.nst = (uint32_t)((n + QF_PTS - 1) / QF_PTS);
+            F.bucket_cap = (uint32_t)std::max<uint64_t>(8 * n / QF_BUCKETS, 1u << 18);
+            F.ids_cap = (uint32_t)(n / 8);
+            F.node_cap = (uint32_t)(n / 64);
+            uint8_t *q = sort_base;  // 16 bytes a point and more; this takes about 5
+            auto part = [&q](uint64_t b) { uint8_t *r = q; q += al256(b); return r; };
+            F.rec = (uint32_t *)part((uint64_t)F.nst * QF_PTS * 4);
+            F.tab = (uint16_t *)part((uint64_t)F.nst * (QF_BUCKETS + 1) * 2);
+            F.tot = (uint32_t *)part(QF_BUCKETS * 4);
+            F.used = (uint32_t *)part(128);
+            F.ids = (uint32_t *)part((uint64_t)F.ids_cap * 4);
+            F.node = (uint4 *)part((uint64_t)F.node_cap * 16);
+            F.host = (uint32_t *)ctx->pinned(ctx->h_io, ctx->h_io_cap, 512 + QF_OUT * 16);
+            if (!F.host) {
+                set_err(ctx, "pinned host allocation failed");
+                return OWM_E_NOMEM;
+            }
+            const int pi = ctx->prof.begin(s, PH_QSTATS);
+            FillRanges z;
+            z.count = 2;
+            z.ptr[0] = (uint32_t *)zero_from;
+            z.len[0] = (uint64_t)(zero_end - zero_from) / 4;
+            z.ptr[1] = F.used;
+            z.len[1] = 32;
+            launch_fill_ranges(s, z);
+            launch_qs_fast(s, F);
+            ctx->prof.end(s, pi, 0, 0, p->policy == OWM_QT_MAXNUMBER ? 5 : 4);
+            HIP_TRY(hipGetLastError(), "statistics launch");
+            HIP_TRY(hipStreamSynchronize(s), "statistics");
+            const uint32_t n_cls = F.host[0], novf = F.host[1], flags = F.host[2];
+            if (flags & 3u) {
+                set_err(ctx, "statistics capacity guard tripped (flags %u)", flags);
+                return OWM_E_INTERNAL;
+            }
+            if (!(flags & (QF_SKEW | QF_DEEP)) && n_cls <= QF_OUT) {
+                done = true;
+                nopen.assign(F.host + 4, F.host + 4 + QS_MAX_DEPTH + 1);
+                if (nopen[QS_MAX_DEPTH])
+                    return too_deep();
+                while (nopen[last])
+                    ++last;
+                struct Cls {
+                    uint32_t depth, points;
+                    uint32_t leaves[2];
+                };
+                const Cls *h = (const Cls *)(F.host + 128);
+                for (uint32_t k = 0; k < n_cls; ++k)
+                    cls.push_back({h[k].depth, h[k].points,
+                                   (uint64_t)h[k].leaves[1] << 32 | h[k].leaves[0]});
+                ovf.resize(novf);
+                if (novf)
+                    HIP_TRY(hipMemcpy(ovf.data(), D.ovf, (uint64_t)novf * 8, hipMemcpyDeviceToHost),
+                            "large leaves D2H");
+                if (novf) {
+                    std::map<std::pair<uint32_t, uint32_t>, uint64_t> big;
+                    for (const uint2 &e : ovf)
+                        ++big[{e.x, e.y}];
+                    for (const auto &e : big)
+                        cls.push_back({e.first.first, e.first.second, e.second});
+                    std::sort(cls.begin(), cls.end(), [](const owm_leaf_bin &a, const owm_leaf_bin &b) {
+                        return a.level != b.level ? a.level < b.level : a.points < b.points;
+                    });
+                }
+                ctx->prof.collect();
+            }
+        }
+        if (!done) {
         int pi = ctx->prof.begin(s, PH_QSTATS);
         launch_fill_u32(s, D.cnt, slots, 0u);
         launch_fill_u32(s, (uint32_t *)zero_from, (uint64_t)(zero_end - zero_from) / 4, 0u);
@@ -236,7 +313,7 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
         }
         // depths in groups of up to 6 (the key-range depths and the point
         // depths apart), then one readback of the open-node counts
-        int d = 1, last = 0;
+        int d = 1;
         float r = r0;
         while (true) {
             if (d == QS_KEY_LEVELS + 1) {
@@ -284,25 +361,17 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
                     ;
                 break;  // the depth-`last` nodes are all leaves
             }
-            if (upto == QS_MAX_DEPTH) {
-                if (p->policy == OWM_QT_MAXNUMBER)
-                    set_err(ctx, "a node holds more than %u points below depth %d: the "
-                                 "reference quadtree never stops splitting there",
-                            p->max_number, QS_MAX_DEPTH);
-                else
-                    set_err(ctx, "minRadius %g: occupied nodes split below depth %d",
-                            (double)p->min_radius, QS_MAX_DEPTH);
-                return OWM_E_ARG;
-            }
+            if (upto == QS_MAX_DEPTH)
+                return too_deep();
         }
         const uint32_t novf = hn[QS_MAX_DEPTH + 1], flags = hn[QS_MAX_DEPTH + 2];
-        std::vector<uint32_t> nopen(hn, hn + QS_MAX_DEPTH + 1);
+        nopen.assign(hn, hn + QS_MAX_DEPTH + 1);
         if (flags) {
             set_err(ctx, "statistics capacity guard tripped (flags %u)", flags);
             return OWM_E_INTERNAL;
         }
         std::vector<unsigned long long> hist((uint64_t)(last + 1) * QS_HB);
-        std::vector<uint2> ovf(novf);
+        ovf.resize(novf);
         HIP_TRY(hipMemcpyAsync(hist.data(), D.hist, hist.size() * 8, hipMemcpyDeviceToHost, s),
                 "histogram D2H");
         if (novf)
@@ -314,13 +383,13 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
         std::map<std::pair<uint32_t, uint32_t>, uint64_t> big;
         for (const uint2 &e : ovf)
             ++big[{e.x, e.y}];
-        std::vector<owm_leaf_bin> cls;
         for (int dd = 0; dd <= last; ++dd) {
             for (uint32_t c = 0; c < QS_HB; ++c)
                 if (hist[(uint64_t)dd * QS_HB + c])
                     cls.push_back({(uint32_t)dd, c, hist[(uint64_t)dd * QS_HB + c]});
             for (auto it = big.lower_bound({(uint32_t)dd, 0}); it != big.end() && it->first.first == (uint32_t)dd; ++it)
                 cls.push_back({it->first.first, it->first.second, it->second});
+        }
         }
         uint64_t leaves = 0, settled = 0, routed = 0;
         for (const auto &c : cls) {
@@ -342,14 +411,15 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
         // per routed point its key or coordinates, node and new state (at
         // least 12), per child slot its count (read and cleared) and remap
         // (12), per new open node a centre
-        uint64_t alg = 20 * n;
-        for (int dd = 1; dd <= last; ++dd) {
+        // (without sorting: x and y read, a record written and read)
+        uint64_t alg = done ? 24 * n : 20 * n;
+        for (int dd = 1; dd <= last && !done; ++dd) {
             if (dd <= sl)
                 alg += 36ull * nopen[dd - 1] + 24ull * nopen[dd];
             else
                 alg += 4 * n + 12 * 4ull * nopen[dd - 1] + 16ull * nopen[dd];
         }
-        if (last > sl)
+        if (last > sl && !done)
             alg += 4 * n + 12 * routed;
         ctx->prof.add_work(PH_QSTATS, alg, n);
         memcpy(out->bbox, box, sizeof box);

@@ -217,3 +217,58 @@ def test_full_size_invariants(ctx):
     assert sum(c * k for _, c, k in got) == len(x)
     # minRadius 0.1 on a 2 km box: every occupied node splits down to depth 13
     assert {d for d, c, _ in got if c > 0} == {13}
+
+
+def _launches(ctx, x, y, box, policy, **kw):
+    ctx.profile(True)
+    both(ctx, x, y, box, policy, **kw)
+    n = ctx.profile_read()["qtree_stats"]["calls"]
+    ctx.profile(False)
+    return n
+
+
+@pytest.mark.parametrize("n", [32_768, 49_152, 70_001, 300_000])
+@pytest.mark.parametrize("max_number,level", [(1, 0), (16, 3), (64, 6), (1500, 2)])
+def test_without_sorting_maxnumber(ctx, n, max_number, level):
+    """The counts of the buckets alone (from 32768 points on), around whole sort
+    tiles; leaves beyond the exact bins at max_number 1500."""
+    say("without sorting", n, max_number, level)
+    x, y, _ = tile_for({"cluster_frac": 0.3, "n_clusters": 9, "cluster_sigma": 4.0}, n).generate()
+    n = _launches(ctx, x, y, synth.bbox(x, y), owm.QT_MAXNUMBER, max_number=max_number, level=level)
+    assert n == 5 or max_number == 1  # at one point a leaf much of the clusters lies below depth 12
+
+
+@pytest.mark.parametrize("radius,level", [(0.5, 3), (2.0, 6), (30.0, 0)])
+def test_without_sorting_minradius(ctx, radius, level):
+    say("without sorting, radius", radius, level)
+    x, y, _ = tile_for({}, 60_000).generate()
+    assert _launches(ctx, x, y, synth.bbox(x, y), owm.QT_MINRADIUS, min_radius=radius, level=level) == 4
+
+
+def test_without_sorting_on_centre_lines(ctx):
+    """A lattice whose every point lies on centre lines of depths up to 12, and
+    its neighbours one ulp either side."""
+    say("without sorting, centre lines")
+    g = np.arange(0, 4097, 16, dtype=np.float64)
+    x, y = (a.ravel() for a in np.meshgrid(g, g))
+    x, y = np.append(x, np.nextafter(x, 0.0)), np.append(y, np.nextafter(y, 1e9))
+    for box in ((0.0, 4096.0, 0.0, 4096.0), (-3.0, 4099.5, 0.0, 4096.0)):
+        # (two points: those at x = 0 have their neighbour on the same spot)
+        assert _launches(ctx, x, y, box, owm.QT_MAXNUMBER, max_number=2, level=2) == 5
+
+
+def test_nodes_below_the_counted_depths(ctx):
+    """Nodes still split at depth 12: few and small ones are followed without
+    sorting; one of more than 1023 points, or a cloud in one bucket, is sorted."""
+    say("nodes below depth 12")
+    rng = np.random.default_rng(8)
+    for pts, spread, counted in ((900, 1e-3, True), (900, 1e-6, True), (1500, 1e-3, False)):
+        x, y, _ = tile_for({}, 60_000).generate()
+        for k in range(6):
+            i = rng.integers(0, len(x), pts)
+            x[i], y[i] = x[k] + spread * rng.random(pts), y[k] + spread * rng.random(pts)
+        n = _launches(ctx, x, y, synth.bbox(x, y), owm.QT_MAXNUMBER, max_number=32, level=3)
+        assert (n == 5) == counted
+    x, y, _ = tile_for({}, 400_000).generate()
+    x[0], y[0] = x[0] + 1e6, y[0] + 1e6
+    assert _launches(ctx, x, y, synth.bbox(x, y), owm.QT_MAXNUMBER, max_number=32, level=3) > 5
