@@ -129,7 +129,10 @@ void owm_ctx_destroy(owm_ctx *ctx)
     delete ctx;
 }
 
-uint64_t owm_ctx_device_bytes(const owm_ctx *ctx) { return ctx ? ctx->held_bytes() : 0; }
+uint64_t owm_ctx_device_bytes(const owm_ctx *ctx)
+{
+    return ctx ? const_cast<owm_ctx *>(ctx)->held_bytes() : 0;
+}
 
 owm_status owm_host_alloc(uint64_t bytes, void **out)
 {
@@ -202,7 +205,7 @@ owm_status upload_cloud(owm_ctx *ctx, const double *x, const double *y, const do
 {
     uint64_t b = al256(n * 8ull);
     if (ctx->upload.bytes < 3 * b) {
-        if (ctx->budget && ctx->held_bytes() - ctx->upload.bytes + 3 * b > ctx->budget) {
+        if (ctx->exceeds(3 * b, &ctx->upload)) {
             set_err(ctx, "input upload needs %llu bytes over the budget", (unsigned long long)(3 * b));
             return OWM_E_BUDGET;
         }
@@ -363,13 +366,27 @@ owm_status owm_tree_build(owm_ctx *ctx, const double *x, const double *y, const 
     tr->P.Q.cell_off.assign(2, 0);
     tr->P.Q.blk_off.assign(2, 0);
     const uint64_t tb = tree_bytes(tr->P.L);
-    if (ctx->budget && ctx->held_bytes() + tb > ctx->budget) {
-        set_err(ctx, "tree needs %llu device bytes over the budget", (unsigned long long)tb);
-        return OWM_E_BUDGET;
+    {
+        // the last freed tree's memory when it fits without waste
+        std::lock_guard<std::mutex> g(ctx->spare_mu);
+        if (ctx->spare.bytes >= tb && ctx->spare.bytes / 2 <= tb)
+            tr->mem.swap(ctx->spare);
     }
-    hipError_t e = tr->mem.reserve(tb, tb);
-    if (e != hipSuccess)
-        return hip_fail(ctx, e, "tree allocation");
+    hipError_t e = hipSuccess;
+    if (!tr->mem.ptr) {
+        if (ctx->exceeds(tb)) {
+            set_err(ctx, "tree needs %llu device bytes over the budget", (unsigned long long)tb);
+            return OWM_E_BUDGET;
+        }
+        e = tr->mem.reserve(tb, tb);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            ctx->release_spare();
+            e = tr->mem.reserve(tb, tb);
+        }
+        if (e != hipSuccess)
+            return hip_fail(ctx, e, "tree allocation");
+    }
     ctx->trees_bytes += tr->mem.bytes;
     carve_tree((uint8_t *)tr->mem.ptr, tr->P.L, tr->T);
     st = ctx->arena.ensure(ctx, table_bytes(1) + build_scratch_bytes(tr->P.L) + 8192);
@@ -412,6 +429,9 @@ void owm_tree_free(owm_tree *tree)
     if (tree->ctx) {
         (void)hipStreamSynchronize(tree->ctx->stream);
         tree->ctx->trees_bytes -= tree->mem.bytes;
+        std::lock_guard<std::mutex> g(tree->ctx->spare_mu);
+        if (tree->mem.bytes <= owm_ctx::SPARE_MAX && tree->mem.bytes >= tree->ctx->spare.bytes)
+            tree->mem.swap(tree->ctx->spare);  // what it held before is freed with the tree
     }
     delete tree;
 }

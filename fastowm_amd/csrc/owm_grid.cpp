@@ -416,8 +416,7 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
                           up256(P.list_cap * GRID_POOLS * 4) + up256(GRID_POOLS * 128) + 2 * up256((nwords + 4) * 4) +
                           up256((gcells + 1) * 4) + up256((nwords / 4096 + 2) * 4) +
                           up256(nseed * 4) + up256((T + 1) * 4ull) + 4096;
-    const uint64_t others = ctx->held_bytes() - ctx->arena.buf.bytes;
-    if (ctx->budget && others + std::max(need, tree_chain_bound(P)) > ctx->budget)
+    if (ctx->exceeds(std::max(need, tree_chain_bound(P)), &ctx->arena.buf))
         return hand_on();
     void *old_arena = ctx->arena.buf.ptr;
     st = ctx->arena.ensure(ctx, need);

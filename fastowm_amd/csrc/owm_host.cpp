@@ -850,7 +850,7 @@ owm_status Arena::ensure(owm_ctx *ctx, uint64_t bytes)
     used = 0;
     if (bytes <= buf.bytes)
         return OWM_OK;
-    if (ctx->budget && ctx->held_bytes() - buf.bytes + bytes > ctx->budget) {
+    if (ctx->exceeds(bytes, &buf)) {
         set_err(ctx, "work needs %llu device bytes, budget is %llu", (unsigned long long)bytes,
                 (unsigned long long)ctx->budget);
         return OWM_E_BUDGET;
@@ -859,6 +859,11 @@ owm_status Arena::ensure(owm_ctx *ctx, uint64_t bytes)
     if (e != hipSuccess)
         return hip_fail(ctx, e, "sync before arena growth");
     e = buf.reserve(bytes, ctx->room_for(buf));
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        ctx->release_spare();
+        e = buf.reserve(bytes, ctx->room_for(buf));
+    }
     if (this == &ctx->arena)
         ctx->graphs.clear();  // captured chains point into the old arena
     if (e != hipSuccess)
@@ -1179,7 +1184,7 @@ owm_status ensure_s1_list(owm_ctx *ctx, uint64_t cap)
 {
     if (cap * 4 <= ctx->s1_list.bytes)
         return OWM_OK;
-    if (ctx->budget && ctx->held_bytes() - ctx->s1_list.bytes + cap * 4 > ctx->budget) {
+    if (ctx->exceeds(cap * 4, &ctx->s1_list)) {
         set_err(ctx, "stage-1 join list needs %llu bytes over the budget", (unsigned long long)(cap * 4));
         return OWM_E_BUDGET;
     }
@@ -1562,7 +1567,7 @@ bool owm_ctx::stage_table(const std::vector<TileDev> &td, const TreeLayout &L, c
     return true;
 }
 
-uint64_t owm_ctx::room_for(const owm::DevBuf &b) const
+uint64_t owm_ctx::room_for(const owm::DevBuf &b)
 {
     if (!budget)
         return ~0ull;
@@ -1570,12 +1575,30 @@ uint64_t owm_ctx::room_for(const owm::DevBuf &b) const
     return budget > others ? budget - others : 0;
 }
 
-uint64_t owm_ctx::held_bytes() const
+uint64_t owm_ctx::held_bytes()
 {
     uint64_t b = arena.buf.bytes + small.buf.bytes + upload.bytes + s1_list.bytes;
     b += box_work.bytes + xyz_text.bytes + xyz_work.bytes + xyz_cloud.bytes + qs_work.bytes;
     b += trees_bytes.load();
-    return b;
+    std::lock_guard<std::mutex> g(spare_mu);
+    return b + spare.bytes;
+}
+
+void owm_ctx::release_spare()
+{
+    std::lock_guard<std::mutex> g(spare_mu);
+    spare.release();
+}
+
+bool owm_ctx::exceeds(uint64_t need, const owm::DevBuf *old)
+{
+    if (!budget)
+        return false;
+    need -= old ? old->bytes : 0;
+    if (held_bytes() + need <= budget)
+        return false;
+    release_spare();
+    return held_bytes() + need > budget;
 }
 
 

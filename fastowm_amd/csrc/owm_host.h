@@ -28,6 +28,12 @@ struct DevBuf {
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf();
     void release();
+    void swap(DevBuf &o)
+    {
+        std::swap(ptr, o.ptr);
+        std::swap(bytes, o.bytes);
+        std::swap(borrowed, o.borrowed);
+    }
     // Grows to at least `need` bytes (with 25% headroom, never above `cap`).
     hipError_t reserve(uint64_t need, uint64_t cap = ~0ull);
 };
@@ -322,6 +328,16 @@ struct owm_ctx {
     owm::DevBuf xyz_text, xyz_work, xyz_cloud;
     owm::DevBuf qs_work;  // quadtree statistics: point state, child slots, histograms
     uint64_t s1_need_max = 0;  // largest join that overflowed its first estimate
+    // The last freed tree's device memory, kept for the next build (allocating and
+    // freeing 130 MB takes 0.37 ms, a third of a 3M-point tree's use): at most
+    // SPARE_MAX bytes, counted as held, given back when the budget or an
+    // allocation needs them, and with the context.  Trees are freed from any thread.
+    static constexpr uint64_t SPARE_MAX = 512ull << 20;
+    std::mutex spare_mu;
+    owm::DevBuf spare;
+    void release_spare();
+    // Whether `need` bytes more (with `old` released) exceed the budget.
+    bool exceeds(uint64_t need, const owm::DevBuf *old = nullptr);
     owm::Tuner tuner;
     std::atomic<uint64_t> trees_bytes{0};
     // pinned host staging: the tile table (tiles, then eight offset arrays, in
@@ -341,9 +357,9 @@ struct owm_ctx {
     // copies the tile table into h_tab (false: no pinned memory)
     bool stage_table(const std::vector<::TileDev> &td, const owm::TreeLayout &L,
                      const owm::QueryLayout &Q);
-    uint64_t held_bytes() const;
+    uint64_t held_bytes();
     // Largest size buffer `b` may grow to without exceeding the budget.
-    uint64_t room_for(const owm::DevBuf &b) const;
+    uint64_t room_for(const owm::DevBuf &b);
     ~owm_ctx();
 };
 

@@ -86,7 +86,7 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
                                w_hist + w_ovf + 256 + w_sort;
         HIP_TRY(hipStreamSynchronize(s), "sync before the statistics");
         if (ctx->qs_work.bytes < total) {
-            if (ctx->budget && ctx->held_bytes() - ctx->qs_work.bytes + total > ctx->budget) {
+            if (ctx->exceeds(total, &ctx->qs_work)) {
                 set_err(ctx, "quadtree statistics need %llu bytes over the budget",
                         (unsigned long long)total);
                 return OWM_E_BUDGET;

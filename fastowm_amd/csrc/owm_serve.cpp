@@ -116,7 +116,7 @@ static void run_group(ServeState *S, owm_ctx *slot, std::vector<std::shared_ptr<
     inplace = inplace && x0 != nullptr;
     owm_status st = OWM_OK;
     if (!inplace && slot->upload.bytes < 3 * b) {
-        if (slot->held_bytes() - slot->upload.bytes + 3 * b > slot->budget) {
+        if (slot->exceeds(3 * b, &slot->upload)) {
             set_err(slot, "group input needs %llu bytes over the slot budget",
                     (unsigned long long)(3 * b));
             st = OWM_E_BUDGET;

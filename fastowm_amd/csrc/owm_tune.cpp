@@ -165,7 +165,7 @@ owm_status owm_autotune(owm_ctx *ctx, const double *x, const double *y, const do
             if (pick.empty())
                 continue;
             const uint64_t b = (pts * 8 + 255) / 256 * 256;
-            if (ctx->budget && ctx->held_bytes() + 3 * b > ctx->budget)
+            if (ctx->exceeds(3 * b))
                 continue;  // no room for a trial copy: keep the default
             HIP_TRY(hipStreamSynchronize(ctx->stream), "tune sync");
             HIP_TRY(sub.reserve(3 * b), "tune buffer");
