@@ -122,6 +122,9 @@ __global__ __launch_bounds__(256) void k_grid_prep(GridDev G, FillRanges r, uint
 // workgroups per CU, centimetre coordinates and clusters ran slower: 8M points
 // 78 us instead of 66, 96 mixed tiles 1.20 ms instead of 1.00; without points
 // near edges it was 2.15 ms against 2.27 for the 329M points).
+// TREE: the points come from a resident tree, whose order only groups them (33 us
+// for its 3M points).
+template <bool TREE>
 __global__ __launch_bounds__(GP_NT, 6) void k_grid_part(GridDev G, const double *__restrict__ X,
                                                       const double *__restrict__ Y,
                                                       const double *__restrict__ Z)
@@ -146,12 +149,20 @@ __global__ __launch_bounds__(GP_NT, 6) void k_grid_part(GridDev G, const double 
 #pragma unroll
     for (int k = 0; k < GP_K; ++k) {
         const uint32_t i = base + min(tid + k * GP_NT, cnt - 1u);
-        x[k] = X[i];
-        y[k] = Y[i];
+        if (TREE) {
+            const double2 v = G.xy[i];
+            x[k] = v.x;
+            y[k] = v.y;
+        } else {
+            x[k] = X[i];
+            y[k] = Y[i];
+        }
     }
 #pragma unroll
-    for (int k = 0; k < GP_K; ++k)
-        z[k] = Z[base + min(tid + k * GP_NT, cnt - 1u)];
+    for (int k = 0; k < GP_K; ++k) {
+        const uint32_t i = base + min(tid + k * GP_NT, cnt - 1u);
+        z[k] = TREE ? G.zi[i].z : Z[i];
+    }
     for (uint32_t b = tid; b < nb; b += GP_NT)
         hist[b] = 0;
     uint32_t key[GP_K];
@@ -174,8 +185,10 @@ __global__ __launch_bounds__(GP_NT, 6) void k_grid_part(GridDev G, const double 
         for (uint32_t e = tid; e < nl; e += GP_NT) {
             const uint32_t slot = sList[e];
             uint32_t cx, cy;
-            const bool okx = axis_col_exact(T.ax[0], axis_passed(T.ax[0], X[base + slot]), cx);
-            const bool oky = axis_col_exact(T.ax[1], axis_passed(T.ax[1], Y[base + slot]), cy);
+            const double xs = TREE ? G.xy[base + slot].x : X[base + slot];
+            const double ys = TREE ? G.xy[base + slot].y : Y[base + slot];
+            const bool okx = axis_col_exact(T.ax[0], axis_passed(T.ax[0], xs), cx);
+            const bool oky = axis_col_exact(T.ax[1], axis_passed(T.ax[1], ys), cy);
             sW[slot] = grid_key(T, cx, cy) | (okx && oky ? 0u : KEY_RARE);
             if (!(okx && oky))
                 atomicAdd(&s_nr, 1u);
@@ -203,11 +216,12 @@ __global__ __launch_bounds__(GP_NT, 6) void k_grid_part(GridDev G, const double 
                 sPool[slot] = pbase != OWM_NONE ? at : 0u;
                 if (pbase == OWM_NONE)
                     continue;
-                const AxisPassed px = axis_passed(T.ax[0], X[i]), py = axis_passed(T.ax[1], Y[i]);
-                const double zi = Z[i];
+                const AxisPassed px = axis_passed(T.ax[0], TREE ? G.xy[i].x : X[i]);
+                const AxisPassed py = axis_passed(T.ax[1], TREE ? G.xy[i].y : Y[i]);
+                const double zi = TREE ? G.zi[i].z : Z[i];
                 GridRare r;
                 r.zk = owm_eligible(zi) ? owm_zkey(zi) : OWM_ZKEY_NONE;
-                r.id = i;
+                r.id = TREE ? G.zi[i].id : i;
                 r.pad = 0;
                 r.wx0 = (uint16_t)px.w_lo;
                 r.wx1 = (uint16_t)px.w_hi;
@@ -330,7 +344,7 @@ __device__ __forceinline__ void flush_rare(const GridDev &G, uint32_t item, cons
 // 0.83 ms against separate key and cell streams, two lanes a segment instead of
 // four to eight 0.74, lane masks instead of bit sets 0.71 ms.  One spare cell for
 // all idle lanes instead of one per lane: 3.1 instead of 1.3 ms (329M points).
-template <int NT, int TWO>
+template <int NT, int TWO, bool TREE>
 __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_t t1,
                                                  uint32_t item0, uint32_t items, uint32_t cells)
 {
@@ -470,8 +484,14 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
                 __syncthreads();
 #pragma unroll
                 for (int k = 0; k < KK; ++k)
-                    if (eq[k])
-                        atomicMin(&sId[cell[k]], id0[k / GB_SEG] + (cw[k] & GRID_SLOT_MASK));
+                    if (eq[k]) {
+                        const uint32_t i = id0[k / GB_SEG] + (cw[k] & GRID_SLOT_MASK);
+                        // (idle lanes may point anywhere: theirs is the spare cell)
+                        if (!TREE)
+                            atomicMin(&sId[cell[k]], i);
+                        else if (cell[k] < nc)
+                            atomicMin(&sId[cell[k]], G.zi[i].id);
+                    }
             }
             __syncthreads();  // sRun is rewritten
         }
@@ -540,7 +560,8 @@ __device__ __forceinline__ void mark_llp(const GridDev &G, const GridTile &T, ui
     const uint32_t bit = 1u << (id & 31u);
     if ((atomicOr(G.llp + (id >> 5), bit) & bit) || T.ax[0].g.n == 0)
         return;
-    const double x = X[id], y = Y[id];
+    const double2 xy = G.pos ? G.xy[G.pos[id]] : make_double2(X[id], Y[id]);
+    const double x = xy.x, y = xy.y;
     const uint32_t x0 = axis_count(T.ax[0].g, x, true, true), x1 = axis_count(T.ax[0].g, x, false, false);
     const uint32_t y0 = axis_count(T.ax[1].g, y, true, true), y1 = axis_count(T.ax[1].g, y, false, false);
     for (uint32_t j = y0; j < y1; ++j)
@@ -743,10 +764,15 @@ __global__ __launch_bounds__(GW_NT) void k_grid_windows(GridDev G, const double 
         const uint32_t q = tid + k * GW_NT;
         if (q < bw * bw) {
             const bool valid = win[k].cnt >= T.min_num_points && win[k].zk != OWM_ZKEY_NONE;
-            win[k].id = valid && (q >> lb) < nj && (q & (bw - 1u)) < ni ? win[k].id : OWM_NONE;
+            const bool in = (q >> lb) < nj && (q & (bw - 1u)) < ni;
+            win[k].id = valid && in ? win[k].id : OWM_NONE;
             sMin[q] = win[k].id;
+            if (G.min_ids && in)
+                G.min_ids[(uint64_t)(j0 + (q >> lb)) * nx + i0 + (q & (bw - 1u))] = win[k].id;
         }
     }
+    if (G.min_ids)
+        return;
     __syncthreads();
     uint32_t act[GW_PER], old[GW_PER];
 #pragma unroll
@@ -858,7 +884,10 @@ void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const do
     if (!sort_tiles)
         return;
     const uint32_t lds = GRID_PTS * 12u + max_nb * 4u;
-    hipLaunchKernelGGL(k_grid_part, dim3(sort_tiles), dim3(GP_NT), lds, s, G, x, y, z);
+    if (G.zi)
+        hipLaunchKernelGGL(k_grid_part<true>, dim3(sort_tiles), dim3(GP_NT), lds, s, G, x, y, z);
+    else
+        hipLaunchKernelGGL(k_grid_part<false>, dim3(sort_tiles), dim3(GP_NT), lds, s, G, x, y, z);
 }
 
 // LDS of the bins: the cells and 64 spare ones.
@@ -873,11 +902,19 @@ void launch_grid_bin(hipStream_t s, const GridDev &G, uint32_t t0, uint32_t t1, 
     // 512 threads where LDS or the number of items leaves few workgroups to a CU
     // (120M points, 64 KB of cells: 1.50 ms with 256 threads, 1.13 with 512; 1M
     // points: 29 and 21 us; 329M points in 27,700 items: 1.00 and 1.04 ms)
-    if (cells > 1024 || items <= 1024)
-        hipLaunchKernelGGL((k_grid_bin<512, 1>), dim3(g), dim3(512), BIN_LDS(cells), s, G, t0, t1,
+    const bool wide = cells > 1024 || items <= 1024;
+    const dim3 grid(g), block(wide ? 512 : 256);
+    if (G.zi && wide)
+        hipLaunchKernelGGL((k_grid_bin<512, 1, true>), grid, block, BIN_LDS(cells), s, G, t0, t1,
+                           item0, items, cells);
+    else if (G.zi)
+        hipLaunchKernelGGL((k_grid_bin<256, 1, true>), grid, block, BIN_LDS(cells), s, G, t0, t1,
+                           item0, items, cells);
+    else if (wide)
+        hipLaunchKernelGGL((k_grid_bin<512, 1, false>), grid, block, BIN_LDS(cells), s, G, t0, t1,
                            item0, items, cells);
     else
-        hipLaunchKernelGGL((k_grid_bin<256, 1>), dim3(g), dim3(256), BIN_LDS(cells), s, G, t0, t1,
+        hipLaunchKernelGGL((k_grid_bin<256, 1, false>), grid, block, BIN_LDS(cells), s, G, t0, t1,
                            item0, items, cells);
 }
 
@@ -899,14 +936,24 @@ void launch_grid_cells(hipStream_t s, const GridDev &G)
     hipLaunchKernelGGL(k_grid_cells, dim3(g), dim3(256), 0, s, G);
 }
 
+__global__ void k_flags_out(const uint32_t *flags, uint32_t *host) { *host = *flags; }
+
+void launch_flags_out(hipStream_t s, const uint32_t *flags, uint32_t *host)
+{
+    hipLaunchKernelGGL(k_flags_out, dim3(1), dim3(1), 0, s, flags, host);
+}
+
 // LDS of more than 64 KB per workgroup is taken by dynamic size alone on
 // gfx950; the attribute tells the runtime to expect it.
 hipError_t grid_kernels_init()
 {
     const std::pair<const void *, int> k[] = {
-        {(const void *)k_grid_part, GRID_PTS * 12 + GRID_MAX_BUCKETS * 4},
-        {(const void *)k_grid_bin<256, 1>, BIN_LDS(GRID_MAX_CELLS)},
-        {(const void *)k_grid_bin<512, 1>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_part<false>, GRID_PTS * 12 + GRID_MAX_BUCKETS * 4},
+        {(const void *)k_grid_part<true>, GRID_PTS * 12 + GRID_MAX_BUCKETS * 4},
+        {(const void *)k_grid_bin<256, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_bin<512, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_bin<256, 1, true>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_bin<512, 1, true>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_windows, GRID_MAX_WIN_CELLS * 16}};
     for (const auto &f : k) {
         const hipError_t e =

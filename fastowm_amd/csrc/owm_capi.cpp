@@ -630,7 +630,15 @@ owm_status owm_stage1(owm_ctx *ctx, owm_tree *tree, const owm_params *params, ui
     Prepared P;
     QueryOut qo;
     uint32_t hc[16];
-    owm_status st = tree_query_sync(ctx, tree, params, 1, 1, nullptr, 0, P, qo, hc);
+    bool done = false;
+    uint64_t nwin = 0;
+    owm_status st = tree_grid(ctx, *tree, *params, true, min_ids, cap, &nwin, done);
+    if (done || st != OWM_OK) {
+        if (derived && st == OWM_OK)
+            owm_derive(params, tree->n, tree->P.box[0].data(), derived);
+        return st;
+    }
+    st = tree_query_sync(ctx, tree, params, 1, 1, nullptr, 0, P, qo, hc);
     if (derived && (st == OWM_OK || st == OWM_E_CAPACITY))
         owm_derive(params, tree->n, P.box[0].data(), derived);
     if (st != OWM_OK)
@@ -725,7 +733,11 @@ owm_status owm_tree_run(owm_ctx *ctx, owm_tree *tree, const owm_params *params, 
     QueryOut qo;
     uint64_t off[2] = {0, 0};
     uint64_t need = 0;
-    owm_status st = tree_query(ctx, tree, params, 1, 4, nullptr, 0, P, qo);
+    bool done = false;
+    owm_status st = tree_grid(ctx, *tree, *params, false, seeds, cap, n_seeds, done);
+    if (done || st != OWM_OK)
+        return st;
+    st = tree_query(ctx, tree, params, 1, 4, nullptr, 0, P, qo);
     if (st == OWM_OK)
         st = read_seeds(ctx, qo, (uint32_t)P.td.size(), seeds, cap, off, &need);
     if (st == OWM_OK && need) {

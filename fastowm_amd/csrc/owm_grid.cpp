@@ -340,9 +340,16 @@ owm_status one_box(owm_ctx *ctx, const double *dx, const double *dy, uint64_t n,
     return any ? st : OWM_OK;
 }
 
+// Where a chain's points are, and what it is to give.
+struct GridSrc {
+    const double *x = nullptr, *y = nullptr, *z = nullptr;
+    const TreeOut *tree = nullptr;  // a resident tree's instead
+    bool minima = false;            // the windows' minima (qo.min_ids), not the seeds
+};
+
 // Everything the chain's launches depend on.
-static void plan_key(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
-                     const GridPlan &P, const GridIo &io, std::vector<uint8_t> &key)
+static void plan_key(owm_ctx *ctx, const GridSrc &src, const GridPlan &P, const GridIo &io,
+                     std::vector<uint8_t> &key)
 {
     auto put = [&key](const void *p, size_t n) {
         const uint8_t *b = (const uint8_t *)p;
@@ -350,10 +357,204 @@ static void plan_key(owm_ctx *ctx, const double *dx, const double *dy, const dou
     };
     key.clear();
     put("grid", 4);
-    const void *ptrs[6] = {dx, dy, dz, ctx->arena.buf.ptr, io.head, ctx->h_tab};
+    const void *ptrs[6] = {src.x, src.y, src.z, ctx->arena.buf.ptr, io.head, ctx->h_tab};
     put(ptrs, sizeof ptrs);
     put(P.t.data(), P.t.size() * sizeof(GridTile));
     put(P.pt_off.data(), P.pt_off.size() * 4);
+}
+
+// Runs the planned chain; its results are in io (and qo) when it comes back.  Not
+// taken: it might not fit the budget where the tree chain would, or too many points
+// lie on edges.
+static owm_status exec_plan(owm_ctx *ctx, const GridPlan &P, const GridIo &io, const GridSrc &src,
+                            uint32_t flags, QueryOut &qo, bool &taken)
+{
+    taken = false;
+    const uint32_t T = (uint32_t)P.t.size();
+    const uint64_t np = P.np;
+    const uint64_t nwords = (np + 31) / 32, items = P.item_off[T], gcells = P.gcell_off[T];
+    const uint64_t nseed = std::min<uint64_t>(np, P.nwin + gcells) + 1;
+    const uint64_t table = up256(T * sizeof(GridTile)) + 6 * up256((T + 1) * 4ull);
+    const uint64_t need = table + up256(P.recs * 12 + 64) + up256(P.tab * 2) +
+                          up256(P.cells * 16) + up256(items * 4) + up256(P.axis_off[T] * 8ull) +
+                          up256(P.pool_cap * GRID_POOLS * sizeof(GridRare)) +
+                          up256(P.list_cap * GRID_POOLS * 4) + up256(GRID_POOLS * 128) + 2 * up256((nwords + 4) * 4) +
+                          up256((gcells + 1) * 4) + up256((nwords / 4096 + 2) * 4) +
+                          up256(nseed * 4) + up256((T + 1) * 4ull) +
+                          (src.minima ? up256(P.nwin * 4) : 0) + 4096;
+    // (a tree's query may leave less room than the tree chain would for the
+    // builds that follow: its scratch grows only where one of this size still fits)
+    if (src.tree ? need > ctx->arena.buf.bytes && ctx->exceeds(need + tree_chain_bound(P))
+                 : ctx->exceeds(std::max(need, tree_chain_bound(P)), &ctx->arena.buf))
+        return OWM_OK;
+    void *old_arena = ctx->arena.buf.ptr;
+    owm_status st = ctx->arena.ensure(ctx, need);
+    if (st != OWM_OK)
+        return st;
+    if (ctx->arena.buf.ptr != old_arena)
+        ctx->graphs.clear();
+    taken = true;
+
+    Arena &A = ctx->arena;
+    hipStream_t s = ctx->stream;
+    // table
+    uint8_t *d = A.take(table);
+    (void)hipStreamSynchronize(s);  // the previous reads of this buffer must have completed
+    uint8_t *h = ctx->pinned(ctx->h_tab, ctx->h_tab_cap, table);
+    if (!d || !h) {
+        set_err(ctx, "pinned host allocation failed");
+        return OWM_E_NOMEM;
+    }
+    bool graph = (flags & OWM_B_GRAPH) != 0;
+    std::vector<uint8_t> key;
+    if (graph || (flags & B_AUTO_GRAPH))
+        plan_key(ctx, src, P, io, key);
+    if (!graph && (flags & B_AUTO_GRAPH)) {
+        graph = !ctx->prof.on && key == ctx->graphs.last_key;
+        ctx->graphs.last_key = key;
+    }
+    GridDev G{};
+    if (src.tree) {
+        G.xy = src.tree->pts.xy;
+        G.zi = src.tree->pts.zi;
+        G.pos = src.tree->pos;
+    }
+    G.ntiles = T;
+    G.ngcell = (uint32_t)gcells;
+    G.tiles = (const GridTile *)d;
+    memcpy(h, P.t.data(), T * sizeof(GridTile));
+    const std::vector<uint32_t> *tabs[6] = {&P.st_off,    &P.item_off, &P.blk_off,
+                                           &P.gcell_off, &P.axis_off, &P.pt_off};
+    const uint32_t *off[6];
+    uint64_t o = up256(T * sizeof(GridTile));
+    for (int k = 0; k < 6; ++k, o += up256((T + 1) * 4ull)) {
+        memcpy(h + o, tabs[k]->data(), (T + 1) * 4ull);
+        off[k] = (const uint32_t *)(d + o);
+    }
+    G.st_off = off[0];
+    G.item_off = off[1];
+    G.blk_off = off[2];
+    G.gcell_off = off[3];
+    G.axis_off = off[4];
+    BatchDev B{};
+    B.ntiles = T;
+    B.np = (uint32_t)np;
+    B.pt_off = off[5];
+    // a few tiles' table is fetched by the chain's first launch
+    const bool fetch = T <= 8;
+    if (!fetch)
+        HIP_TRY(hipMemcpyAsync(d, h, table, hipMemcpyHostToDevice, s), "upload table");
+
+    auto body = [&]() -> owm_status {
+        // (a lane's last load may reach 36 bytes past its run)
+        G.rec = (uint32_t *)A.take(P.recs * 12 + 64);
+        G.tab = (uint16_t *)A.take(P.tab * 2);
+        G.cells = (uint4 *)A.take(P.cells * 16);
+        G.heads = (uint32_t *)A.take(items * 4);
+        G.wcols = (int2 *)A.take(P.axis_off[T] * 8ull);
+        G.pool = (GridRare *)A.take(P.pool_cap * GRID_POOLS * sizeof(GridRare));
+        G.pool_cap = (uint32_t)P.pool_cap;
+        G.list = (uint32_t *)A.take(P.list_cap * GRID_POOLS * 4);
+        G.list_cap = (uint32_t)P.list_cap;
+        G.pool_used = (uint32_t *)A.take(GRID_POOLS * 128);
+        G.seen = (uint32_t *)A.take((nwords + 4) * 4);
+        G.llp = (uint32_t *)A.take((nwords + 4) * 4);
+        G.cell_flag = (uint32_t *)A.take((gcells + 1) * 4);
+        uint32_t *lookback = (uint32_t *)A.take((nwords / 4096 + 2) * 4);
+        uint32_t *out = (uint32_t *)A.take(nseed * 4);
+        uint32_t *seed_off = (uint32_t *)A.take((T + 1) * 4ull);
+        if (src.minima)
+            G.min_ids = (uint32_t *)A.take(P.nwin * 4);
+        uint32_t *cnt = (uint32_t *)A.take(1024);
+        if (!cnt) {
+            set_err(ctx, "scratch arena exhausted (grid)");
+            return OWM_E_INTERNAL;
+        }
+        G.err = cnt + 3;
+        FillRanges z;
+        auto zero = [&](uint32_t *p, uint64_t words) {
+            z.ptr[z.count] = p;
+            z.len[z.count++] = words;
+        };
+        zero(cnt, 16);
+        zero(G.pool_used, GRID_POOLS * 32);
+        zero(G.seen, nwords + 4);
+        zero(G.llp, nwords + 4);
+        zero(G.cell_flag, gcells + 1);
+        zero(lookback, nwords / 4096 + 2);
+        launch_grid_prep(s, G, z, P.axis_off[T], fetch ? (const uint32_t *)h : nullptr,
+                         (uint32_t)(table / 4));
+        int pi = ctx->prof.begin(s, PH_GRID_PART);
+        launch_grid_part(s, G, src.x, src.y, src.z, P.st_off[T], P.max_nb);
+        // x, y and z read; a record written
+        ctx->prof.end(s, pi, 36ull * np, np);
+        pi = ctx->prof.begin(s, PH_GRID_BIN);
+        for (const GridPlan::Class &c : P.cls)
+            launch_grid_bin(s, G, c.t0, c.t1, P.item_off[c.t0],
+                            P.item_off[c.t1] - P.item_off[c.t0], c.cells);
+        ctx->prof.end(s, pi, 12ull * np + 16ull * P.cells, np, (uint32_t)P.cls.size());
+        pi = ctx->prof.begin(s, PH_GRID_WIN);
+        launch_grid_windows(s, G, src.x, src.y, P.blk_off[T], P.win_cells);
+        ctx->prof.end(s, pi, 16ull * P.cells + 8ull * P.nwin, P.nwin);
+        if (src.minima) {
+            launch_flags_out(s, cnt + 3, io.head + 1);
+            HIP_TRY(hipGetLastError(), "grid chain launch");
+            qo.min_ids = G.min_ids;
+            return OWM_OK;
+        }
+        if (gcells) {
+            pi = ctx->prof.begin(s, PH_STAGE3);
+            launch_grid_cells(s, G);
+            ctx->prof.end(s, pi, 12ull * gcells, gcells);
+        }
+        pi = ctx->prof.begin(s, PH_MERGE);
+        SeedOut S;
+        S.ntiles = T;
+        S.pt_off = B.pt_off;
+        S.err = cnt + 3;
+        S.host = io.head;
+        S.host_off = io.off;
+        S.host_ids = io.ids;
+        S.host_cap = GridIo::IDS;
+        launch_seeds(s, B, G.llp, (uint32_t)nwords, out, (uint32_t)nseed, seed_off, cnt + 2,
+                     lookback, cnt + 7, S);
+        ctx->prof.end(s, pi, 4ull * nwords, nwords);
+        HIP_TRY(hipGetLastError(), "grid chain launch");
+        qo.cnt = cnt;
+        qo.seeds = out;
+        return OWM_OK;
+    };
+    st = run_chain(ctx, graph, std::move(key), A, qo, body);
+    if (st != OWM_OK)
+        return st;
+    HIP_TRY(hipStreamSynchronize(s), "pipeline");
+    ctx->prof.collect();
+    const uint32_t err = io.head[1];
+    if (err & ~GRID_ERR_POOL) {
+        set_err(ctx, "device capacity guard tripped (flags %u)", err);
+        return OWM_E_INTERNAL;
+    }
+    taken = !(err & GRID_ERR_POOL);
+    return OWM_OK;
+}
+
+// The seeds of a finished chain.
+static owm_status copy_seeds(owm_ctx *ctx, const GridIo &io, const QueryOut &qo, uint32_t n_tiles,
+                             uint32_t *seeds, uint64_t cap, uint64_t *seed_off_host)
+{
+    const uint64_t ns = io.head[0];
+    for (uint32_t t = 0; t <= n_tiles; ++t)
+        seed_off_host[t] = io.off[t];
+    if (ns > cap) {
+        set_err(ctx, "seed buffer holds %llu, %llu needed", (unsigned long long)cap,
+                (unsigned long long)ns);
+        return OWM_E_CAPACITY;
+    }
+    if (ns <= GridIo::IDS)
+        memcpy(seeds, io.ids, ns * 4);
+    else
+        HIP_TRY(hipMemcpy(seeds, qo.seeds, ns * 4, hipMemcpyDeviceToHost), "seeds D2H");
+    return OWM_OK;
 }
 
 owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
@@ -406,170 +607,73 @@ owm_status run_grid(owm_ctx *ctx, const double *dx, const double *dy, const doub
     GridPlan P;
     if (!make_plan(ctx, tiles, n_tiles, box, P))
         return hand_on();
-    const uint32_t T = n_tiles;
-    const uint64_t nwords = (np + 31) / 32, items = P.item_off[T], gcells = P.gcell_off[T];
-    const uint64_t nseed = std::min<uint64_t>(np, P.nwin + gcells) + 1;
-    const uint64_t table = up256(T * sizeof(GridTile)) + 6 * up256((T + 1) * 4ull);
-    const uint64_t need = table + up256(P.recs * 12 + 64) + up256(P.tab * 2) +
-                          up256(P.cells * 16) + up256(items * 4) + up256(P.axis_off[T] * 8ull) +
-                          up256(P.pool_cap * GRID_POOLS * sizeof(GridRare)) +
-                          up256(P.list_cap * GRID_POOLS * 4) + up256(GRID_POOLS * 128) + 2 * up256((nwords + 4) * 4) +
-                          up256((gcells + 1) * 4) + up256((nwords / 4096 + 2) * 4) +
-                          up256(nseed * 4) + up256((T + 1) * 4ull) + 4096;
-    if (ctx->exceeds(std::max(need, tree_chain_bound(P)), &ctx->arena.buf))
-        return hand_on();
-    void *old_arena = ctx->arena.buf.ptr;
-    st = ctx->arena.ensure(ctx, need);
+    GridSrc src;
+    src.x = dx;
+    src.y = dy;
+    src.z = dz;
+    QueryOut qo;
+    st = exec_plan(ctx, P, io, src, flags, qo, handled);
     if (st != OWM_OK)
         return st;
-    if (ctx->arena.buf.ptr != old_arena)
-        ctx->graphs.clear();
-    handled = true;
+    if (!handled)
+        return hand_on();
+    return copy_seeds(ctx, io, qo, n_tiles, seeds, cap, seed_off_host);
+}
 
-    Arena &A = ctx->arena;
-    hipStream_t s = ctx->stream;
-    // table
-    uint8_t *d = A.take(table);
-    (void)hipStreamSynchronize(s);  // the previous reads of this buffer must have completed
-    uint8_t *h = ctx->pinned(ctx->h_tab, ctx->h_tab_cap, table);
-    if (!d || !h) {
+owm_status tree_grid(owm_ctx *ctx, const owm_tree &tree, const owm_params &params, bool minima,
+                     uint32_t *out, uint64_t cap, uint64_t *n_out, bool &handled)
+{
+    handled = false;
+    if (!tree.n || ctx->tuner.forced || getenv("OWM_NO_GRID"))
+        return OWM_OK;
+    owm_tile t{};
+    t.n = tree.n;
+    t.params = params;
+    std::vector<std::array<double, 4>> box(1);
+    if (params.flags & OWM_F_HAVE_BBOX)
+        memcpy(box[0].data(), params.bbox, sizeof(double) * 4);
+    else
+        box[0] = tree.P.box[0];
+    // The chain reads every point, the tree chain the leaves under the windows'
+    // edges: a query of a part of the tree stays there.  So do large trees with
+    // small windows, whose order leaves the partition's runs uneven (minima and
+    // seeds, windows of 600 points, 3M points: 125 us against 183 by the tree
+    // chain, 8M 231 and 325, 16M 434 and 537, 60M 3450 and 1829; windows of 2400
+    // points, 3M points: 172 and 595 us, 16M 418 and 807, 60M 1566 and 1182).
+    const std::array<double, 4> &tb = tree.P.box[0];
+    for (int a = 0; a < 4; a += 2)
+        if (!(box[0][a] <= tb[a] && tb[a + 1] <= box[0][a + 1]))
+            return OWM_OK;
+    const double per_window = (double)tree.n * params.wsize * params.wsize /
+                              ((tb[1] - tb[0]) * (tb[3] - tb[2]));
+    if (tree.n > (8u << 20) && !(tree.n <= (32u << 20) && per_window >= 2000.0))
+        return OWM_OK;
+    GridPlan P;
+    if (!make_plan(ctx, &t, 1, box, P))
+        return OWM_OK;
+    if (minima && P.nwin > cap)
+        return OWM_OK;  // the tree chain reports it
+    const GridIo io(ctx, 1);
+    if (!io.head) {
         set_err(ctx, "pinned host allocation failed");
         return OWM_E_NOMEM;
     }
-    bool graph = (flags & OWM_B_GRAPH) != 0;
-    std::vector<uint8_t> key;
-    if (graph || (flags & B_AUTO_GRAPH))
-        plan_key(ctx, dx, dy, dz, P, io, key);
-    if (!graph && (flags & B_AUTO_GRAPH)) {
-        graph = !ctx->prof.on && key == ctx->graphs.last_key;
-        ctx->graphs.last_key = key;
-    }
-    GridDev G{};
-    G.ntiles = T;
-    G.ngcell = (uint32_t)gcells;
-    G.tiles = (const GridTile *)d;
-    memcpy(h, P.t.data(), T * sizeof(GridTile));
-    const std::vector<uint32_t> *src[6] = {&P.st_off,    &P.item_off, &P.blk_off,
-                                           &P.gcell_off, &P.axis_off, &P.pt_off};
-    const uint32_t *off[6];
-    uint64_t o = up256(T * sizeof(GridTile));
-    for (int k = 0; k < 6; ++k, o += up256((T + 1) * 4ull)) {
-        memcpy(h + o, src[k]->data(), (T + 1) * 4ull);
-        off[k] = (const uint32_t *)(d + o);
-    }
-    G.st_off = off[0];
-    G.item_off = off[1];
-    G.blk_off = off[2];
-    G.gcell_off = off[3];
-    G.axis_off = off[4];
-    BatchDev B{};
-    B.ntiles = T;
-    B.np = (uint32_t)np;
-    B.pt_off = off[5];
-    // a few tiles' table is fetched by the chain's first launch
-    const bool fetch = T <= 8;
-    if (!fetch)
-        HIP_TRY(hipMemcpyAsync(d, h, table, hipMemcpyHostToDevice, s), "upload table");
-
+    GridSrc src;
+    src.tree = &tree.T;
+    src.minima = minima;
     QueryOut qo;
-    auto body = [&]() -> owm_status {
-        // (a lane's last load may reach 36 bytes past its run)
-        G.rec = (uint32_t *)A.take(P.recs * 12 + 64);
-        G.tab = (uint16_t *)A.take(P.tab * 2);
-        G.cells = (uint4 *)A.take(P.cells * 16);
-        G.heads = (uint32_t *)A.take(items * 4);
-        G.wcols = (int2 *)A.take(P.axis_off[T] * 8ull);
-        G.pool = (GridRare *)A.take(P.pool_cap * GRID_POOLS * sizeof(GridRare));
-        G.pool_cap = (uint32_t)P.pool_cap;
-        G.list = (uint32_t *)A.take(P.list_cap * GRID_POOLS * 4);
-        G.list_cap = (uint32_t)P.list_cap;
-        G.pool_used = (uint32_t *)A.take(GRID_POOLS * 128);
-        G.seen = (uint32_t *)A.take((nwords + 4) * 4);
-        G.llp = (uint32_t *)A.take((nwords + 4) * 4);
-        G.cell_flag = (uint32_t *)A.take((gcells + 1) * 4);
-        uint32_t *lookback = (uint32_t *)A.take((nwords / 4096 + 2) * 4);
-        uint32_t *out = (uint32_t *)A.take(nseed * 4);
-        uint32_t *seed_off = (uint32_t *)A.take((T + 1) * 4ull);
-        uint32_t *cnt = (uint32_t *)A.take(1024);
-        if (!cnt) {
-            set_err(ctx, "scratch arena exhausted (grid)");
-            return OWM_E_INTERNAL;
-        }
-        G.err = cnt + 3;
-        FillRanges z;
-        auto zero = [&](uint32_t *p, uint64_t words) {
-            z.ptr[z.count] = p;
-            z.len[z.count++] = words;
-        };
-        zero(cnt, 16);
-        zero(G.pool_used, GRID_POOLS * 32);
-        zero(G.seen, nwords + 4);
-        zero(G.llp, nwords + 4);
-        zero(G.cell_flag, gcells + 1);
-        zero(lookback, nwords / 4096 + 2);
-        launch_grid_prep(s, G, z, P.axis_off[T], fetch ? (const uint32_t *)h : nullptr,
-                         (uint32_t)(table / 4));
-        int pi = ctx->prof.begin(s, PH_GRID_PART);
-        launch_grid_part(s, G, dx, dy, dz, P.st_off[T], P.max_nb);
-        // x, y and z read; a record written
-        ctx->prof.end(s, pi, 36ull * np, np);
-        pi = ctx->prof.begin(s, PH_GRID_BIN);
-        for (const GridPlan::Class &c : P.cls)
-            launch_grid_bin(s, G, c.t0, c.t1, P.item_off[c.t0],
-                            P.item_off[c.t1] - P.item_off[c.t0], c.cells);
-        ctx->prof.end(s, pi, 12ull * np + 16ull * P.cells, np, (uint32_t)P.cls.size());
-        pi = ctx->prof.begin(s, PH_GRID_WIN);
-        launch_grid_windows(s, G, dx, dy, P.blk_off[T], P.win_cells);
-        ctx->prof.end(s, pi, 16ull * P.cells + 8ull * P.nwin, P.nwin);
-        if (gcells) {
-            pi = ctx->prof.begin(s, PH_STAGE3);
-            launch_grid_cells(s, G);
-            ctx->prof.end(s, pi, 12ull * gcells, gcells);
-        }
-        pi = ctx->prof.begin(s, PH_MERGE);
-        SeedOut S;
-        S.ntiles = T;
-        S.pt_off = B.pt_off;
-        S.err = cnt + 3;
-        S.host = io.head;
-        S.host_off = io.off;
-        S.host_ids = io.ids;
-        S.host_cap = GridIo::IDS;
-        launch_seeds(s, B, G.llp, (uint32_t)nwords, out, (uint32_t)nseed, seed_off, cnt + 2,
-                     lookback, cnt + 7, S);
-        ctx->prof.end(s, pi, 4ull * nwords, nwords);
-        HIP_TRY(hipGetLastError(), "grid chain launch");
-        qo.cnt = cnt;
-        qo.seeds = out;
-        return OWM_OK;
-    };
-    st = run_chain(ctx, graph, std::move(key), A, qo, body);
-    if (st != OWM_OK)
+    owm_status st = exec_plan(ctx, P, io, src, 0, qo, handled);
+    if (st != OWM_OK || !handled)
         return st;
-    HIP_TRY(hipStreamSynchronize(s), "pipeline");
-    ctx->prof.collect();
-    const uint32_t err = io.head[1];
-    if (err & ~GRID_ERR_POOL) {
-        set_err(ctx, "device capacity guard tripped (flags %u)", err);
-        return OWM_E_INTERNAL;
+    if (minima) {
+        *n_out = P.nwin;
+        HIP_TRY(hipMemcpy(out, qo.min_ids, P.nwin * 4, hipMemcpyDeviceToHost), "min_ids D2H");
+        return OWM_OK;
     }
-    if (err & GRID_ERR_POOL) {
-        handled = false;
-        return hand_on();
-    }
-    const uint64_t ns = io.head[0];
-    for (uint32_t t = 0; t <= n_tiles; ++t)
-        seed_off_host[t] = io.off[t];
-    if (ns > cap) {
-        set_err(ctx, "seed buffer holds %llu, %llu needed", (unsigned long long)cap,
-                (unsigned long long)ns);
-        return OWM_E_CAPACITY;
-    }
-    if (ns <= GridIo::IDS)
-        memcpy(seeds, io.ids, ns * 4);
-    else
-        HIP_TRY(hipMemcpy(seeds, qo.seeds, ns * 4, hipMemcpyDeviceToHost), "seeds D2H");
-    return OWM_OK;
+    uint64_t off[2] = {0, 0};
+    st = copy_seeds(ctx, io, qo, 1, out, cap, off);
+    *n_out = off[1];
+    return st;
 }
 
 }  // namespace owm

@@ -16,6 +16,7 @@
 #include "owm_kernels.h"
 
 struct owm_ctx;
+struct owm_tree;
 
 namespace owm {
 
@@ -254,6 +255,10 @@ constexpr uint32_t B_AUTO_GRAPH = 1u << 31;
 owm_status run_batch(owm_ctx *ctx, const double *dx, const double *dy, const double *dz,
                      const owm_tile *tiles, uint32_t n_tiles, uint32_t flags, uint32_t *seeds,
                      uint64_t cap, uint64_t *seed_off_host);
+// A query of a resident tree by the same chain on the tree's points: the
+// windows' minima, or the seeds.  handled as for run_grid.
+owm_status tree_grid(owm_ctx *ctx, const owm_tree &tree, const owm_params &params, bool minima,
+                     uint32_t *out, uint64_t cap, uint64_t *n_out, bool &handled);
 // Exact box (min x, max x, min y, max y) of a cloud of fewer than 2^32 points in
 // device memory; any: it has finite points.
 owm_status one_box(owm_ctx *ctx, const double *dx, const double *dy, uint64_t n, double *box,

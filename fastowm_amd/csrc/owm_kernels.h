@@ -170,6 +170,12 @@ struct GridTile {
 };
 
 struct GridDev {
+    // the points of a resident tree (else the caller's arrays, passed beside): in
+    // its order, with their indices; sorted position of an index
+    const double2 *xy;
+    const PointZ *zi;
+    const uint32_t *pos;
+    uint32_t *min_ids;  // not null: the windows' minima alone (one tile, row-major)
     uint32_t ntiles, ngcell;
     const GridTile *tiles;
     const uint32_t *st_off, *item_off, *blk_off, *gcell_off;  // [ntiles + 1] each
@@ -209,6 +215,8 @@ constexpr uint32_t GRID_MAX_WIN_CELLS = 9216;
 void launch_grid_windows(hipStream_t s, const GridDev &G, const double *x, const double *y,
                          uint32_t blocks, uint32_t cells_cap);
 void launch_grid_cells(hipStream_t s, const GridDev &G);
+// *flags to host memory.
+void launch_flags_out(hipStream_t s, const uint32_t *flags, uint32_t *host);
 
 // ---- .xyz reader (xyz.hip) ----
 // The text buffer is zero-padded to a whole number of xyz_chunk_bytes() plus

@@ -177,3 +177,51 @@ def test_dense_seeds_over_many_tiles(ctx):
             clouds.append(c)
         wants = _batch(ctx, clouds, [(3, 4, 0.0)] * len(sizes))
         assert sum(len(w) for w in wants) > 0.3 * sum(sizes)
+
+
+@pytest.mark.parametrize("n,leaf", [(3, 1), (64, 32), (4097, 8), (50_001, 32), (300_000, 16)])
+@pytest.mark.parametrize("cm", [False, True])
+def test_resident_tree(ctx, n, leaf, cm):
+    """Minima and seeds of a resident tree (its points permuted) by the chain:
+    several parameters, a box of the query's own, ties, points on edges."""
+    say("grid chain, resident tree", n, leaf, cm)
+    t = synth.scaled(synth.config_c1(seed=n), max(n, 400))
+    x, y, z = (a[:n].copy() for a in t.generate())
+    if n < 4:
+        x, y = np.array([0.0, 40.5, 11.0]), np.array([1.0, 30.5, 12.0])
+    z = np.round(z, 1)
+    if cm:
+        x, y = np.round(x, 2), np.round(y, 2)
+    box = synth.bbox(x, y)
+    tree = ctx.parallel_qtree(x, y, z, leaf_size=leaf)
+    for ws, bs, ov, b in [(10, 20, 0.8, None), (7, 13, 0.5, None), (8, 0, 0.0, None), (3, 1, 0.0, None),
+                          (12, 20, 0.75, (box[0] - 7.0, box[1] + 3.0, box[2] - 2.0, box[3] + 9.0)),
+                          (9, 12, 0.7, (box[0] + 5.0, box[1] + 3.0, box[2] - 2.0, box[3] - 9.0))]:
+        inside = b is None or (b[0] <= box[0] and box[1] <= b[1] and b[2] <= box[2] and box[3] <= b[3])
+        p = O.params(ws, bs, ov, b or box, n, leaf)
+        ctx.profile(True)
+        gm, d = ctx.stage1(tree, ws, ov, bs, bbox=b)
+        seeds = ctx.tree_run(tree, ws, bs, ov, bbox=b)
+        calls = ctx.profile_read()
+        ctx.profile(False)
+        assert calls["grid_partition"]["calls"] == (2 if inside else 0)
+        assert (d.ncols, d.nrows) == (p.ncols, p.nrows)
+        assert np.array_equal(gm, O.Tree(x, y, z, p).stage1())
+        assert np.array_equal(seeds, O.run(x, y, z, ws, bs, ov, leaf, b or box)[0])
+    tree.free()
+
+
+def test_resident_tree_falls_back(ctx):
+    """More points on edges than the pool holds: the tree chain answers."""
+    say("grid chain, resident tree falls back")
+    rng = np.random.default_rng(10)
+    n = 400_000
+    x, y = (rng.integers(0, 801, n).astype(np.float64) for _ in range(2))
+    z = np.round(rng.normal(50.0, 3.0, n), 1)
+    box = synth.bbox(x, y)
+    p = O.params(8, 20, 0.5, box, n, 32)
+    tree = ctx.parallel_qtree(x, y, z)
+    gm, _ = ctx.stage1(tree, 8, 0.5, 20)
+    assert np.array_equal(gm, O.Tree(x, y, z, p).stage1())
+    assert np.array_equal(ctx.tree_run(tree, 8, 20, 0.5), O.run(x, y, z, 8, 20, 0.5, 32)[0])
+    tree.free()
