@@ -225,3 +225,23 @@ def test_resident_tree_falls_back(ctx):
     assert np.array_equal(gm, O.Tree(x, y, z, p).stage1())
     assert np.array_equal(ctx.tree_run(tree, 8, 20, 0.5), O.run(x, y, z, 8, 20, 0.5, 32)[0])
     tree.free()
+
+
+@pytest.mark.parametrize("frac", [0.02, 0.3, 0.97])
+def test_box_of_a_part(ctx, frac):
+    """A box given that holds a part of the points: most lie before the first
+    edges or behind the last ones; some not a number."""
+    say("grid chain, box of a part", frac)
+    t = synth.scaled(synth.config_c1(seed=3), 60_000)
+    x, y, z = t.generate()
+    x[::997], y[5::997] = np.nan, np.inf
+    x0, x1, y0, y1 = synth.bbox(x[np.isfinite(x)], y[np.isfinite(y)])
+    box = (x0 + 0.1 * frac * (x1 - x0), x0 + frac * (x1 - x0), y0, y0 + max(frac, 0.2) * (y1 - y0))
+    for ws, bs, ov in ((10, 20, 0.8), (7, 13, 0.5), (8, 0, 0.0)):
+        want, _, _ = O.run(x, y, z, ws, bs, ov, 32, box)
+        ctx.profile(True)
+        got = ctx.run_tile(x, y, z, ws, bs, ov, bbox=box)
+        calls = ctx.profile_read()
+        ctx.profile(False)
+        assert calls["grid_partition"]["calls"] == 1
+        assert np.array_equal(got, want)
