@@ -24,6 +24,7 @@
 // column; k_grid_part puts their exact window and cell ranges into a pool,
 // k_grid_bin lists each bucket's, and the last two kernels add them.
 #include "owm_kernels.h"
+#include <algorithm>
 #include <utility>
 
 namespace owm {
@@ -317,8 +318,9 @@ struct __attribute__((packed, aligned(4))) RecWord {
 constexpr uint32_t GB_RARE = 512;   // points without a column listed before a flush
 
 // Appends the listed pool entries to the item's chain of blocks {count, next
-// block, entries}.  Every thread of the workgroup calls it.
-template <int NT>
+// block, entries}, whose head is kept in `head` (SUB: in memory, other workgroups
+// append too).  Every thread of the workgroup calls it.
+template <int NT, bool SUB>
 __device__ __forceinline__ void flush_rare(const GridDev &G, uint32_t item, const uint32_t *list,
                                            uint32_t n, uint32_t *s_base, uint32_t &head)
 {
@@ -334,12 +336,42 @@ __device__ __forceinline__ void flush_rare(const GridDev &G, uint32_t item, cons
     if (base != OWM_NONE) {
         if (threadIdx.x == 0) {
             G.list[base] = n;
-            G.list[base + 1] = head;
+            G.list[base + 1] = SUB ? atomicExch(G.heads + item, base) : head;
         }
         for (uint32_t e = threadIdx.x; e < n; e += NT)
             G.list[base + 2 + e] = list[e];
         head = base;
     }
+    __syncthreads();
+}
+
+// Queues an item's points in the sort tiles [s0, s0 + len), pts at most.  own: its
+// owner, last group, number of stretches and tile.  Every thread of the workgroup calls it.
+template <int NT>
+__device__ __forceinline__ void queue_rest(const GridDev &G, const GridTile &T, uint32_t item,
+                                           uint32_t s0, uint32_t len, uint32_t pts, uint32_t *own,
+                                           uint32_t *s_base)
+{
+    const GridHeavy H(G, T.heavy_cap);
+    const uint32_t ns = min((pts + T.heavy_sub - 1) / T.heavy_sub, len);
+    if (threadIdx.x == 0) {
+        const uint32_t at = atomicAdd(H.n, ns);
+        const bool room = at + ns <= T.heavy_cap;
+        *s_base = room ? at : OWM_NONE;
+        if (room) {
+            own[0] = min(own[0], at);
+            H.grp[at] = make_uint2(ns, own[1]);
+            own[1] = at;
+            own[2] += ns;
+        } else {
+            atomicOr(G.err, GRID_ERR_POOL);
+        }
+    }
+    __syncthreads();
+    const uint32_t at = *s_base, owner = own[0];
+    if (at != OWM_NONE)
+        for (uint32_t i = threadIdx.x; i < ns; i += NT)
+            H.q[at + i] = make_uint4(item, s0 + len * i / ns, s0 + len * (i + 1) / ns, owner);
     __syncthreads();
 }
 
@@ -356,35 +388,38 @@ __device__ __forceinline__ void flush_rare(const GridDev &G, uint32_t item, cons
 // 0.83 ms against separate key and cell streams, two lanes a segment instead of
 // four to eight 0.74, lane masks instead of bit sets 0.71 ms.  One spare cell for
 // all idle lanes instead of one per lane: 3.1 instead of 1.3 ms (329M points).
-template <int NT, int TWO, bool TREE>
-__global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_t t1,
-                                                 uint32_t item0, uint32_t items, uint32_t cells)
+//
+// A share of more than T.heavy points (clouds with most points in a few square
+// metres) would keep one workgroup busy long after the others: further stretches
+// of its sort tiles are queued and binned by the launch below (SUB), each into
+// cells of its own, which the last of an item's adds up.  95 % of 20M points in
+// 5 m x 5 m: 64 -> 0.48 ms; density falling with the distance from a scanner:
+// 0.66 -> 0.29 ms; clouds without such shares pay the empty launch and the test
+// (20M points 100 -> 105 us, 120M 0.61 -> 0.64 ms).
+template <int NT, int TWO, bool TREE, bool SUB>
+__device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t item,
+                                          uint32_t cells, uint32_t st0, uint32_t st1, uint4 *out)
 {
     constexpr int KK = GB_SEG * TWO;
     extern __shared__ unsigned long long s_bin[];
     unsigned long long *sZ = s_bin;                 // [cells + 64]
     uint32_t *sId = (uint32_t *)(sZ + cells + 64);  // [cells + 64]
     uint32_t *sCnt = sId + cells + 64;              // [cells + 64]
-    __shared__ uint32_t s_t, s_base, s_nr, s_w[NT / 64];
+    __shared__ uint32_t s_base, s_nr, s_w[NT / 64], s_own[4];
     __shared__ uint2 sRun[GB_RUNS];
     __shared__ uint32_t sRare[GB_RARE];
     const uint32_t tid = threadIdx.x;
-    // consecutive items (neighbouring buckets, whose runs share cache lines)
-    // on one XCD: workgroups go round the eight XCDs
-    const uint32_t per = (items + 7u) / 8u;
-    const uint32_t rel = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
-    if (rel >= items)
-        return;
-    const uint32_t item = item0 + rel;
-    if (tid == 0)
+    if (tid == 0) {
         s_nr = 0;
-    const uint32_t t = find_entry(G.item_off, t0, t1, item, &s_t);
+        s_own[0] = s_own[1] = OWM_NONE;
+        s_own[2] = 0;
+        s_own[3] = t;
+    }
     const GridTile &T = G.tiles[t];
     const uint32_t lc = T.lw + T.lh, nc = 1u << lc, pt_off = T.pt_off, rec_off = T.rec_off;
-    const uint32_t q = item - T.item_off, bucket = q / T.split, part = q - bucket * T.split;
-    const uint32_t st0 = (uint32_t)((uint64_t)T.nst * part / T.split);
-    const uint32_t st1 = (uint32_t)((uint64_t)T.nst * (part + 1) / T.split);
+    const uint32_t bucket = (item - T.item_off) / T.split;
     const uint32_t nb1 = T.nb + 1, lpr = T.lpr, seg_pts = (uint32_t)GB_SEG << lpr;
+    uint32_t left = T.heavy;  // points until the item is heavy
     for (uint32_t c = tid; c < nc + 64; c += NT) {
         sZ[c] = OWM_ZKEY_NONE;
         sId[c] = OWM_NONE;
@@ -406,6 +441,15 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
         const uint32_t nseg = (o1 - o0 + seg_pts - 1) / seg_pts;
         uint32_t total;
         const uint32_t at0 = block_scan<NT>(nseg, s_w, total);
+        if (!SUB) {
+            const uint32_t pts = __builtin_amdgcn_readfirstlane(total) * seg_pts;
+            if (__builtin_expect(pts > left, 0)) {
+                queue_rest<NT>(G, T, item, s0, min((uint32_t)NT, st1 - s0), pts, s_own, &s_base);
+                total = 0;
+            } else {
+                left -= pts;
+            }
+        }
         for (uint32_t p0 = 0; p0 < total; p0 += GB_RUNS) {
             for (uint32_t e = max(at0, p0); e < min(at0 + nseg, p0 + GB_RUNS); ++e) {
                 const uint32_t a = o0 + (e - at0) * seg_pts;
@@ -469,7 +513,7 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
                 // (no thread appends between the two barriers: the test is uniform)
                 if (s_nr > GB_RARE) {
                     do {
-                        flush_rare<NT>(G, item, sRare, GB_RARE, &s_base, head);
+                        flush_rare<NT, SUB>(G, item, sRare, GB_RARE, &s_base, head);
                         if (tid == 0)
                             s_nr = 0;
                         __syncthreads();
@@ -511,21 +555,38 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
     __syncthreads();
     const uint32_t n_r = min(s_nr, GB_RARE);
     if (n_r)
-        flush_rare<NT>(G, item, sRare, n_r, &s_base, head);
-    if (tid == 0)
+        flush_rare<NT, SUB>(G, item, sRare, n_r, &s_base, head);
+    if (!SUB && tid == 0) {
         G.heads[item] = head;
-    uint4 *out = G.cells + T.cell_off + ((uint64_t)q << lc);
+        if (s_own[0] != OWM_NONE)
+            ((uint4 *)GridHeavy(G, T.heavy_cap).own)[s_own[0]] = make_uint4(s_own[1], s_own[2], 0u, s_own[3]);
+    }
+    if (!SUB)
+        out = G.cells + T.cell_off + ((uint64_t)(item - T.item_off) << lc);
     for (uint32_t c = tid; c < nc; c += NT) {
         const unsigned long long zk = sZ[c];
         out[c] = make_uint4((uint32_t)zk, (uint32_t)(zk >> 32), sId[c], sCnt[c]);
     }
 }
 
-// -------------------------------------------------------------- windows --
-
-constexpr int GW_NT = 512;
-constexpr uint32_t GW_SEGS = 512;  // pool blocks a window block can meet
-constexpr int GW_PER = 32 * 32 / GW_NT;  // windows per thread, at most
+template <int NT, int TWO, bool TREE>
+__global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_t t1,
+                                                 uint32_t item0, uint32_t items, uint32_t cells)
+{
+    __shared__ uint32_t s_t;
+    // consecutive items (neighbouring buckets, whose runs share cache lines)
+    // on one XCD: workgroups go round the eight XCDs
+    const uint32_t per = (items + 7u) / 8u;
+    const uint32_t rel = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+    if (rel >= items)
+        return;
+    const uint32_t item = item0 + rel;
+    const uint32_t t = find_entry(G.item_off, t0, t1, item, &s_t);
+    const GridTile &T = G.tiles[t];
+    const uint32_t q = item - T.item_off, part = q % T.split;
+    bin_range<NT, TWO, TREE, false>(G, t, item, cells, (uint32_t)((uint64_t)T.nst * part / T.split),
+                                    (uint32_t)((uint64_t)T.nst * (part + 1) / T.split), nullptr);
+}
 
 struct CellAgg {
     unsigned long long zk;
@@ -540,6 +601,65 @@ __device__ __forceinline__ void agg_add(CellAgg &a, unsigned long long zk, uint3
         a.id = id;
     }
 }
+
+// The queued stretches (none for most clouds: 4 us).
+template <int NT, bool TREE>
+__global__ __launch_bounds__(NT) void k_grid_heavy(GridDev G, uint32_t cap,
+                                                   uint32_t cells)
+{
+    __shared__ uint32_t s_last;
+    const uint32_t tid = threadIdx.x;
+    // (an overfull queue has entries that were never written)
+    if (*G.err & GRID_ERR_POOL)
+        return;
+    const GridHeavy H(G, cap);
+    const uint32_t n = min(*H.n, cap);
+    for (uint32_t e = blockIdx.x; e < n; e += gridDim.x) {
+        const uint4 v = H.q[e];
+        uint32_t *own = H.own + 4 * v.w;
+        const uint32_t t = own[3];
+        bin_range<NT, 1, TREE, true>(G, t, v.x, cells, v.y, v.z,
+                                     H.cells + (uint64_t)e * cells);
+        // the last of the item's adds them up: every wave's stores have reached
+        // the L2, the fence makes them visible beyond this XCD
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0) {
+            __threadfence();
+            s_last = atomicAdd(own + 2, 1u) + 1u == own[1];
+        }
+        __syncthreads();
+        const bool last = s_last;
+        if (last) {
+            __threadfence();
+            const GridTile &T = G.tiles[t];
+            const uint32_t lc = T.lw + T.lh;
+            uint4 *out = G.cells + T.cell_off + ((uint64_t)(v.x - T.item_off) << lc);
+            for (uint32_t c = tid; c < 1u << lc; c += NT) {
+                const uint4 o = out[c];
+                CellAgg a = {(unsigned long long)o.y << 32 | o.x, o.z, o.w};
+                for (uint32_t g = own[0]; g != OWM_NONE;) {
+                    const uint2 grp = H.grp[g];
+                    const uint4 *p = H.cells + (uint64_t)g * cells + c;
+#pragma unroll 4
+                    for (uint32_t k = 0; k < grp.x; ++k) {
+                        const uint4 w = p[(uint64_t)k * cells];
+                        agg_add(a, (unsigned long long)w.y << 32 | w.x, w.z, w.w);
+                    }
+                    g = grp.y;
+                }
+                out[c] = make_uint4((uint32_t)a.zk, (uint32_t)(a.zk >> 32), a.id, a.cnt);
+            }
+        }
+        __syncthreads();  // s_last and the cells in LDS are rewritten
+    }
+}
+
+// -------------------------------------------------------------- windows --
+
+constexpr int GW_NT = 512;
+constexpr uint32_t GW_SEGS = 512;  // pool blocks a window block can meet
+constexpr int GW_PER = 32 * 32 / GW_NT;  // windows per thread, at most
 
 // The cell of column c and row r in its bucket's first share (the others follow
 // at the bucket's size).
@@ -928,6 +1048,13 @@ void launch_grid_bin(hipStream_t s, const GridDev &G, uint32_t t0, uint32_t t1, 
                            item0, items, cells);
 }
 
+void launch_grid_heavy(hipStream_t s, const GridDev &G, uint32_t cap, uint32_t cells)
+{
+    const auto k = G.zi ? k_grid_heavy<512, true> : k_grid_heavy<512, false>;
+    hipLaunchKernelGGL(k, dim3(std::min(cap, 256u)), dim3(512), BIN_LDS(cells), s, G, cap,
+                       cells);
+}
+
 void launch_grid_windows(hipStream_t s, const GridDev &G, const double *x, const double *y,
                          uint32_t blocks, uint32_t cells_cap)
 {
@@ -964,6 +1091,8 @@ hipError_t grid_kernels_init()
         {(const void *)k_grid_bin<512, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_bin<256, 1, true>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_bin<512, 1, true>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_heavy<512, false>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_heavy<512, true>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_windows, GRID_MAX_WIN_CELLS * 16}};
     for (const auto &f : k) {
         const hipError_t e =

@@ -25,7 +25,7 @@ struct GridPlan {
     };
     std::vector<Class> cls;
     uint64_t np = 0, recs = 0, cells = 0, tab = 0, nwin = 0, nleaf = 0, pool_cap = 0, list_cap = 0;
-    uint32_t max_nb = 1, win_cells = 1024;
+    uint32_t max_nb = 1, win_cells = 1024, heavy_cap = 0, heavy_cells = 0;
 };
 
 // Bucket cells up to which tiles share a launch of the bins: the LDS of the
@@ -87,6 +87,10 @@ static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64
     // two; 96 mixed tiles: 0.67 ms with one, 0.69 with two, 0.72 with four).
     const double run = T.nst ? (double)n / ((double)T.nst * T.nb) : 1.0;
     T.lpr = run <= 6.0 ? 0 : run <= 64.0 ? 1 : run <= 128.0 ? 2 : 3;
+    // An item is heavy at three times the mean (counted in whole segments), and not
+    // below 65536 points: some 70 us of a workgroup's time.
+    const double mean_item = ((double)mean + (double)T.nst * (2 << T.lpr)) / T.split;
+    T.heavy = (uint32_t)std::max(65536.0, 3.0 * mean_item);
     return true;
 }
 
@@ -188,6 +192,19 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
         P.gcell_off[t + 1] = (uint32_t)gc;
         P.axis_off[t + 1] = P.axis_off[t] + T.ax[0].w.n + T.ax[1].w.n;
         P.max_nb = std::max(P.max_nb, T.nb);
+    }
+    // heavy stretches: 256 of the whole launch's points, their share of the ends
+    // of groups and of segments that are not full
+    for (const GridTile &T : P.t) {
+        P.heavy_cells = std::max(P.heavy_cells, 1u << (T.lw + T.lh));
+        if (T.n > T.heavy)
+            P.heavy_cap = (uint32_t)std::min<uint64_t>(64 + P.np / 8192, 2048);
+    }
+    for (GridTile &T : P.t) {
+        if (!P.heavy_cap)  // (by the estimate a small tile's item may seem heavy)
+            T.heavy = ~0u;
+        T.heavy_sub = (uint32_t)std::max<uint64_t>(16384, P.np / 256);
+        T.heavy_cap = P.heavy_cap;
     }
     // a quarter of the points may lie on edges before the tree chain takes over
     P.pool_cap = (P.np / 4 + 65536) / GRID_POOLS;
@@ -381,6 +398,7 @@ static owm_status exec_plan(owm_ctx *ctx, const GridPlan &P, const GridIo &io, c
                           up256(P.list_cap * GRID_POOLS * 4) + up256(GRID_POOLS * 128) + 2 * up256((nwords + 4) * 4) +
                           up256((gcells + 1) * 4) + up256((nwords / 4096 + 2) * 4) +
                           up256(nseed * 4) + up256((T + 1) * 4ull) +
+                          up256(GridHeavy::bytes(P.heavy_cap, P.heavy_cells)) +
                           (src.minima ? up256(P.nwin * 4) : 0) + 4096;
     // (a tree's query may leave less room than the tree chain would for the
     // builds that follow: its scratch grows only where one of this size still fits)
@@ -460,6 +478,7 @@ static owm_status exec_plan(owm_ctx *ctx, const GridPlan &P, const GridIo &io, c
         G.seen = (uint32_t *)A.take((nwords + 4) * 4);
         G.llp = (uint32_t *)A.take((nwords + 4) * 4);
         G.cell_flag = (uint32_t *)A.take((gcells + 1) * 4);
+        G.heavy = (uint4 *)A.take(GridHeavy::bytes(P.heavy_cap, P.heavy_cells));
         uint32_t *lookback = (uint32_t *)A.take((nwords / 4096 + 2) * 4);
         uint32_t *out = (uint32_t *)A.take(nseed * 4);
         uint32_t *seed_off = (uint32_t *)A.take((T + 1) * 4ull);
@@ -492,6 +511,8 @@ static owm_status exec_plan(owm_ctx *ctx, const GridPlan &P, const GridIo &io, c
         for (const GridPlan::Class &c : P.cls)
             launch_grid_bin(s, G, c.t0, c.t1, P.item_off[c.t0],
                             P.item_off[c.t1] - P.item_off[c.t0], c.cells);
+        if (P.heavy_cap)
+            launch_grid_heavy(s, G, P.heavy_cap, P.heavy_cells);
         ctx->prof.end(s, pi, 12ull * np + 16ull * P.cells, np, (uint32_t)P.cls.size());
         pi = ctx->prof.begin(s, PH_GRID_WIN);
         launch_grid_windows(s, G, src.x, src.y, P.blk_off[T], P.win_cells);

@@ -139,7 +139,8 @@ constexpr uint32_t GRID_CELL_BITS = 13, GRID_MAX_CELLS = 1u << GRID_CELL_BITS;
 constexpr uint32_t GRID_CELL_MASK = GRID_MAX_CELLS - 1u;
 constexpr uint32_t GRID_MAX_BUCKETS = 8192;
 constexpr uint32_t GRID_POOLS = 64;  // shares of the pool, each with a cursor of its own
-// bits of *err: the pool of points without a column is full; a window block
+// bits of *err: the pool of points without a column (or its lists, or the queue of
+// heavy stretches) is full; a window block
 // has more rows than planned (cannot happen)
 constexpr uint32_t GRID_ERR_POOL = 32u, GRID_ERR_ROWS = 64u;
 
@@ -163,6 +164,9 @@ struct GridTile {
     uint32_t lw, lh;             // a bucket is 2^lw columns x 2^lh rows
     uint32_t nbx, nby, nb;       // buckets
     uint32_t split, item_off;    // items: each bucket's sort tiles in `split` shares
+    // points of an item beyond which its rest is queued, and of a queued stretch;
+    // the queue's capacity (the same for all tiles of a launch)
+    uint32_t heavy, heavy_sub, heavy_cap;
     uint32_t lpr;                // lanes per run segment (log2) of the bins
     uint32_t lbw, nblkx, blk_off;  // window blocks of 2^lbw x 2^lbw
     uint32_t gcell_off;          // first stage-3 cell
@@ -193,7 +197,28 @@ struct GridDev {
     uint32_t pool_cap, list_cap;  // entries (words) per share
     uint32_t *seen, *llp;    // point bitmaps: one window, two (LLPs, then seeds)
     uint32_t *cell_flag;     // [ngcell] stage-3 cells that hold an LLP
+    uint4 *heavy;            // GridHeavy
     uint32_t *err;
+};
+
+// Queued stretches of heavy items, all in one piece of memory that few registers
+// address: {item, sort tiles [first, end), owner}; at an item's first stretch, its
+// owner, {last group, stretches, those done, tile}; at a group's first, {stretches,
+// the item's previous group}; cells, `stride` per stretch.  Their number is kept
+// behind *err.
+struct GridHeavy {
+    uint4 *q, *cells;
+    uint32_t *own, *n;
+    uint2 *grp;
+    __host__ __device__ GridHeavy(const GridDev &G, uint32_t cap)
+        : q(G.heavy), cells(G.heavy + 2ull * cap + (cap + 1u) / 2u),
+          own((uint32_t *)(G.heavy + cap)), n(G.err + 5), grp((uint2 *)(G.heavy + 2ull * cap))
+    {
+    }
+    static uint64_t bytes(uint64_t cap, uint64_t stride)
+    {
+        return (2 * cap + (cap + 1) / 2 + cap * stride) * 16;
+    }
 };
 
 // Raises the kernels' LDS limits; once per device.
@@ -209,6 +234,8 @@ void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const do
 // largest bucket's.
 void launch_grid_bin(hipStream_t s, const GridDev &G, uint32_t t0, uint32_t t1, uint32_t item0,
                      uint32_t items, uint32_t cells);
+// The items' queued stretches; cells: the largest bucket's, and the stride.
+void launch_grid_heavy(hipStream_t s, const GridDev &G, uint32_t cap, uint32_t cells);
 // cells_cap: cells under a window block (at least the windows of a block), at
 // most GRID_MAX_WIN_CELLS
 constexpr uint32_t GRID_MAX_WIN_CELLS = 9216;

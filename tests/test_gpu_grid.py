@@ -245,3 +245,37 @@ def test_box_of_a_part(ctx, frac):
         ctx.profile(False)
         assert calls["grid_partition"]["calls"] == 1
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n,blobs", [(70_000, 1), (300_000, 1), (1_500_000, 1), (1_500_000, 3)])
+@pytest.mark.parametrize("order", ["random", "sorted"])
+def test_heavy_buckets(ctx, n, blobs, order):
+    """Most points in a few square metres: stretches of one bucket's points binned
+    by several workgroups and added up; ties, and points on edges (listed by
+    several workgroups) among them.  As a whole run, in a batch, captured, and of
+    a resident tree."""
+    say("grid chain, heavy buckets", n, blobs, order)
+    rng = np.random.default_rng(n + blobs)
+    side = 400.0
+    x, y = rng.random(n) * side, rng.random(n) * side
+    k = int(n * 0.9)
+    at = rng.random((blobs, 2)) * (side - 20.0) + 5.0
+    b = rng.integers(0, blobs, k)
+    x[:k], y[:k] = at[b, 0] + rng.random(k) * 6.0, at[b, 1] + rng.random(k) * 6.0
+    x[: k // 50], y[: k // 70] = np.round(x[: k // 50]), np.round(y[: k // 70])
+    z = np.round(rng.normal(50.0, 2.0, n), 1)
+    z[::5003] = np.nan
+    if order == "random":
+        p = rng.permutation(n)
+        x, y, z = x[p], y[p], z[p]
+    want = _run(ctx, x, y, z, 10, 20, 0.8)
+    _run(ctx, x, y, z, 7, 13, 0.5)
+    tree = ctx.parallel_qtree(x, y, z)
+    assert np.array_equal(ctx.tree_run(tree, 10, 20, 0.8), want)
+    tree.free()
+    for graph in (False, True, True, True):
+        got = ctx.batch_run(*(np.concatenate([a, a]) for a in (x, y, z)),
+                            [(n, dict(wsize=10, bsize=20, overlap=0.8)),
+                             (n, dict(wsize=7, bsize=13, overlap=0.5))], graph=graph)
+        assert np.array_equal(got[0], want)
+        assert np.array_equal(got[1], O.run(x, y, z, 7, 13, 0.5, 32)[0])
