@@ -55,14 +55,15 @@ static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64
     // this many of them.  More buckets give a small launch more workgroups (1M
     // points: bins 21 us with 8192 points a bucket, 11 us with 2048); fewer give
     // a large one longer runs, which cost fewer loads (20M points: 129 us with
-    // 900 buckets, 102 us with 450) and fewer items (512 tiles, 329M points: 1.05
-    // ms with 4096 points a bucket, 0.99 ms with 8192).
+    // 900 buckets, 98 us with 450, 84 with 225; 12M points: 70 and 64 us with 512
+    // and 256) and fewer items (512 tiles, 329M points: 1.05 ms with 4096 points a
+    // bucket, 0.99 ms with 8192).
     const uint32_t cx = T.ax[0].ncol, cy = T.ax[1].ncol;
     auto buckets = [&](uint32_t lw, uint32_t lh) {
         return ((uint64_t)(cx - 1) / (1u << lw) + 1) * ((uint64_t)(cy - 1) / (1u << lh) + 1);
     };
     const uint64_t per = launch_points <= (2u << 20) ? 2048 : launch_points <= (16u << 20) ? 4096 : 8192;
-    const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(n / per, 16), 512);
+    const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(n / per, 16), launch_points <= (8u << 20) ? 512 : 256);
     uint32_t lw = 3, lh = 3;
     while (buckets(lw, lh) > want && lw + lh < 12)
         (lw <= lh ? lw : lh) += 1;
@@ -84,9 +85,10 @@ static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64
     // A lane reads four consecutive points of a run, a segment is 2^lpr lanes:
     // small segments waste the fewest lanes at the ends of runs, larger ones cost
     // fewer list entries (10k points in 16 buckets: 19 us with one lane, 13 with
-    // two; 96 mixed tiles: 0.67 ms with one, 0.69 with two, 0.72 with four).
+    // two; 96 mixed tiles: 0.67 ms with one, 0.69 with two, 0.72 with four; 100M
+    // points in runs of three: 1.01 ms with one, 0.87 with two).
     const double run = T.nst ? (double)n / ((double)T.nst * T.nb) : 1.0;
-    T.lpr = run <= 6.0 ? 0 : run <= 64.0 ? 1 : run <= 128.0 ? 2 : 3;
+    T.lpr = run <= 6.0 && n <= (8u << 20) ? 0 : run <= 64.0 ? 1 : run <= 128.0 ? 2 : 3;
     // An item is heavy at three times the mean (counted in whole segments), and not
     // below 65536 points: some 70 us of a workgroup's time.
     const double mean_item = ((double)mean + (double)T.nst * (2 << T.lpr)) / T.split;
