@@ -6,7 +6,7 @@
 // it lies in: its count and its (z, index).  The chain therefore streams the
 // cloud twice and works on cells from there on:
 //   k_grid_part     reads x, y, z once (24 B a point) and writes, per sort tile
-//                   of GRID_PTS points, the points grouped by bucket (a rectangle
+//                   of 2^lsp points, the points grouped by bucket (a rectangle
 //                   of cells that fits LDS) as z key and cell (12 B a point), all
 //                   writes linear, and where each bucket's run starts
 //   k_grid_bin      gathers a bucket's runs (12 B a point), reduces them in LDS
@@ -29,7 +29,7 @@
 
 namespace owm {
 
-constexpr int GP_NT = 512, GP_K = GRID_PTS / GP_NT;
+constexpr int GP_NT = 512;
 constexpr uint32_t KEY_NONE = 0x7FFFFFFFu, KEY_RARE = 0x80000000u;
 
 // Table entry whose range of off[] holds v, found by the whole workgroup at
@@ -137,17 +137,19 @@ __global__ __launch_bounds__(256) void k_grid_prep(GridDev G, FillRanges r, uint
 // of the tile) are in no window and no cell and get no record; kept, one workgroup
 // of the bins would gather them (20M points, a box of a tenth of each side: bins
 // 7.9 -> 0.02 ms, the whole run 8.3 -> 0.18 ms).  The test adds nothing measurable.
-template <bool TREE>
+template <bool TREE, int LSP>
 __global__ __launch_bounds__(GP_NT, 6) void k_grid_part(GridDev G, const double *__restrict__ X,
                                                       const double *__restrict__ Y,
                                                       const double *__restrict__ Z)
 {
+    constexpr uint32_t PTS = 1u << LSP;
+    constexpr int GP_K = PTS / GP_NT;
     extern __shared__ uint4 s_part[];
-    uint32_t *sRec = (uint32_t *)s_part;              // [GRID_PTS] records by bucket
-    uint32_t *hist = sRec + 3 * GRID_PTS;             // [nb + 1] counts, then offsets
+    uint32_t *sRec = (uint32_t *)s_part;              // [PTS] records by bucket
+    uint32_t *hist = sRec + 3 * PTS;             // [nb + 1] counts, then offsets
     uint32_t *sList = sRec;                           // points near an edge
-    uint32_t *sPool = sList + GRID_PTS;               // pool entry of a slot without a column
-    uint32_t *sW = sPool + GRID_PTS;                  // exact key of a slot near an edge
+    uint32_t *sPool = sList + PTS;               // pool entry of a slot without a column
+    uint32_t *sW = sPool + PTS;                  // exact key of a slot near an edge
     __shared__ uint32_t s_t, s_n, s_nr, s_base, s_w[GP_NT / 64];
     const uint32_t tid = threadIdx.x, u = blockIdx.x;
     if (tid == 0)
@@ -155,8 +157,8 @@ __global__ __launch_bounds__(GP_NT, 6) void k_grid_part(GridDev G, const double 
     const uint32_t t = find_entry(G.st_off, 0, G.ntiles, u, &s_t);
     const GridTile &T = G.tiles[t];
     const uint32_t st = u - T.st_off;
-    const uint32_t base = T.pt_off + st * GRID_PTS;
-    const uint32_t cnt = min((uint32_t)GRID_PTS, T.n - st * GRID_PTS);
+    const uint32_t base = T.pt_off + st * PTS;
+    const uint32_t cnt = min(PTS, T.n - st * PTS);
     const uint32_t nb = T.nb;
     double x[GP_K], y[GP_K], z[GP_K];
 #pragma unroll
@@ -301,7 +303,7 @@ __global__ __launch_bounds__(GP_NT, 6) void k_grid_part(GridDev G, const double 
     __syncthreads();
     // four records are three 16-byte words; a tile's records start at a multiple
     // of four, and the words behind its last record are its own padding
-    uint4 *out = (uint4 *)G.rec + ((uint64_t)T.rec_off + st * GRID_PTS) / 4 * 3;
+    uint4 *out = (uint4 *)G.rec + ((uint64_t)T.rec_off + st * PTS) / 4 * 3;
     const uint32_t words = (total + 3) / 4 * 3;
     for (uint32_t i = tid; i < words; i += GP_NT)
         out[i] = s_part[i];
@@ -419,6 +421,7 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
     const uint32_t lc = T.lw + T.lh, nc = 1u << lc, pt_off = T.pt_off, rec_off = T.rec_off;
     const uint32_t bucket = (item - T.item_off) / T.split;
     const uint32_t nb1 = T.nb + 1, lpr = T.lpr, seg_pts = (uint32_t)GB_SEG << lpr;
+    const uint32_t lsp = T.lsp;
     uint32_t left = T.heavy;  // points until the item is heavy
     for (uint32_t c = tid; c < nc + 64; c += NT) {
         sZ[c] = OWM_ZKEY_NONE;
@@ -453,7 +456,7 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
         for (uint32_t p0 = 0; p0 < total; p0 += GB_RUNS) {
             for (uint32_t e = max(at0, p0); e < min(at0 + nseg, p0 + GB_RUNS); ++e) {
                 const uint32_t a = o0 + (e - at0) * seg_pts;
-                sRun[e - p0] = make_uint2(s * GRID_PTS + a, min(seg_pts, o1 - a));
+                sRun[e - p0] = make_uint2((s << lsp) + a, min(seg_pts, o1 - a));
             }
             __syncthreads();
             const uint32_t here = min((uint32_t)GB_RUNS, total - p0);
@@ -464,7 +467,7 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
                 for (int h = 0; h < TWO; ++h) {
                     const uint32_t e = r0 + h * ngrp + grp;
                     const uint2 run = e < here ? sRun[e] : make_uint2(0u, 0u);
-                    id0[h] = pt_off + (run.x & ~GRID_SLOT_MASK);
+                    id0[h] = pt_off + (run.x >> lsp << lsp);
                     RecWord w[3] = {};
                     if (first < run.y) {
                         // four records in three loads (the last may hold the next
@@ -1011,12 +1014,14 @@ void launch_grid_prep(hipStream_t s, const GridDev &G, const FillRanges &r, uint
 }
 
 void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const double *y,
-                      const double *z, uint32_t sort_tiles, uint32_t max_nb)
+                      const double *z, uint32_t sort_tiles, uint32_t lsp, uint32_t max_nb)
 {
     if (!sort_tiles)
         return;
-    const uint32_t lds = GRID_PTS * 12u + (max_nb + 1) * 4u;
-    const auto k = G.zi ? k_grid_part<true> : k_grid_part<false>;
+    const uint32_t lds = (12u << lsp) + (max_nb + 1) * 4u;
+    const auto k = lsp == 10 ? (G.zi ? k_grid_part<true, 10> : k_grid_part<false, 10>)
+                   : lsp == 11 ? (G.zi ? k_grid_part<true, 11> : k_grid_part<false, 11>)
+                               : (G.zi ? k_grid_part<true, 12> : k_grid_part<false, 12>);
     hipLaunchKernelGGL(k, dim3(sort_tiles), dim3(GP_NT), lds, s, G, x, y, z);
 }
 
@@ -1085,8 +1090,12 @@ void launch_flags_out(hipStream_t s, const uint32_t *flags, uint32_t *host)
 hipError_t grid_kernels_init()
 {
     const std::pair<const void *, int> k[] = {
-        {(const void *)k_grid_part<false>, GRID_PTS * 12 + (GRID_MAX_BUCKETS + 1) * 4},
-        {(const void *)k_grid_part<true>, GRID_PTS * 12 + (GRID_MAX_BUCKETS + 1) * 4},
+        {(const void *)k_grid_part<false, 10>, (12 << 10) + (GRID_MAX_BUCKETS + 1) * 4},
+        {(const void *)k_grid_part<true, 10>, (12 << 10) + (GRID_MAX_BUCKETS + 1) * 4},
+        {(const void *)k_grid_part<false, 11>, (12 << 11) + (GRID_MAX_BUCKETS + 1) * 4},
+        {(const void *)k_grid_part<true, 11>, (12 << 11) + (GRID_MAX_BUCKETS + 1) * 4},
+        {(const void *)k_grid_part<false, 12>, (12 << 12) + (GRID_MAX_BUCKETS + 1) * 4},
+        {(const void *)k_grid_part<true, 12>, (12 << 12) + (GRID_MAX_BUCKETS + 1) * 4},
         {(const void *)k_grid_bin<256, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_bin<512, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_bin<256, 1, true>, BIN_LDS(GRID_MAX_CELLS)},

@@ -131,10 +131,9 @@ void launch_agg_levels(hipStream_t s, const TreeOut &T, const AggLevels &V);
 void launch_karras(hipStream_t s, const BatchDev &B, const TreeOut &T, const AggLevels &V);
 
 // ---- column grid (grid.hip) ----
-// Points per sort tile of the partition, and the packed (cell, slot) word: a
-// point's cell within its bucket above its slot within the sort tile.
-constexpr uint32_t GRID_SLOT_BITS = 12, GRID_PTS = 1u << GRID_SLOT_BITS;
-constexpr uint32_t GRID_SLOT_MASK = GRID_PTS - 1u;
+// The packed (cell, slot) word: a point's cell within its bucket above its slot
+// within its sort tile (of 2^lsp points, lsp <= GRID_SLOT_BITS).
+constexpr uint32_t GRID_SLOT_BITS = 12, GRID_SLOT_MASK = (1u << GRID_SLOT_BITS) - 1u;
 constexpr uint32_t GRID_CELL_BITS = 13, GRID_MAX_CELLS = 1u << GRID_CELL_BITS;
 constexpr uint32_t GRID_CELL_MASK = GRID_MAX_CELLS - 1u;
 constexpr uint32_t GRID_MAX_BUCKETS = 8192;
@@ -160,7 +159,7 @@ struct GridTile {
     uint64_t cell_off;  // first grid cell: [nb][split][2^(lw + lh)]
     uint32_t pt_off, n;
     uint32_t rec_off;            // first record (a multiple of 4)
-    uint32_t st_off, nst;        // sort tiles
+    uint32_t st_off, nst, lsp;   // sort tiles, of 2^lsp points (the same for all tiles of a launch)
     uint32_t lw, lh;             // a bucket is 2^lw columns x 2^lh rows
     uint32_t nbx, nby, nb;       // buckets
     uint32_t split, item_off;    // items: each bucket's sort tiles in `split` shares
@@ -229,7 +228,7 @@ hipError_t grid_kernels_init();
 void launch_grid_prep(hipStream_t s, const GridDev &G, const FillRanges &r, uint32_t windows,
                       const uint32_t *host_table, uint32_t table_words);
 void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const double *y,
-                      const double *z, uint32_t sort_tiles, uint32_t max_nb);
+                      const double *z, uint32_t sort_tiles, uint32_t lsp, uint32_t max_nb);
 // Items [item0, item0 + items) of the table entries [t0, t1); cells: the
 // largest bucket's.
 void launch_grid_bin(hipStream_t s, const GridDev &G, uint32_t t0, uint32_t t1, uint32_t item0,

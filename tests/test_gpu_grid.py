@@ -279,3 +279,12 @@ def test_heavy_buckets(ctx, n, blobs, order):
                              (n, dict(wsize=7, bsize=13, overlap=0.5))], graph=graph)
         assert np.array_equal(got[0], want)
         assert np.array_equal(got[1], O.run(x, y, z, 7, 13, 0.5, 32)[0])
+
+
+@pytest.mark.parametrize("n", [1023, 1025, 131_072, 131_073, 132_097, 524_288, 524_289, 528_385])
+def test_sort_tile_sizes(ctx, n):
+    """Either side of the points at which sort tiles grow, and of their ends."""
+    say("grid chain, sort tiles", n)
+    x, y, z = (a[:n].copy() for a in synth.scaled(synth.config_c1(seed=n), n).generate())
+    _run(ctx, x, y, z, 10, 20, 0.8)
+    _run(ctx, np.round(x, 2), np.round(y, 2), z, 7, 13, 0.5)
