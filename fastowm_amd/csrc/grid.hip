@@ -29,7 +29,8 @@
 
 namespace owm {
 
-constexpr int GP_NT = 512;
+// threads of the partition
+constexpr int gp_threads(int lsp) { return lsp == 13 ? 1024 : 512; }
 constexpr uint32_t KEY_NONE = 0x7FFFFFFFu, KEY_RARE = 0x80000000u;
 
 // Table entry whose range of off[] holds v, found by the whole workgroup at
@@ -137,13 +138,14 @@ __global__ __launch_bounds__(256) void k_grid_prep(GridDev G, FillRanges r, uint
 // of the tile) are in no window and no cell and get no record; kept, one workgroup
 // of the bins would gather them (20M points, a box of a tenth of each side: bins
 // 7.9 -> 0.02 ms, the whole run 8.3 -> 0.18 ms).  The test adds nothing measurable.
+// LSP 13: 100 KB of LDS, one workgroup per CU, for runs that would else be short.
 template <bool TREE, int LSP>
-__global__ __launch_bounds__(GP_NT, 6) void k_grid_part(GridDev G, const double *__restrict__ X,
+__global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_part(GridDev G, const double *__restrict__ X,
                                                       const double *__restrict__ Y,
                                                       const double *__restrict__ Z)
 {
     constexpr uint32_t PTS = 1u << LSP;
-    constexpr int GP_K = PTS / GP_NT;
+    constexpr int GP_NT = gp_threads(LSP), GP_K = PTS / GP_NT;
     extern __shared__ uint4 s_part[];
     uint32_t *sRec = (uint32_t *)s_part;              // [PTS] records by bucket
     uint32_t *hist = sRec + 3 * PTS;             // [nb + 1] counts, then offsets
@@ -1020,9 +1022,10 @@ void launch_grid_part(hipStream_t s, const GridDev &G, const double *x, const do
         return;
     const uint32_t lds = (12u << lsp) + (max_nb + 1) * 4u;
     const auto k = lsp == 10 ? (G.zi ? k_grid_part<true, 10> : k_grid_part<false, 10>)
+                   : lsp == 13 ? k_grid_part<false, 13>  // (no tree of that size comes here)
                    : lsp == 11 ? (G.zi ? k_grid_part<true, 11> : k_grid_part<false, 11>)
                                : (G.zi ? k_grid_part<true, 12> : k_grid_part<false, 12>);
-    hipLaunchKernelGGL(k, dim3(sort_tiles), dim3(GP_NT), lds, s, G, x, y, z);
+    hipLaunchKernelGGL(k, dim3(sort_tiles), dim3(gp_threads(lsp)), lds, s, G, x, y, z);
 }
 
 // LDS of the bins: the cells and 64 spare ones.
@@ -1096,6 +1099,7 @@ hipError_t grid_kernels_init()
         {(const void *)k_grid_part<true, 11>, (12 << 11) + (GRID_MAX_BUCKETS + 1) * 4},
         {(const void *)k_grid_part<false, 12>, (12 << 12) + (GRID_MAX_BUCKETS + 1) * 4},
         {(const void *)k_grid_part<true, 12>, (12 << 12) + (GRID_MAX_BUCKETS + 1) * 4},
+        {(const void *)k_grid_part<false, 13>, (12 << 13) + (GRID_MAX_BUCKETS + 1) * 4},
         {(const void *)k_grid_bin<256, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_bin<512, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_bin<256, 1, true>, BIN_LDS(GRID_MAX_CELLS)},

@@ -32,6 +32,29 @@ struct GridPlan {
 // largest bucket of a launch bounds the workgroups per CU for all of them.
 static int cell_class(uint32_t cells) { return cells <= 1024 ? 0 : cells <= 4096 ? 1 : 2; }
 
+// Sort tiles of 2^lsp points, and what follows from them.
+static void sort_tiles(GridTile &T, uint32_t lsp)
+{
+    T.lsp = lsp;
+    T.nst = (uint32_t)((T.n + (1ull << T.lsp) - 1) >> T.lsp);
+    const uint64_t mean = T.n / T.nb;
+    // A bucket's points beyond 32768 are shared out: more workgroups, more partial
+    // cells for the windows to add up (120M points: bins + windows 0.90 ms with
+    // 16384, 0.69 with 32768, 0.75 with 65536).
+    T.split = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(mean / 32768, 1), 16);
+    // A lane reads four consecutive points of a run, a segment is 2^lpr lanes:
+    // small segments waste the fewest lanes at the ends of runs, larger ones cost
+    // fewer list entries (10k points in 16 buckets: 19 us with one lane, 13 with
+    // two; 96 mixed tiles: 0.67 ms with one, 0.69 with two, 0.72 with four; 100M
+    // points in runs of three: 1.01 ms with one, 0.87 with two).
+    const double run = T.nst ? (double)T.n / ((double)T.nst * T.nb) : 1.0;
+    T.lpr = run <= 6.0 && T.n <= (8u << 20) ? 0 : run <= 64.0 ? 1 : run <= 128.0 ? 2 : 3;
+    // An item is heavy at three times the mean (counted in whole segments), and not
+    // below 65536 points: some 70 us of a workgroup's time.
+    const double mean_item = ((double)mean + (double)T.nst * (2 << T.lpr)) / T.split;
+    T.heavy = (uint32_t)std::max(65536.0, 3.0 * mean_item);
+}
+
 // Fills one tile's grid; false when the chain does not take it.
 static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64_t n,
                       uint64_t launch_points, uint32_t lsp)
@@ -76,24 +99,7 @@ static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64
     T.nbx = (cx - 1) / (1u << lw) + 1;
     T.nby = (cy - 1) / (1u << lh) + 1;
     T.nb = T.nbx * T.nby;
-    T.lsp = lsp;
-    T.nst = (uint32_t)((n + (1ull << T.lsp) - 1) >> T.lsp);
-    const uint64_t mean = n / T.nb;
-    // A bucket's points beyond 32768 are shared out: more workgroups, more partial
-    // cells for the windows to add up (120M points: bins + windows 0.90 ms with
-    // 16384, 0.69 with 32768, 0.75 with 65536).
-    T.split = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(mean / 32768, 1), 16);
-    // A lane reads four consecutive points of a run, a segment is 2^lpr lanes:
-    // small segments waste the fewest lanes at the ends of runs, larger ones cost
-    // fewer list entries (10k points in 16 buckets: 19 us with one lane, 13 with
-    // two; 96 mixed tiles: 0.67 ms with one, 0.69 with two, 0.72 with four; 100M
-    // points in runs of three: 1.01 ms with one, 0.87 with two).
-    const double run = T.nst ? (double)n / ((double)T.nst * T.nb) : 1.0;
-    T.lpr = run <= 6.0 && n <= (8u << 20) ? 0 : run <= 64.0 ? 1 : run <= 128.0 ? 2 : 3;
-    // An item is heavy at three times the mean (counted in whole segments), and not
-    // below 65536 points: some 70 us of a workgroup's time.
-    const double mean_item = ((double)mean + (double)T.nst * (2 << T.lpr)) / T.split;
-    T.heavy = (uint32_t)std::max(65536.0, 3.0 * mean_item);
+    sort_tiles(T, lsp);
     return true;
 }
 
@@ -125,7 +131,7 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
     // less work each (10k points: partition 14.8 -> 9.6 us with 1024; 300k points: 14.8
     // -> 11.2 with 2048, bins 12.0 -> 11.9; 1M points: 16.7 -> 14.1, but bins 12.1 ->
     // 12.9 for the shorter runs, 102 us a run with either).
-    const uint32_t lsp = launch_points <= (1u << 17) ? 10 : launch_points <= (1u << 19) ? 11 : 12;
+    uint32_t lsp = launch_points <= (1u << 17) ? 10 : launch_points <= (1u << 19) ? 11 : 12;
     P.pt_off.assign(n_tiles + 1, 0);
     for (uint32_t t = 0; t < n_tiles; ++t) {
         Derived D;
@@ -139,6 +145,17 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
         P.nwin += (uint64_t)D.ncols * D.nrows;
         P.nleaf += tiles[t].n / std::max(pick_leaf(ctx, tiles[t].n, 0), 1u) + 1;
     }
+    // 8192 points where the runs of every tile would be short, in launches that fill
+    // the device often (a workgroup has a CU to itself): partition and bins, 100M
+    // points in runs of three 654 + 882 us with 4096, 733 + 595 with 8192; 120M in
+    // runs of eight 805 + 637 and 869 + 492; 40M in runs of six 252 + 251 and 308 +
+    // 199; 20M in runs of twenty 123 + 85 and 173 + 70.
+    bool brief = launch_points >= (48u << 20);
+    for (const GridTile &T : raw)
+        brief = brief && (T.n == 0 || T.nb > 341);
+    if (brief)
+        for (GridTile &T : raw)
+            sort_tiles(T, 13);
     P.np = P.pt_off[n_tiles];
     // blocks of 32x32 windows where there are enough of them to occupy the
     // device and their cells fit (48 KB), else smaller

@@ -133,7 +133,7 @@ void launch_karras(hipStream_t s, const BatchDev &B, const TreeOut &T, const Agg
 // ---- column grid (grid.hip) ----
 // The packed (cell, slot) word: a point's cell within its bucket above its slot
 // within its sort tile (of 2^lsp points, lsp <= GRID_SLOT_BITS).
-constexpr uint32_t GRID_SLOT_BITS = 12, GRID_SLOT_MASK = (1u << GRID_SLOT_BITS) - 1u;
+constexpr uint32_t GRID_SLOT_BITS = 13, GRID_SLOT_MASK = (1u << GRID_SLOT_BITS) - 1u;
 constexpr uint32_t GRID_CELL_BITS = 13, GRID_MAX_CELLS = 1u << GRID_CELL_BITS;
 constexpr uint32_t GRID_CELL_MASK = GRID_MAX_CELLS - 1u;
 constexpr uint32_t GRID_MAX_BUCKETS = 8192;

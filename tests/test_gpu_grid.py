@@ -288,3 +288,24 @@ def test_sort_tile_sizes(ctx, n):
     x, y, z = (a[:n].copy() for a in synth.scaled(synth.config_c1(seed=n), n).generate())
     _run(ctx, x, y, z, 10, 20, 0.8)
     _run(ctx, np.round(x, 2), np.round(y, 2), z, 7, 13, 0.5)
+
+
+@pytest.mark.parametrize("cm", [False, True])
+def test_largest_sort_tiles(ctx, cm):
+    """A sparse tile of 50M points takes the largest sort tiles; against the tree
+    chain (an explicit leaf size), which is compared with the oracle elsewhere."""
+    say("grid chain, largest sort tiles", cm)
+    n = (48 << 20) + 8191
+    rng = np.random.default_rng(48)
+    side = np.sqrt(n / 3.0)
+    x, y = rng.random(n) * side, rng.random(n) * side
+    z = np.round(rng.normal(50.0, 3.0, n), 1)
+    if cm:
+        x, y = np.round(x, 2), np.round(y, 2)
+    want = ctx.run_tile(x, y, z, 10, 20, 0.8, 32)
+    ctx.profile(True)
+    got = ctx.run_tile(x, y, z, 10, 20, 0.8)
+    calls = ctx.profile_read()
+    ctx.profile(False)
+    assert calls["grid_partition"]["calls"] == 1
+    assert np.array_equal(got, want) and len(want) > 300_000
