@@ -345,7 +345,7 @@ void launch_qs_level(hipStream_t s, const QsDev &D, int d, float rd, double off)
 // (16 B a point read, 4 written), k_qs_bins counts a node's points per depth-12
 // cell in LDS and sums the counts upwards, depth by depth; k_qs_out does the
 // depths above and leaves the classes in host memory.  20M points, 24 bytes each:
-// 68 + 118 + 20 us, against 833 us for path keys (20 B), their histogram (4 B),
+// 68 + 99 + 20 us, against 833 us for path keys (20 B), their histogram (4 B),
 // three sort passes (8 B each) and binary searches per node.  The partition runs
 // at 5.9 TB/s; the bins are bound by latency (two workgroups of 64 KB of counts
 // to a CU, each a chain of run starts, records and twelve barriers).
@@ -537,24 +537,34 @@ __device__ __forceinline__ bool qf_depth(const QsFast &F, int d, const uint32_t 
     return open != 0;
 }
 
-constexpr int QB_NT = 512;
+// Two workgroups to a CU by their LDS: 1024 threads each fill its wave slots and
+// keep twice the loads of 512 in flight (20M points with clusters 121 -> 101 us,
+// 99 with the next chunk's run starts loaded ahead; 60M uniform points, all
+// launches: 418 -> 397 us).
+constexpr int QB_NT = 1024;
+
+// A bucket's run in sort tile s: its start, and above it its points.
+__device__ __forceinline__ uint32_t qf_run(const QsFast &F, uint32_t bucket, uint32_t s)
+{
+    if (s >= F.nst)
+        return 0;
+    const uint16_t *row = F.tab + (uint64_t)s * (QF_BUCKETS + 1) + bucket;
+    return (uint32_t)row[0] | (uint32_t)(row[1] - row[0]) << 16;
+}
 
 // Every run of a bucket, 16 lanes a run and four runs a group in flight:
-// f(record, sort tile).
+// f(record, sort tile).  v: the run in sort tile threadIdx.x.
 template <class Fn>
-__device__ __forceinline__ void qf_runs(const QsFast &F, uint32_t bucket, uint32_t *s_run, Fn f)
+__device__ __forceinline__ void qf_runs(const QsFast &F, uint32_t bucket, uint32_t v, uint32_t *s_run,
+                                        Fn f)
 {
     const uint32_t tid = threadIdx.x, grp = tid >> 4, gl = tid & 15u;
     constexpr uint32_t G = QB_NT / 16;
     for (uint32_t s0 = 0; s0 < F.nst; s0 += QB_NT) {
-        uint32_t v = 0;
-        if (s0 + tid < F.nst) {
-            const uint16_t *row = F.tab + (uint64_t)(s0 + tid) * (QF_BUCKETS + 1) + bucket;
-            v = (uint32_t)row[0] | (uint32_t)(row[1] - row[0]) << 16;
-        }
         __syncthreads();
         s_run[tid] = v;
         __syncthreads();
+        v = qf_run(F, bucket, s0 + QB_NT + tid);
         const uint32_t here = min((uint32_t)QB_NT, F.nst - s0);
         for (uint32_t r0 = grp; r0 < here; r0 += 4 * G) {
             uint32_t rec[4][2], len[4];
@@ -583,7 +593,7 @@ __device__ __forceinline__ void qf_runs(const QsFast &F, uint32_t bucket, uint32
     __syncthreads();
 }
 
-__global__ __launch_bounds__(QB_NT) void k_qs_bins(QsFast F)
+__global__ __launch_bounds__(QB_NT, 8) void k_qs_bins(QsFast F)
 {
     extern __shared__ uint4 s_qb[];
     uint32_t *bins = (uint32_t *)s_qb;  // [QF_BINS]
@@ -592,11 +602,10 @@ __global__ __launch_bounds__(QB_NT) void k_qs_bins(QsFast F)
     const uint32_t tid = threadIdx.x;
     // neighbouring buckets, whose runs share cache lines, on one XCD
     const uint32_t bucket = (blockIdx.x & 7u) * (QF_BUCKETS / 8) + (blockIdx.x >> 3);
-    uint32_t sum = 0, total;
-    for (uint32_t s = tid; s < F.nst; s += QB_NT) {
-        const uint16_t *row = F.tab + (uint64_t)s * (QF_BUCKETS + 1) + bucket;
-        sum += (uint32_t)(row[1] - row[0]);
-    }
+    const uint32_t run0 = qf_run(F, bucket, tid);
+    uint32_t sum = run0 >> 16, total;
+    for (uint32_t s = tid + QB_NT; s < F.nst; s += QB_NT)
+        sum += qf_run(F, bucket, s) >> 16;
     for (uint32_t b = tid; b < QF_BINS / 4; b += QB_NT)
         s_qb[b] = make_uint4(0, 0, 0, 0);
     for (uint32_t k = tid; k < QS_HB; k += QB_NT)
@@ -611,7 +620,7 @@ __global__ __launch_bounds__(QB_NT) void k_qs_bins(QsFast F)
             atomicOr(F.D.flags, QF_SKEW);
         return;
     }
-    qf_runs(F, bucket, s_run, [&](uint32_t r, uint32_t) { atomicAdd(&bins[r >> QF_SLOT_BITS], 1u); });
+    qf_runs(F, bucket, run0, s_run, [&](uint32_t r, uint32_t) { atomicAdd(&bins[r >> QF_SLOT_BITS], 1u); });
     uint32_t pc[QF_BINS / 4 / QB_NT];
     const bool deep = qf_depth<QB_NT>(F, QF_DEPTH, bins, QF_BINS / 4, s_hist, &s_open, pc);
     // cells still open: their points are listed by cell for k_qs_deep
@@ -646,7 +655,7 @@ __global__ __launch_bounds__(QB_NT) void k_qs_bins(QsFast F)
                 }
             }
             __syncthreads();
-            qf_runs(F, bucket, s_run, [&](uint32_t r, uint32_t st) {
+            qf_runs(F, bucket, qf_run(F, bucket, tid), s_run, [&](uint32_t r, uint32_t st) {
                 const uint32_t b = r >> QF_SLOT_BITS;
                 if (bins[b] != OWM_NONE)
                     F.ids[atomicAdd(&bins[b], 1u)] = st * QF_PTS + (r & QF_SLOT_MASK);
