@@ -309,3 +309,15 @@ def test_largest_sort_tiles(ctx, cm):
     ctx.profile(False)
     assert calls["grid_partition"]["calls"] == 1
     assert np.array_equal(got, want) and len(want) > 300_000
+
+
+@pytest.mark.parametrize("tiles,n,grid", [(64, 300, True), (65, 4095, False), (65, 4096, True), (300, 50, False)])
+def test_many_small_tiles(ctx, tiles, n, grid):
+    """Either side of the rule that leaves many tiles of few points to the tree chain."""
+    say("grid chain, many small tiles", tiles, n)
+    clouds = [synth.scaled(synth.config_c1(seed=s), n).generate() for s in range(tiles)]
+    ctx.profile(True)
+    _batch(ctx, clouds, [(10, 20, 0.8)] * tiles)
+    calls = ctx.profile_read()
+    ctx.profile(False)
+    assert (calls["grid_partition"]["calls"] > 0) == grid
