@@ -18,7 +18,7 @@
 // aggregates, about 35 B by stage 1 on window columns) a point moves 52 B after
 // its box is known.  Measured on MI355X: 512 uneven tiles (329M points) 14.6 ->
 // 5.3 ms (partition 2.3, bins 1.0, windows 0.3 ms), a 120M-point tile 6.6 ->
-// 1.9 ms, 20M points with clusters 1.38 -> 0.46 ms, 1M points 0.32 -> 0.10 ms,
+// 1.9 ms, 20M points with clusters 1.38 -> 0.43 ms, 1M points 0.32 -> 0.10 ms,
 // 10k points 0.25 -> 0.07 ms.
 // Points that lie on an edge (or between the two edges of a pair) have no
 // column; k_grid_part puts their exact window and cell ranges into a pool,
