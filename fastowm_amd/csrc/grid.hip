@@ -229,10 +229,12 @@ __global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_par
                 const uint32_t slot = sList[e], i = base + slot;
                 if (!(sW[slot] & KEY_RARE))
                     continue;
-                const uint32_t at = pbase + atomicAdd(&s_nr, 1u);
-                sPool[slot] = pbase != OWM_NONE ? at : 0u;
-                if (pbase == OWM_NONE)
+                if (pbase == OWM_NONE) {  // no room: nobody may read a place for it
+                    sW[slot] = nb << GRID_CELL_BITS;
                     continue;
+                }
+                const uint32_t at = pbase + atomicAdd(&s_nr, 1u);
+                sPool[slot] = at;
                 const AxisPassed px = axis_passed(T.ax[0], TREE ? G.xy[i].x : X[i]);
                 const AxisPassed py = axis_passed(T.ax[1], TREE ? G.xy[i].y : Y[i]);
                 const double zi = TREE ? G.zi[i].z : Z[i];

@@ -1,0 +1,63 @@
+"""The column-grid chain at the limits of its scratch memory: calls it hands to the
+tree chain, and calls that only just stay with it.  Which chain answered is read
+from the phases' launches; seeds are ids, against the oracle equal or wrong."""
+import numpy as np
+import pytest
+
+import pyoracle as O
+from fastowm_amd import owm, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print("[case]", *a, flush=True)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with owm.Context(0) as c:
+        # scratch of a larger call, so that nothing below starts from cleared memory
+        t = synth.scaled(synth.config_c2(seed=1), 2_000_003)
+        c.run_tile(*t.generate(), 12, 20, 0.8)
+        yield c
+
+
+def profiled(ctx, f):
+    ctx.profile(True)
+    got = f()
+    calls = {k: v["calls"] for k, v in ctx.profile_read().items()}
+    ctx.profile(False)
+    return got, calls
+
+
+def raster(side, origin=0.0, seed=0):
+    """side x side points one metre apart."""
+    g = origin + np.arange(side, dtype=np.float64)
+    x, y = (a.ravel() for a in np.meshgrid(g, g))
+    return x, y, np.round(np.random.default_rng(seed).normal(50.0, 3.0, len(x)), 1)
+
+
+@pytest.mark.parametrize("side,p", [(450, (10, 20, 0.9)), (450, (5, 20, 0.8)), (800, (5, 20, 0.8))])
+def test_full_pool(ctx, side, p):
+    """Rasters whose every point lies on an edge, in both sizes of sort tiles: as a
+    tile, beside a plain tile in a batch, and as a resident tree."""
+    say("grid limits, full pool", side, p)
+    c = raster(side, 512_000.0)
+    want = O.run(*c, *p, 32)[0]
+    got, calls = profiled(ctx, lambda: ctx.run_tile(*c, *p))
+    assert calls["grid_partition"] and calls["sort_tree_pass"] and np.array_equal(got, want)
+    plain = synth.scaled(synth.config_c1(seed=2), 132_072).generate()
+    q = dict(wsize=10, bsize=20, overlap=0.8)
+    desc = [(len(plain[0]), q), (len(c[0]), dict(wsize=p[0], bsize=p[1], overlap=p[2]))]
+    both = [np.concatenate(a) for a in zip(plain, c)]
+    for graph in (False, True, True, True):
+        a, b = ctx.batch_run(*both, desc, graph=graph)
+        assert np.array_equal(a, O.run(*plain, 10, 20, 0.8, 32)[0]) and np.array_equal(b, want)
+    tree = ctx.parallel_qtree(*c)
+    (minima, _), calls = profiled(ctx, lambda: ctx.stage1(tree, p[0], p[2], p[1]))
+    assert calls["grid_partition"] and calls["stage1"]
+    box = synth.bbox(c[0], c[1])
+    assert np.array_equal(minima, O.Tree(*c, O.params(*p, box, len(c[0]), 32)).stage1())
+    assert np.array_equal(ctx.tree_run(tree, *p), want)
+    tree.free()

@@ -1,0 +1,121 @@
+"""The column-grid chain's kernels and planning code on the CPU (tests/hipcpu):
+what cannot be provoked on a device, or must not be before it is right.  Against
+the oracle: seeds are ids, equal or wrong."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import pyoracle as O
+from fastowm_amd import synth
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "fastowm_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    """The chain built for the CPU: LDS arrays whose size the launch gives are globals
+    there, and the one inline wait has nothing to wait for."""
+    d = tmp_path_factory.mktemp("grid_cpu")
+    with open(os.path.join(CSRC, "grid.hip")) as f:
+        text = f.read()
+    text = text.replace("extern __shared__", "extern").replace(
+        'asm volatile("s_waitcnt vmcnt(0)" ::: "memory");', "")
+    assert "asm" not in text
+    src, out = str(d / "grid_source.h"), str(d / "grid_cpu")
+    with open(src, "w") as f:
+        f.write(text)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-D__HIPCC__", f'-DGRID_SOURCE="{src}"',
+                    "-I", os.path.join(HERE, "hipcpu"), "-I", CSRC, "-Wl,--unresolved-symbols=ignore-all", "-o", out,
+                    os.path.join(HERE, "hipcpu", "grid_cpu.cpp"), os.path.join(CSRC, "owm_grid.cpp"),
+                    os.path.join(CSRC, "owm_host.cpp")], check=True)
+    return out
+
+
+def chain(exe, clouds, params, mode=0, poke=0, calls=1, boxes=None):
+    """(taken, flags, ids per tile) of the chain for these tiles."""
+    head = [mode, poke, calls, len(clouds)]
+    for k, (c, p) in enumerate(zip(clouds, params)):
+        box = boxes[k] if boxes else None
+        head += [len(c[0]), *p, 1 if box else 0, *(box or (0, 0, 0, 0))]
+    paths = exe + ".in", exe + ".out"
+    with open(paths[0], "wb") as f:
+        np.array(head, np.float64).tofile(f)
+        for k in range(3):
+            np.concatenate([c[k] for c in clouds]).astype(np.float64).tofile(f)
+    r = subprocess.run([exe, *paths], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stderr)
+    with open(paths[1], "rb") as f:
+        status, taken, flags, count, stray = np.fromfile(f, np.int64, 5)
+        off = np.fromfile(f, np.int64, len(clouds) + 1)
+        ids = np.fromfile(f, np.uint32, count)
+    assert status == 0 and stray == 0
+    return bool(taken), int(flags), [ids[a:b] for a, b in zip(off, off[1:])] if taken else None
+
+
+def oracle(c, p, box=None):
+    return O.run(*c, *p, 32, box)[0]
+
+
+def raster(side, step=1.0, seed=0):
+    """side x side points on a lattice."""
+    g = np.arange(side) * step
+    x, y = (a.ravel().astype(np.float64) for a in np.meshgrid(g, g))
+    z = np.round(np.random.default_rng(seed).normal(50.0, 3.0, len(x)), 1)
+    return x, y, z
+
+
+def test_answers(exe):
+    """The chain on the CPU equals the oracle: plain tiles, centimetres, a resident
+    tree's seeds and minima, heavy stretches."""
+    t = synth.scaled(synth.config_c1(seed=3), 9_001).generate()
+    cm = tuple(np.round(a, 2) for a in synth.scaled(synth.config_c1(seed=4), 20_000).generate())
+    p = (10, 20, 0.8)
+    taken, flags, got = chain(exe, [t, cm], [p, (7, 13, 0.5)])
+    assert taken and flags == 0
+    assert np.array_equal(got[0], oracle(t, p)) and np.array_equal(got[1], oracle(cm, (7, 13, 0.5)))
+    taken, _, got = chain(exe, [cm], [p], mode=1)
+    assert taken and np.array_equal(got[0], oracle(cm, p))
+    taken, _, got = chain(exe, [cm], [p], mode=2)
+    assert taken and np.array_equal(
+        got[0], O.Tree(*cm, O.params(*p, synth.bbox(cm[0], cm[1]), len(cm[0]), 32)).stage1())
+
+
+@pytest.mark.parametrize("side,p", [(450, (10, 20, 0.9)), (800, (5, 20, 0.8))])
+def test_full_pool(exe, side, p):
+    """A raster whose every point lies on an edge: more than the pool holds.  The chain
+    hands the call on, and no kernel took a place that was never written for a point
+    (grid_cpu's device memory starts with points whose ids lie far out of range)."""
+    c = raster(side)
+    for mode in (0, 1, 2):
+        taken, flags, _ = chain(exe, [c], [p], mode=mode)
+        assert not taken and flags & 32
+
+
+def test_full_pool_beside_a_plain_tile(exe):
+    """The first share of the pool is the plain tile's, which has no use for it."""
+    plain = synth.scaled(synth.config_c1(seed=3), 132_072).generate()
+    taken, flags, _ = chain(exe, [plain, raster(247)], [(10, 20, 0.8), (5, 20, 0.8)])
+    assert not taken and flags & 32
+
+
+def heavy_cloud(n=160_000, seed=5, on_edges=0):
+    """Most points in a few square metres."""
+    rng = np.random.default_rng(seed)
+    x, y = rng.random(n) * 400.0, rng.random(n) * 400.0
+    k = int(n * 0.95)
+    x[:k], y[:k] = 101.0 + rng.random(k) * 6.0, 203.0 + rng.random(k) * 6.0
+    m = on_edges
+    x[:m], y[:m] = np.round(x[:m]), np.round(y[:m])
+    s = rng.permutation(n)
+    return x[s], y[s], np.round(rng.normal(50.0, 2.0, n), 1)
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("edges", [0, 3000])
+def test_heavy_stretches(exe, mode, edges):
+    c, p = heavy_cloud(on_edges=edges), (10, 20, 0.8)
+    taken, flags, got = chain(exe, [c], [p], mode=mode)
+    assert taken and flags == 0 and np.array_equal(got[0], oracle(c, p))
