@@ -371,6 +371,7 @@ __device__ __forceinline__ void queue_rest(const GridDev &G, const GridTile &T, 
             own[2] += ns;
         } else {
             atomicOr(G.err, GRID_ERR_POOL);
+            G.err[GRID_QUEUE_FULL] = 1u;
         }
     }
     __syncthreads();
@@ -616,8 +617,10 @@ __global__ __launch_bounds__(NT) void k_grid_heavy(GridDev G, uint32_t cap,
 {
     __shared__ uint32_t s_last;
     const uint32_t tid = threadIdx.x;
-    // (an overfull queue has entries that were never written)
-    if (*G.err & GRID_ERR_POOL)
+    // An overfull queue has entries that were never written.  (Not *G.err, which this
+    // launch may set: a workgroup's waves that read it at different times could go
+    // different ways, some into the barriers, some out.)
+    if (G.err[GRID_QUEUE_FULL])
         return;
     const GridHeavy H(G, cap);
     const uint32_t n = min(*H.n, cap);

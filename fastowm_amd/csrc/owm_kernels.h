@@ -142,6 +142,8 @@ constexpr uint32_t GRID_POOLS = 64;  // shares of the pool, each with a cursor o
 // heavy stretches) is full; a window block
 // has more rows than planned (cannot happen)
 constexpr uint32_t GRID_ERR_POOL = 32u, GRID_ERR_ROWS = 64u;
+// Word behind *err that k_grid_bin alone sets, and only later launches read.
+constexpr uint32_t GRID_QUEUE_FULL = 1u;
 
 // A point without a column (on an edge, or between the edges of a pair) with
 // the windows [wx0, wx1) x [wy0, wy1) and stage-3 cells [gx0, gx1) x [gy0, gy1)

@@ -3,10 +3,11 @@
 //   grid_cpu IN OUT
 // IN: doubles {mode, poke, calls, tiles, then per tile {n, wsize, bsize,
 // overlap, has box, box[4]}}, then x, y, z.  Modes: 0 a whole run, 1 the seeds and
-// 2 the minima of a resident tree (one tile, its points in reverse).  poke: every
-// workgroup of k_grid_heavy finds GRID_ERR_POOL set by another one of the launch before
-// its wave 4 first runs.  OUT: int64 {status, taken, flags, count, stray marks}, tile
-// ranges (tiles + 1 of them), ids.
+// 2 the minima of a resident tree (one tile, its points in reverse).  poke: 1, every
+// workgroup of k_grid_heavy finds GRID_ERR_POOL set by another one of the launch
+// before its wave 4 first runs; 2, the queue of heavy stretches holds two.
+// OUT: int64 {status, taken, flags, count, stray marks}, tile ranges (tiles + 1
+// of them), ids.
 #include "../../fastowm_amd/csrc/owm_host.h"
 #include <math.h>
 
@@ -111,8 +112,11 @@ int main(int argc, char **argv)
     hipcpu::before_launch = [&](const void *k, const void *arg) {
         if (k != (const void *)&k_flags_out)  // (whose first argument is no GridDev)
             err = ((const GridDev *)arg)->err;
+        if (head[1] == 2 && k == (const void *)&k_grid_bin<512, 1, false>)
+            for (uint32_t t = 0; t < T; ++t)
+                const_cast<GridTile *>(((const GridDev *)arg)->tiles)[t].heavy_cap = 2;
     };
-    if (head[1])
+    if (head[1] == 1)
         hipcpu::before_wave = [&](const void *k, uint32_t, uint32_t w) {
             if (w == 4 && (k == (const void *)&k_grid_heavy<512, false> ||
                            k == (const void *)&k_grid_heavy<512, true>))

@@ -119,3 +119,19 @@ def test_heavy_stretches(exe, mode, edges):
     c, p = heavy_cloud(on_edges=edges), (10, 20, 0.8)
     taken, flags, got = chain(exe, [c], [p], mode=mode)
     assert taken and flags == 0 and np.array_equal(got[0], oracle(c, p))
+
+
+def test_flag_raised_during_the_heavy_launch(exe):
+    """Another workgroup of the launch finds its list full while waves of this one
+    start: a workgroup's waves go on or stop together."""
+    c, p = heavy_cloud(on_edges=3000), (10, 20, 0.8)
+    taken, _, _ = chain(exe, [c], [p], poke=1)
+    assert not taken
+
+
+def test_full_queue(exe):
+    """More heavy stretches than the queue holds: entries that were never written are
+    not taken for stretches."""
+    c, p = heavy_cloud(on_edges=3000), (10, 20, 0.8)
+    taken, flags, _ = chain(exe, [c], [p], poke=2)
+    assert not taken and flags & 32
