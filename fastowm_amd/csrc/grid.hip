@@ -124,6 +124,16 @@ __global__ __launch_bounds__(256) void k_grid_prep(GridDev G, FillRanges r, uint
 
 // ------------------------------------------------------------- partition --
 
+// Word k of *p as other XCDs' atomics leave it (agent scope: sc1).  To the compiler an
+// atomic load might write, and what follows it would not come by scalar loads: the
+// partition would keep the tile's fields in lanes' registers and spill them (8M
+// points 97 -> 154 us).
+__device__ __forceinline__ uint32_t load_past_caches(uint32_t *p, uint32_t k)
+{
+    return __builtin_amdgcn_raw_buffer_load_b32(
+        __builtin_amdgcn_make_buffer_rsrc(p, 0, 4 * k + 4, 0x00027000), 4 * k, 0, 16);
+}
+
 // Bound by HBM: 36 B a point at 5.2 TB/s (2.27 ms for 329M points; a plain copy
 // reaches 4.9 TB/s).  The output of a sort tile is one linear stretch, so runs
 // need no global offsets (no histogram pass, no look-back); the bins gather
@@ -152,11 +162,16 @@ __global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_par
     uint32_t *sList = sRec;                           // points near an edge
     uint32_t *sPool = sList + PTS;               // pool entry of a slot without a column
     uint32_t *sW = sPool + PTS;                  // exact key of a slot near an edge
-    __shared__ uint32_t s_t, s_n, s_nr, s_base, s_w[GP_NT / 64];
+    __shared__ uint32_t s_t, s_n, s_nr, s_base, s_stop, s_w[GP_NT / 64];
     const uint32_t tid = threadIdx.x, u = blockIdx.x;
-    if (tid == 0)
+    if (tid == 0) {
         s_n = s_nr = 0;
+        // (other workgroups may set it meanwhile: one thread reads it for all)
+        s_stop = load_past_caches(G.err, GRID_STOP_PART);
+    }
     const uint32_t t = find_entry(G.st_off, 0, G.ntiles, u, &s_t);
+    if (s_stop)
+        return;
     const GridTile &T = G.tiles[t];
     const uint32_t st = u - T.st_off;
     const uint32_t base = T.pt_off + st * PTS;
@@ -219,8 +234,11 @@ __global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_par
                 const uint32_t share = u & (GRID_POOLS - 1u);
                 const uint32_t at = atomicAdd(G.pool_used + share * 32, nr);
                 s_base = at + nr <= G.pool_cap ? share * G.pool_cap + at : OWM_NONE;
-                if (s_base == OWM_NONE)
+                const bool many = nr * 6 > cnt && atomicAdd(G.pool_used + 8, 1u) >= G.many_cap;
+                if (s_base == OWM_NONE || many) {
                     atomicOr(G.err, GRID_ERR_POOL);
+                    atomicOr(G.err + GRID_STOP_PART, 1u);
+                }
                 s_nr = 0;
             }
             __syncthreads();
@@ -334,8 +352,10 @@ __device__ __forceinline__ void flush_rare(const GridDev &G, uint32_t item, cons
         const uint32_t share = item & (GRID_POOLS - 1u);
         const uint32_t at = atomicAdd(G.pool_used + share * 32 + 16, n + 2u);
         *s_base = at + n + 2u <= G.list_cap ? share * G.list_cap + at : OWM_NONE;
-        if (*s_base == OWM_NONE)
+        if (*s_base == OWM_NONE) {
             atomicOr(G.err, GRID_ERR_POOL);
+            G.err[SUB ? GRID_STOP_HEAVY : GRID_STOP_BIN] = 1u;
+        }
     }
     __syncthreads();
     const uint32_t base = *s_base;
@@ -371,7 +391,7 @@ __device__ __forceinline__ void queue_rest(const GridDev &G, const GridTile &T, 
             own[2] += ns;
         } else {
             atomicOr(G.err, GRID_ERR_POOL);
-            G.err[GRID_QUEUE_FULL] = 1u;
+            G.err[GRID_STOP_BIN] = 1u;
         }
     }
     __syncthreads();
@@ -582,6 +602,8 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
                                                  uint32_t item0, uint32_t items, uint32_t cells)
 {
     __shared__ uint32_t s_t;
+    if (G.err[GRID_STOP_PART])
+        return;
     // consecutive items (neighbouring buckets, whose runs share cache lines)
     // on one XCD: workgroups go round the eight XCDs
     const uint32_t per = (items + 7u) / 8u;
@@ -620,7 +642,7 @@ __global__ __launch_bounds__(NT) void k_grid_heavy(GridDev G, uint32_t cap,
     // An overfull queue has entries that were never written.  (Not *G.err, which this
     // launch may set: a workgroup's waves that read it at different times could go
     // different ways, some into the barriers, some out.)
-    if (G.err[GRID_QUEUE_FULL])
+    if (G.err[GRID_STOP_PART] | G.err[GRID_STOP_BIN])
         return;
     const GridHeavy H(G, cap);
     const uint32_t n = min(*H.n, cap);
@@ -727,6 +749,8 @@ __global__ __launch_bounds__(GW_NT) void k_grid_windows(GridDev G, const double 
     __shared__ int sx0[32], sx1[32], sy0[32], sy1[32];
     __shared__ uint2 sSeg[GW_SEGS];
     const uint32_t tid = threadIdx.x;
+    if (G.err[GRID_STOP_PART] | G.err[GRID_STOP_BIN] | G.err[GRID_STOP_HEAVY])
+        return;
     if (tid == 0)
         s_nseg = 0;
     const uint32_t t = find_entry(G.blk_off, 0, G.ntiles, blockIdx.x, &s_t);
@@ -816,6 +840,8 @@ __global__ __launch_bounds__(GW_NT) void k_grid_windows(GridDev G, const double 
             }
     }
     __syncthreads();
+    if (s_nseg > GW_SEGS)  // (flagged above)
+        return;
     // rows to window columns: a row belongs to bw lanes of one wave, whose
     // reads of it all precede its writes
     for (uint32_t rr = tid >> lb; rr < nr; rr += GW_NT >> lb) {
@@ -840,7 +866,7 @@ __global__ __launch_bounds__(GW_NT) void k_grid_windows(GridDev G, const double 
                 agg_add(win[k], mZ[r * pitch + w], mId[r * pitch + w], mCnt[r * pitch + w]);
     }
     __syncthreads();  // the row sums are no longer needed: their memory holds the windows
-    const uint32_t nseg = min(s_nseg, GW_SEGS);
+    const uint32_t nseg = s_nseg;
     if (nseg) {
         const uint32_t lane = tid & 63, wv = tid >> 6;
 #pragma unroll
@@ -945,6 +971,8 @@ __global__ __launch_bounds__(256) void k_grid_cells(GridDev G)
 {
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (*G.err)  // (this launch sets none)
+        return;
     for (uint32_t c = blockIdx.x * 4 + w; c < G.ngcell; c += gridDim.x * 4) {
         if (G.cell_flag[c])
             continue;

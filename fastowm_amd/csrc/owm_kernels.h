@@ -142,8 +142,11 @@ constexpr uint32_t GRID_POOLS = 64;  // shares of the pool, each with a cursor o
 // heavy stretches) is full; a window block
 // has more rows than planned (cannot happen)
 constexpr uint32_t GRID_ERR_POOL = 32u, GRID_ERR_ROWS = 64u;
-// Word behind *err that k_grid_bin alone sets, and only later launches read.
-constexpr uint32_t GRID_QUEUE_FULL = 1u;
+// Words behind *err: the launch found that the chain will not answer the call.
+// k_grid_part's later workgroups and every later launch then return at once.  A launch
+// sets its own word and branches on those before it, which no longer change (the
+// partition's is read by one thread of a workgroup).
+constexpr uint32_t GRID_STOP_PART = 1u, GRID_STOP_BIN = 2u, GRID_STOP_HEAVY = 3u;
 
 // A point without a column (on an edge, or between the edges of a pair) with
 // the windows [wx0, wx1) x [wy0, wy1) and stage-3 cells [gx0, gx1) x [gy0, gy1)
@@ -194,8 +197,11 @@ struct GridDev {
     GridRare *pool;          // points without a column
     uint32_t *heads;         // [items] the item's first block in list, or OWM_NONE
     uint32_t *list;          // blocks {n, next block, n pool entries}
-    uint32_t *pool_used;     // [GRID_POOLS * 32] used of each share of pool (word 0) and list (16)
+    // [GRID_POOLS * 32] used of each share of pool (word 0) and list (16); word 8 of the
+    // first: sort tiles with many points without a column
+    uint32_t *pool_used;
     uint32_t pool_cap, list_cap;  // entries (words) per share
+    uint32_t many_cap;       // sort tiles with many points without a column before the call is handed on
     uint32_t *seen, *llp;    // point bitmaps: one window, two (LLPs, then seeds)
     uint32_t *cell_flag;     // [ngcell] stage-3 cells that hold an LLP
     uint4 *heavy;            // GridHeavy

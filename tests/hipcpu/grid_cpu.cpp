@@ -6,8 +6,9 @@
 // 2 the minima of a resident tree (one tile, its points in reverse).  poke: 1, every
 // workgroup of k_grid_heavy finds GRID_ERR_POOL set by another one of the launch
 // before its wave 4 first runs; 2, the queue of heavy stretches holds two.
-// OUT: int64 {status, taken, flags, count, stray marks}, tile ranges (tiles + 1
-// of them), ids.
+// OUT: int64 {status, taken, flags, count, stray marks, barriers passed by launches that
+// began after the flag was raised, by k_grid_part, its workgroups}, tile ranges (tiles
+// + 1 of them), ids.
 #include "../../fastowm_amd/csrc/owm_host.h"
 #include <math.h>
 
@@ -109,9 +110,25 @@ int main(int argc, char **argv)
     hipcpu::stale.assign((const unsigned char *)&low, (const unsigned char *)(&low + 1));
     owm_ctx *ctx = new owm_ctx;
     uint32_t *err = nullptr;
+    int64_t after = 0, part = 0, groups = 0, mark = 0, kind = 0;
+    auto count_barriers = [&]() {
+        (kind == 1 ? after : part) += kind ? hipcpu::barriers - mark : 0;
+        mark = hipcpu::barriers;
+        kind = 0;
+    };
     hipcpu::before_launch = [&](const void *k, const void *arg) {
         if (k != (const void *)&k_flags_out)  // (whose first argument is no GridDev)
             err = ((const GridDev *)arg)->err;
+        count_barriers();
+        const void *const parts[4] = {(const void *)&k_grid_part<false, 10>, (const void *)&k_grid_part<false, 11>,
+                                      (const void *)&k_grid_part<false, 12>, (const void *)&k_grid_part<true, 12>};
+        for (const void *p : parts)
+            if (k == p) {
+                groups = ((const GridDev *)arg)->st_off[((const GridDev *)arg)->ntiles];
+                kind = 2;
+            }
+        if (!kind && k != (const void *)&k_grid_prep && k != (const void *)&k_flags_out && *err)
+            kind = 1;
         if (head[1] == 2 && k == (const void *)&k_grid_bin<512, 1, false>)
             for (uint32_t t = 0; t < T; ++t)
                 const_cast<GridTile *>(((const GridDev *)arg)->tiles)[t].heavy_cap = 2;
@@ -157,8 +174,9 @@ int main(int argc, char **argv)
     if (status == 0 && !taken)
         count = 0;
     FILE *o = fopen(argv[2], "wb");
-    const int64_t head_out[5] = {status, taken, err ? *err : 0, (int64_t)count, stray};
-    fwrite(head_out, 8, 5, o);
+    count_barriers();
+    const int64_t head_out[8] = {status, taken, err ? *err : 0, (int64_t)count, stray, after, part, groups};
+    fwrite(head_out, 8, 8, o);
     fwrite(off.data(), 8, T + 1, o);
     fwrite(ids.data(), 4, count, o);
     fclose(o);

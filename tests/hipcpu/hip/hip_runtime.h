@@ -62,6 +62,7 @@ inline bool any = false, any_out = false;
 inline const std::function<void()> *body = nullptr;
 // called before the given wave of a workgroup first runs: kernel, workgroup, wave
 inline std::function<void(const void *, uint32_t, uint32_t)> before_wave;
+inline uint64_t barriers = 0;  // passed by workgroups so far
 // called before a launch: kernel, its first argument
 inline std::function<void(const void *, const void *)> before_launch;
 
@@ -134,6 +135,7 @@ inline void run_block(const void *kernel, uint32_t n)
             return;
         if (done)
             die("a barrier that some threads left behind");
+        ++barriers;
         any_out = any;
         any = false;
         for (uint32_t i = 0; i < n; ++i)
@@ -230,6 +232,13 @@ inline unsigned long long __ballot(int p)
         if (((hipcpu::arrived[w] >> l) & 1ull) && hipcpu::snap[w][l])
             m |= 1ull << l;
     return m;
+}
+inline const char *__builtin_amdgcn_make_buffer_rsrc(void *p, int, uint32_t, uint32_t) { return (const char *)p; }
+inline uint32_t __builtin_amdgcn_raw_buffer_load_b32(const char *p, uint32_t at, uint32_t, int)
+{
+    uint32_t v;
+    memcpy(&v, p + at, 4);
+    return v;
 }
 template <class T> T min(T a, T b) { return b < a ? b : a; }
 template <class T> T max(T a, T b) { return a < b ? b : a; }

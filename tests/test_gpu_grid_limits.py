@@ -61,3 +61,21 @@ def test_full_pool(ctx, side, p):
     assert np.array_equal(minima, O.Tree(*c, O.params(*p, box, len(c[0]), 32)).stage1())
     assert np.array_equal(ctx.tree_run(tree, *p), want)
     tree.free()
+
+
+@pytest.mark.parametrize("frac,grid", [(0.10, True), (0.30, False)])
+def test_many_on_edges(ctx, frac, grid):
+    """More than 4M points: beyond a sixth of them on edges the tree chain answers.
+    Against the tree chain, which is compared with the oracle elsewhere."""
+    say("grid limits, many on edges", frac)
+    rng = np.random.default_rng(4)
+    n = (4 << 20) + 5
+    side = 900.0
+    x, y = rng.random(n) * side, rng.random(n) * side
+    x[:2], y[:2] = (0.0, side), (0.0, side)
+    m = rng.random(n) < frac
+    x[m] = np.floor(x[m])
+    c = x, y, np.round(rng.normal(50.0, 3.0, n), 1)
+    want = ctx.run_tile(*c, 5, 20, 0.8, 32)
+    got, calls = profiled(ctx, lambda: ctx.run_tile(*c, 5, 20, 0.8))
+    assert (calls["sort_tree_pass"] == 0) == grid and np.array_equal(got, want)

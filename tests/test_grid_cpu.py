@@ -48,10 +48,11 @@ def chain(exe, clouds, params, mode=0, poke=0, calls=1, boxes=None):
     r = subprocess.run([exe, *paths], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, (r.returncode, r.stderr)
     with open(paths[1], "rb") as f:
-        status, taken, flags, count, stray = np.fromfile(f, np.int64, 5)
+        status, taken, flags, count, stray, *work = np.fromfile(f, np.int64, 8)
         off = np.fromfile(f, np.int64, len(clouds) + 1)
         ids = np.fromfile(f, np.uint32, count)
     assert status == 0 and stray == 0
+    chain.after, chain.part, chain.groups = work
     return bool(taken), int(flags), [ids[a:b] for a, b in zip(off, off[1:])] if taken else None
 
 
@@ -135,3 +136,32 @@ def test_full_queue(exe):
     c, p = heavy_cloud(on_edges=3000), (10, 20, 0.8)
     taken, flags, _ = chain(exe, [c], [p], poke=2)
     assert not taken and flags & 32
+
+
+def test_handed_on_early(exe):
+    """A raster whose every point lies on an edge: once the pool is full no further
+    sort tile is partitioned, and the launches behind it do nothing."""
+    taken, flags, _ = chain(exe, [raster(800)], [(5, 20, 0.8)])
+    assert not taken and flags & 32
+    whole = chain.part
+    chain(exe, [tuple(a * 0.93 for a in raster(800))], [(5, 20, 0.8)])  # (off the edges: every sort tile)
+    per_tile = chain.part / chain.groups
+    assert chain.after == 0 and whole < 0.6 * per_tile * chain.groups
+
+
+@pytest.mark.parametrize("frac,ok", [(0.10, True), (0.25, False)])
+def test_many_on_edges(exe, frac, ok):
+    """Beyond 4M points a sixth of the points on edges in a quarter of the sort tiles
+    decides; a few sort tiles full of them do not."""
+    n = (4 << 20) + 4096
+    rng = np.random.default_rng(3)
+    side = 400.0
+    x, y = rng.random(n) * side, rng.random(n) * side
+    x[:2], y[:2] = (0.0, side), (0.0, side)
+    x[rng.random(n) < frac] //= 1.0
+    x[200_000:260_000] //= 1.0
+    z = np.round(rng.normal(50.0, 3.0, n), 1)
+    taken, flags, got = chain(exe, [(x, y, z)], [(5, 20, 0.8)])
+    assert taken == ok and (flags == 0) == ok and chain.after == 0
+    # (a taken cloud passes 11 barriers a sort tile)
+    assert ok or chain.part < 0.4 * 11 * chain.groups
