@@ -231,9 +231,14 @@ __global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_par
             // their ranges go to the pool (counted again: few points take this)
             __syncthreads();
             if (tid == 0) {
-                const uint32_t share = u & (GRID_POOLS - 1u);
-                const uint32_t at = atomicAdd(G.pool_used + share * 32, nr);
-                s_base = at + nr <= G.pool_cap ? share * G.pool_cap + at : OWM_NONE;
+                // (a share asked for more than it has left is closed, and the next one
+                // asked: points on edges may lie in few sort tiles)
+                s_base = OWM_NONE;
+                for (uint32_t k = 0; k < GRID_POOLS && s_base == OWM_NONE; ++k) {
+                    const uint32_t share = (u + k) & (GRID_POOLS - 1u);
+                    const uint32_t at = atomicAdd(G.pool_used + share * 32, nr);
+                    s_base = at + nr <= G.pool_cap ? share * G.pool_cap + at : OWM_NONE;
+                }
                 const bool many = nr * 6 > cnt && atomicAdd(G.pool_used + 8, 1u) >= G.many_cap;
                 if (s_base == OWM_NONE || many) {
                     atomicOr(G.err, GRID_ERR_POOL);
@@ -349,7 +354,9 @@ __device__ __forceinline__ void flush_rare(const GridDev &G, uint32_t item, cons
                                            uint32_t n, uint32_t *s_base, uint32_t &head)
 {
     if (threadIdx.x == 0) {
-        const uint32_t share = item & (GRID_POOLS - 1u);
+        // (the first entry spreads an item's blocks over the shares: most listed points
+        // may lie in one bucket)
+        const uint32_t share = (item + list[0]) & (GRID_POOLS - 1u);
         const uint32_t at = atomicAdd(G.pool_used + share * 32 + 16, n + 2u);
         *s_base = at + n + 2u <= G.list_cap ? share * G.list_cap + at : OWM_NONE;
         if (*s_base == OWM_NONE) {
@@ -794,10 +801,11 @@ __global__ __launch_bounds__(GW_NT) void k_grid_windows(GridDev G, const double 
             while (h != OWM_NONE) {
                 const uint32_t n = G.list[h], next = G.list[h + 1];
                 const uint32_t e = atomicAdd(&s_nseg, 1u);
-                if (e < GW_SEGS)
-                    sSeg[e] = make_uint2(h + 2, n);
-                else
+                if (e >= GW_SEGS) {
                     atomicOr(G.err, GRID_ERR_POOL);
+                    break;
+                }
+                sSeg[e] = make_uint2(h + 2, n);
                 h = next;
             }
         }

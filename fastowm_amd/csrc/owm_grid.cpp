@@ -231,9 +231,11 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
         T.heavy_sub = (uint32_t)std::max<uint64_t>(16384, P.np / 256);
         T.heavy_cap = P.heavy_cap;
     }
-    // a quarter of the points may lie on edges before the tree chain takes over
-    P.pool_cap = (P.np / 4 + 65536) / GRID_POOLS;
-    P.list_cap = P.pool_cap + P.pool_cap / 64 + 2 * (items / GRID_POOLS + 1);
+    // A quarter of the points may lie on edges before the tree chain takes over.  The
+    // end of a share that a sort tile's points do not fit is lost, so every share has
+    // room for one more; the lists' blocks are spread by chance, over twice the words.
+    P.pool_cap = (P.np / 4 + 65536) / GRID_POOLS + (1u << P.t[0].lsp);
+    P.list_cap = 2 * P.pool_cap + 2 * (items / GRID_POOLS + 1) + 1024;
     // A point without a column costs the windows 0.3 ns and more, ten times what the
     // chain takes for another, so beyond 4M points (where launches no longer bound the
     // tree chain) clouds with more than a sixth of them are the tree chain's (windows of

@@ -79,3 +79,41 @@ def test_many_on_edges(ctx, frac, grid):
     want = ctx.run_tile(*c, 5, 20, 0.8, 32)
     got, calls = profiled(ctx, lambda: ctx.run_tile(*c, 5, 20, 0.8))
     assert (calls["sort_tree_pass"] == 0) == grid and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("frac", [0.05, 0.12, 0.24])
+@pytest.mark.parametrize("order", ["random", "scan"])
+def test_share_on_edges(ctx, frac, order):
+    """A share of the points on edges, in one tile and in one of a batch: below a
+    quarter the column grid answers, every window block meets listed points."""
+    say("grid limits, share on edges", frac, order)
+    rng = np.random.default_rng(int(100 * frac))
+    n = 300_000
+    x, y = rng.random(n) * 190.0, rng.random(n) * 190.0
+    x[:2], y[:2] = (0.0, 190.0), (0.0, 190.0)
+    m = rng.random(n) < frac / 2
+    x[m], y[~m & (rng.random(n) < frac / 2)] = np.round(x[m]), 77.0
+    if order == "scan":
+        s = np.argsort(y, kind="stable")
+        x, y = x[s], y[s]
+    c = x, y, np.round(rng.normal(50.0, 3.0, n), 1)
+    want = O.run(*c, 5, 20, 0.8, 32)[0]
+    got, calls = profiled(ctx, lambda: ctx.run_tile(*c, 5, 20, 0.8))
+    assert calls["grid_partition"] == 1 and calls["sort_tree_pass"] == 0
+    assert np.array_equal(got, want)
+
+
+def test_longest_lists(ctx):
+    """More listed points in one bucket than a window block takes: the tree chain
+    answers.  Against the tree chain, as above."""
+    say("grid limits, longest lists")
+    rng = np.random.default_rng(9)
+    n = 2_000_000
+    x, y = rng.random(n) * 500.0, rng.random(n) * 500.0
+    m = rng.random(n) < 0.2
+    x[m], y[m] = 100.0, 140.0 + rng.random(m.sum())
+    x[:2], y[:2] = (0.0, 500.0), (0.0, 500.0)
+    c = x, y, np.round(rng.normal(50.0, 3.0, n), 1)
+    want = ctx.run_tile(*c, 10, 20, 0.8, 32)
+    got, calls = profiled(ctx, lambda: ctx.run_tile(*c, 10, 20, 0.8))
+    assert calls["sort_tree_pass"] > 0 and np.array_equal(got, want)

@@ -95,11 +95,15 @@ def test_full_pool(exe, side, p):
         assert not taken and flags & 32
 
 
-def test_full_pool_beside_a_plain_tile(exe):
-    """The first share of the pool is the plain tile's, which has no use for it."""
-    plain = synth.scaled(synth.config_c1(seed=3), 132_072).generate()
-    taken, flags, _ = chain(exe, [plain, raster(247)], [(10, 20, 0.8), (5, 20, 0.8)])
-    assert not taken and flags & 32
+@pytest.mark.parametrize("side,ok", [(247, True), (560, False)])
+def test_raster_beside_a_plain_tile(exe, side, ok):
+    """The first shares of the pool are the plain tile's, which has no use for them."""
+    tiles = synth.scaled(synth.config_c1(seed=3), 132_072).generate(), raster(side)
+    params = (10, 20, 0.8), (5, 20, 0.8)
+    taken, flags, got = chain(exe, tiles, params)
+    assert taken == ok and bool(flags & 32) != ok
+    for k in range(2 if ok else 0):
+        assert np.array_equal(got[k], oracle(tiles[k], params[k]))
 
 
 def heavy_cloud(n=160_000, seed=5, on_edges=0):
@@ -165,3 +169,35 @@ def test_many_on_edges(exe, frac, ok):
     assert taken == ok and (flags == 0) == ok and chain.after == 0
     # (a taken cloud passes 11 barriers a sort tile)
     assert ok or chain.part < 0.4 * 11 * chain.groups
+
+
+@pytest.mark.parametrize("place", ["sort tiles", "bucket"])
+def test_places_of_other_shares(exe, place):
+    """Points on edges in few sort tiles, or in one bucket: the pool's and the lists'
+    shares lend each other room."""
+    rng = np.random.default_rng(8)
+    n = 300_000
+    x, y = rng.random(n) * 300.0, rng.random(n) * 300.0
+    if place == "sort tiles":  # every 64th of 2048 points, whose share is the same
+        m = (np.arange(n) // 2048) % 64 == 5
+        x[m] = np.floor(x[m])
+    else:
+        m = rng.random(n) < 0.03
+        x[m], y[m] = 100.0 + np.floor(rng.random(m.sum()) * 3.0), 140.0 + rng.random(m.sum()) * 3.0
+    x[:2], y[:2] = (0.0, 300.0), (0.0, 300.0)
+    c, p = (x, y, np.round(rng.normal(50.0, 3.0, n), 1)), (5, 20, 0.8)
+    for mode in (0, 1):
+        taken, flags, got = chain(exe, [c], [p], mode=mode)
+        assert taken and flags == 0 and np.array_equal(got[0], oracle(c, p))
+
+
+def test_longest_lists(exe):
+    """More listed points in one bucket than a window block takes: handed on."""
+    rng = np.random.default_rng(9)
+    n = 1_900_000
+    x, y = rng.random(n) * 500.0, rng.random(n) * 500.0
+    m = rng.random(n) < 0.2
+    x[m], y[m] = 100.0, 140.0 + rng.random(m.sum())
+    x[:2], y[:2] = (0.0, 500.0), (0.0, 500.0)
+    taken, flags, _ = chain(exe, [(x, y, np.round(rng.normal(50.0, 3.0, n), 1))], [(10, 20, 0.8)])
+    assert not taken and flags & 32
