@@ -164,11 +164,12 @@ __global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_par
     uint32_t *sW = sPool + PTS;                  // exact key of a slot near an edge
     __shared__ uint32_t s_t, s_n, s_nr, s_base, s_stop, s_w[GP_NT / 64];
     const uint32_t tid = threadIdx.x, u = blockIdx.x;
-    if (tid == 0) {
+    if (tid == 0)
         s_n = s_nr = 0;
-        // (other workgroups may set it meanwhile: one thread reads it for all)
+    // (other workgroups may set it meanwhile: one thread reads it for all, the last,
+    // which has no part in finding the tile of most launches)
+    if (tid == GP_NT - 1)
         s_stop = load_past_caches(G.err, GRID_STOP_PART);
-    }
     const uint32_t t = find_entry(G.st_off, 0, G.ntiles, u, &s_t);
     if (s_stop)
         return;
