@@ -462,10 +462,8 @@ static owm_status exec_plan(owm_ctx *ctx, const GridPlan &P, const GridIo &io, c
     std::vector<uint8_t> key;
     if (graph || (flags & B_AUTO_GRAPH))
         plan_key(ctx, src, P, io, key);
-    if (!graph && (flags & B_AUTO_GRAPH)) {
-        graph = !ctx->prof.on && key == ctx->graphs.last_key;
-        ctx->graphs.last_key = key;
-    }
+    if (!graph && (flags & B_AUTO_GRAPH))
+        graph = ctx->graphs.last_grid.repeats(key) && !ctx->prof.on;
     GridDev G{};
     if (src.tree) {
         G.xy = src.tree->pts.xy;

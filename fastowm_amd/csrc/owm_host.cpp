@@ -1272,7 +1272,8 @@ void GraphCache::clear()
         if (s.exec)
             (void)hipGraphExecDestroy(s.exec);
     slots.clear();
-    last_key.clear();
+    last_grid.key.clear();
+    last_tree.key.clear();
 }
 
 // Enqueues a chain (body), or replays it from the graph captured for its key.
@@ -1411,8 +1412,7 @@ owm_status run_batch(owm_ctx *ctx, const double *dx, const double *dy, const dou
             // graph, captured on the first repeat; phase timing keeps it eager
             std::vector<uint8_t> key;
             graph_key(ctx, dx, dy, dz, P, key);
-            graph = !ctx->prof.on && key == ctx->graphs.last_key;
-            ctx->graphs.last_key.swap(key);
+            graph = ctx->graphs.last_tree.repeats(key) && !ctx->prof.on;
         }
         Arena &A = ctx->arena;
         uint32_t *guard = (uint32_t *)A.take(256);

@@ -311,7 +311,17 @@ struct GraphCache {
         uint64_t used_after = 0;  // arena offset after the chain's allocations
     };
     std::vector<Slot> slots;
-    std::vector<uint8_t> last_key;  // key of the last auto-graph call (repeat detection)
+    // Whether a chain's key is that of its last auto-graph call.  A call that the column
+    // grid hands on runs both chains, so each has a last key of its own.
+    struct Last {
+        std::vector<uint8_t> key;
+        bool repeats(const std::vector<uint8_t> &k)
+        {
+            const bool same = k == key;
+            key = k;
+            return same;
+        }
+    } last_grid, last_tree;
     void clear();
     ~GraphCache();
 };

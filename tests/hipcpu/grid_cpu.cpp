@@ -3,11 +3,13 @@
 //   grid_cpu IN OUT
 // IN: doubles {mode, poke, calls, tiles, then per tile {n, wsize, bsize,
 // overlap, has box, box[4]}}, then x, y, z.  Modes: 0 a whole run, 1 the seeds and
-// 2 the minima of a resident tree (one tile, its points in reverse).  poke: 1, every
+// 2 the minima of a resident tree (one tile, its points in reverse); 3 whole runs that
+// may replay, each followed by the tree chain's look at its own key.  poke: 1, every
 // workgroup of k_grid_heavy finds GRID_ERR_POOL set by another one of the launch
 // before its wave 4 first runs; 2, the queue of heavy stretches holds two.
 // OUT: int64 {status, taken, flags, count, stray marks, barriers passed by launches that
-// began after the flag was raised, by k_grid_part, its workgroups}, tile ranges (tiles
+// began after the flag was raised, by k_grid_part, its workgroups, replays of the chain,
+// calls in which the tree chain's key repeats}, tile ranges (tiles
 // + 1 of them), ids.
 #include "../../fastowm_amd/csrc/owm_host.h"
 #include <math.h>
@@ -110,7 +112,7 @@ int main(int argc, char **argv)
     hipcpu::stale.assign((const unsigned char *)&low, (const unsigned char *)(&low + 1));
     owm_ctx *ctx = new owm_ctx;
     uint32_t *err = nullptr;
-    int64_t after = 0, part = 0, groups = 0, mark = 0, kind = 0;
+    int64_t after = 0, part = 0, groups = 0, mark = 0, kind = 0, repeats = 0;
     auto count_barriers = [&]() {
         (kind == 1 ? after : part) += kind ? hipcpu::barriers - mark : 0;
         mark = hipcpu::barriers;
@@ -145,10 +147,13 @@ int main(int argc, char **argv)
     int64_t status = 0;
     uint64_t count = 0;
     for (int k = 0; k < calls; ++k) {
-        if (mode == 0) {
+        if (mode == 0 || mode == 3) {
             std::vector<owm_tile> boxed;
-            status = run_grid(ctx, x, y, z, tiles.data(), T, 0, ids.data(), ids.size(), off.data(), boxed, taken);
+            status = run_grid(ctx, x, y, z, tiles.data(), T, mode ? B_AUTO_GRAPH : 0, ids.data(), ids.size(),
+                              off.data(), boxed, taken);
             count = off[T];
+            if (mode)
+                repeats += ctx->graphs.last_tree.repeats({'t', 'r', 'e', 'e'});
             continue;
         }
         owm_tree tree;
@@ -175,8 +180,9 @@ int main(int argc, char **argv)
         count = 0;
     FILE *o = fopen(argv[2], "wb");
     count_barriers();
-    const int64_t head_out[8] = {status, taken, err ? *err : 0, (int64_t)count, stray, after, part, groups};
-    fwrite(head_out, 8, 8, o);
+    const int64_t head_out[10] = {status, taken, err ? *err : 0, (int64_t)count, stray, after, part, groups,
+                                  (int64_t)hipcpu::graph_launches, repeats};
+    fwrite(head_out, 8, 10, o);
     fwrite(off.data(), 8, T + 1, o);
     fwrite(ids.data(), 4, count, o);
     fclose(o);

@@ -147,6 +147,7 @@ struct Graph {
     std::vector<std::function<void()>> nodes;
 };
 inline Graph *capture = nullptr;
+inline uint64_t graph_launches = 0;
 
 template <class T, class... A> const void *first_of(const T &t, const A &...) { return &t; }
 
@@ -315,6 +316,7 @@ inline hipError_t hipGraphDestroy(hipGraph_t g) { delete g; return hipSuccess; }
 inline hipError_t hipGraphExecDestroy(hipGraphExec_t g) { delete g; return hipSuccess; }
 inline hipError_t hipGraphLaunch(hipGraphExec_t g, hipStream_t)
 {
+    ++hipcpu::graph_launches;
     for (auto &f : g->nodes)
         f();
     return hipSuccess;

@@ -3,6 +3,7 @@ tree chain, and calls that only just stay with it.  Which chain answered is read
 from the phases' launches; seeds are ids, against the oracle equal or wrong."""
 import numpy as np
 import pytest
+import torch
 
 import pyoracle as O
 from fastowm_amd import owm, synth
@@ -117,3 +118,17 @@ def test_longest_lists(ctx):
     want = ctx.run_tile(*c, 10, 20, 0.8, 32)
     got, calls = profiled(ctx, lambda: ctx.run_tile(*c, 10, 20, 0.8))
     assert calls["sort_tree_pass"] > 0 and np.array_equal(got, want)
+
+
+def test_handed_on_calls_replay(ctx):
+    """A repeated call on device memory, handed on each time: its chains are replayed from
+    the third call on; other calls lie between."""
+    say("grid limits, replays of calls handed on")
+    c, p = raster(450, 512_000.0), (5, 20, 0.8)
+    d = [torch.from_numpy(a).cuda() for a in c]
+    e = [torch.from_numpy(a).cuda() for a in raster(450, 512_000.0, seed=1)]
+    wants = [O.run(*c, *p, 32)[0], O.run(*raster(450, 512_000.0, seed=1), *p, 32)[0]]
+    for k in (0, 0, 0, 0, 1, 0, 1, 1, 1, 0):
+        assert np.array_equal(ctx.run_tile(*(d, e)[k], *p), wants[k])
+    d[2].copy_(e[2])  # the same memory, other heights
+    assert np.array_equal(ctx.run_tile(*d, *p), wants[1])

@@ -48,11 +48,11 @@ def chain(exe, clouds, params, mode=0, poke=0, calls=1, boxes=None):
     r = subprocess.run([exe, *paths], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, (r.returncode, r.stderr)
     with open(paths[1], "rb") as f:
-        status, taken, flags, count, stray, *work = np.fromfile(f, np.int64, 8)
+        status, taken, flags, count, stray, *work = np.fromfile(f, np.int64, 10)
         off = np.fromfile(f, np.int64, len(clouds) + 1)
         ids = np.fromfile(f, np.uint32, count)
     assert status == 0 and stray == 0
-    chain.after, chain.part, chain.groups = work
+    chain.after, chain.part, chain.groups, chain.replays, chain.repeats = work
     return bool(taken), int(flags), [ids[a:b] for a, b in zip(off, off[1:])] if taken else None
 
 
@@ -201,3 +201,9 @@ def test_longest_lists(exe):
     x[:2], y[:2] = (0.0, 500.0), (0.0, 500.0)
     taken, flags, _ = chain(exe, [(x, y, np.round(rng.normal(50.0, 3.0, n), 1))], [(10, 20, 0.8)])
     assert not taken and flags & 32
+
+
+def test_handed_on_calls_replay(exe):
+    """A repeated call that the chain hands on: both chains find their last key again."""
+    taken, _, _ = chain(exe, [raster(450)], [(5, 20, 0.8)], mode=3, calls=4)
+    assert not taken and chain.replays == 3 and chain.repeats == 3
