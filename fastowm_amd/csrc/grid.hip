@@ -232,11 +232,12 @@ __global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_par
             // their ranges go to the pool (counted again: few points take this)
             __syncthreads();
             if (tid == 0) {
-                // (a share asked for more than it has left is closed, and the next one
-                // asked: points on edges may lie in few sort tiles)
+                // (a share asked for more than it has left is closed, and some others are
+                // asked: points on edges may lie in few sort tiles; 64 tries in a row
+                // kept the last sort tiles of a full pool 25 us)
                 s_base = OWM_NONE;
-                for (uint32_t k = 0; k < GRID_POOLS && s_base == OWM_NONE; ++k) {
-                    const uint32_t share = (u + k) & (GRID_POOLS - 1u);
+                for (uint32_t k = 0; k < 8 && s_base == OWM_NONE; ++k) {
+                    const uint32_t share = (u + 9 * k) & (GRID_POOLS - 1u);
                     const uint32_t at = atomicAdd(G.pool_used + share * 32, nr);
                     s_base = at + nr <= G.pool_cap ? share * G.pool_cap + at : OWM_NONE;
                 }
