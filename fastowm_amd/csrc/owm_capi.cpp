@@ -210,7 +210,7 @@ owm_status upload_cloud(owm_ctx *ctx, const double *x, const double *y, const do
             return OWM_E_BUDGET;
         }
         (void)hipStreamSynchronize(ctx->stream);
-        hipError_t e = ctx->upload.reserve(3 * b, ctx->room_for(ctx->upload));
+        hipError_t e = ctx->grow(ctx->upload, 3 * b, ctx->room_for(ctx->upload));
         if (e != hipSuccess)
             return hip_fail(ctx, e, "upload buffer");
     }
@@ -378,12 +378,7 @@ owm_status owm_tree_build(owm_ctx *ctx, const double *x, const double *y, const 
             set_err(ctx, "tree needs %llu device bytes over the budget", (unsigned long long)tb);
             return OWM_E_BUDGET;
         }
-        e = tr->mem.reserve(tb, tb);
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            ctx->release_spare();
-            e = tr->mem.reserve(tb, tb);
-        }
+        e = ctx->grow(tr->mem, tb, tb);
         if (e != hipSuccess)
             return hip_fail(ctx, e, "tree allocation");
     }

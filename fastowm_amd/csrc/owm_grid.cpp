@@ -275,7 +275,7 @@ static owm_status take_few_boxes(owm_ctx *ctx, const double *dx, const double *d
 {
     hipStream_t s = ctx->stream;
     if (!ctx->box_work.ptr) {
-        HIP_TRY(ctx->box_work.reserve(box_work_bytes()), "box work");
+        HIP_TRY(ctx->grow(ctx->box_work, box_work_bytes()), "box work");
         launch_fill_u32(s, (uint32_t *)ctx->box_work.ptr, BOX_TILES, 0u);
     }
     BoxArgs a{};

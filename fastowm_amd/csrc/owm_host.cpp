@@ -859,12 +859,7 @@ owm_status Arena::ensure(owm_ctx *ctx, uint64_t bytes)
     hipError_t e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess)
         return hip_fail(ctx, e, "sync before arena growth");
-    e = buf.reserve(bytes, ctx->room_for(buf));
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        ctx->release_spare();
-        e = buf.reserve(bytes, ctx->room_for(buf));
-    }
+    e = ctx->grow(buf, bytes, ctx->room_for(buf));
     if (this == &ctx->arena)
         ctx->graphs.clear();  // captured chains point into the old arena
     if (e != hipSuccess)
@@ -1190,7 +1185,7 @@ owm_status ensure_s1_list(owm_ctx *ctx, uint64_t cap)
         return OWM_E_BUDGET;
     }
     HIP_TRY(hipStreamSynchronize(ctx->stream), "sync before list growth");
-    HIP_TRY(ctx->s1_list.reserve(cap * 4, ctx->room_for(ctx->s1_list)), "stage-1 join list");
+    HIP_TRY(ctx->grow(ctx->s1_list, cap * 4, ctx->room_for(ctx->s1_list)), "stage-1 join list");
     return OWM_OK;
 }
 
@@ -1589,6 +1584,18 @@ void owm_ctx::release_spare()
 {
     std::lock_guard<std::mutex> g(spare_mu);
     spare.release();
+}
+
+hipError_t owm_ctx::grow(owm::DevBuf &b, uint64_t need, uint64_t cap)
+{
+    hipError_t e = b.reserve(need, cap);
+    if (e != hipErrorOutOfMemory || b.borrowed)
+        return e;
+    (void)hipGetLastError();
+    release_spare();
+    if (owner)
+        owner->release_spare();
+    return b.reserve(need, cap);
 }
 
 bool owm_ctx::exceeds(uint64_t need, const owm::DevBuf *old)

@@ -35,8 +35,12 @@ struct DevBuf {
         std::swap(bytes, o.bytes);
         std::swap(borrowed, o.borrowed);
     }
-    // Grows to at least `need` bytes (with 25% headroom, never above `cap`).
-    hipError_t reserve(uint64_t need, uint64_t cap = ~0ull);
+
+private:
+    // Grows to at least `need` bytes (with 25% headroom, never above `cap`).  Callers
+    // go through owm_ctx::grow, which gives kept memory back where this fails.
+    hipError_t reserve(uint64_t need, uint64_t cap);
+    friend struct ::owm_ctx;
 };
 
 // Bump allocator over one device buffer, reset at the start of every run.
@@ -345,12 +349,17 @@ struct owm_ctx {
     uint64_t s1_need_max = 0;  // largest join that overflowed its first estimate
     // The last freed tree's device memory, kept for the next build (allocating and
     // freeing 130 MB takes 0.37 ms, a third of a 3M-point tree's use): at most
-    // SPARE_MAX bytes, counted as held, given back when the budget or an
-    // allocation needs them, and with the context.  Trees are freed from any thread.
+    // SPARE_MAX bytes, counted as held, given back when the budget (exceeds) or an
+    // allocation (grow) needs them, when serving starts, and with the context.  Trees are
+    // freed from any thread.
     static constexpr uint64_t SPARE_MAX = 512ull << 20;
     std::mutex spare_mu;
     owm::DevBuf spare;
+    owm_ctx *owner = nullptr;  // serving slots: the context whose spare they may claim
     void release_spare();
+    // Grows a buffer of this context; out of memory, the spare (the owner's too) is
+    // given back and the allocation tried again.
+    hipError_t grow(owm::DevBuf &b, uint64_t need, uint64_t cap = ~0ull);
     // Whether `need` bytes more (with `old` released) exceed the budget.
     bool exceeds(uint64_t need, const owm::DevBuf *old = nullptr);
     owm::Tuner tuner;

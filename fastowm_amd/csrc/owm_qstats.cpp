@@ -91,7 +91,7 @@ owm_status owm_qtree_stats(owm_ctx *ctx, const double *x, const double *y, uint6
                         (unsigned long long)total);
                 return OWM_E_BUDGET;
             }
-            HIP_TRY(ctx->qs_work.reserve(total, ctx->room_for(ctx->qs_work)), "statistics buffer");
+            HIP_TRY(ctx->grow(ctx->qs_work, total, ctx->room_for(ctx->qs_work)), "statistics buffer");
         }
         uint8_t *w = (uint8_t *)ctx->qs_work.ptr;
         auto take = [&w](uint64_t b) { uint8_t *r = w; w += b; return r; };

@@ -122,7 +122,7 @@ static void run_group(ServeState *S, owm_ctx *slot, std::vector<std::shared_ptr<
             st = OWM_E_BUDGET;
         } else {
             (void)hipStreamSynchronize(slot->stream);
-            hipError_t e = slot->upload.reserve(3 * b, slot->room_for(slot->upload));
+            hipError_t e = slot->grow(slot->upload, 3 * b, slot->room_for(slot->upload));
             if (e != hipSuccess)
                 st = hip_fail(slot, e, "serving upload buffer");
         }
@@ -364,6 +364,7 @@ owm_status owm_serve_start(owm_ctx *ctx, uint32_t max_inflight, uint32_t max_bat
         ServeState *S = new ServeState();
         S->owner = ctx;
         S->max_batch = max_batch_tiles ? max_batch_tiles : 64;
+        ctx->release_spare();  // (the slots' share of the budget)
         uint64_t held = ctx->held_bytes();
         uint64_t avail = ctx->budget > held ? ctx->budget - held : 0;
         S->tree_budget = avail / 4;
@@ -379,6 +380,7 @@ owm_status owm_serve_start(owm_ctx *ctx, uint32_t max_inflight, uint32_t max_bat
                 return st;
             }
             slot->tuner = ctx->tuner;
+            slot->owner = ctx;
             S->slots.push_back(slot);
         }
         ctx->serve = S;

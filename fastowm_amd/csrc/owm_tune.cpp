@@ -168,7 +168,7 @@ owm_status owm_autotune(owm_ctx *ctx, const double *x, const double *y, const do
             if (ctx->exceeds(3 * b))
                 continue;  // no room for a trial copy: keep the default
             HIP_TRY(hipStreamSynchronize(ctx->stream), "tune sync");
-            HIP_TRY(sub.reserve(3 * b), "tune buffer");
+            HIP_TRY(ctx->grow(sub, 3 * b), "tune buffer");
             double *sx = (double *)sub.ptr, *sy = (double *)((uint8_t *)sub.ptr + b),
                    *sz = (double *)((uint8_t *)sub.ptr + 2 * b);
             std::vector<owm_tile> st_tiles;

@@ -91,7 +91,7 @@ owm_status owm_xyz_parse(owm_ctx *ctx, const char *text, uint64_t bytes, owm_clo
         // text | chunk counts | chunk offsets | counters
         const uint64_t w_text = al256(padded), w_cnt = al256(nch * 4), w_off = al256((nch + 1) * 8);
         HIP_TRY(hipStreamSynchronize(s), "sync before the reader");
-        HIP_TRY(ctx->xyz_text.reserve(w_text + w_cnt + w_off + 256, ctx->room_for(ctx->xyz_text)),
+        HIP_TRY(ctx->grow(ctx->xyz_text, w_text + w_cnt + w_off + 256, ctx->room_for(ctx->xyz_text)),
                 "reader text buffer");
         uint8_t *dt = (uint8_t *)ctx->xyz_text.ptr;
         uint32_t *cnt = (uint32_t *)(dt + w_text);
@@ -122,7 +122,7 @@ owm_status owm_xyz_parse(owm_ctx *ctx, const char *text, uint64_t bytes, owm_clo
         const uint64_t w_nl = al256(std::max<uint64_t>(nnl, 1) * 8);
         const uint64_t w_xyz = al256(std::max<uint64_t>(nlines, 1) * 8);
         const uint64_t w_list = al256((uint64_t)cap * 8);
-        HIP_TRY(ctx->xyz_work.reserve(w_nl + 3 * w_xyz + 3 * w_list, ctx->room_for(ctx->xyz_work)),
+        HIP_TRY(ctx->grow(ctx->xyz_work, w_nl + 3 * w_xyz + 3 * w_list, ctx->room_for(ctx->xyz_work)),
                 "reader work buffer");
         uint8_t *dw = (uint8_t *)ctx->xyz_work.ptr;
         uint64_t *nlpos = (uint64_t *)dw;
@@ -182,7 +182,7 @@ owm_status owm_xyz_parse(owm_ctx *ctx, const char *text, uint64_t bytes, owm_clo
         if (!hl.empty()) {
             DevBuf tmp;
             const uint64_t m = hl.size();
-            HIP_TRY(tmp.reserve(al256(m * 8) + m * 24, al256(m * 8) + m * 24), "host values");
+            HIP_TRY(ctx->grow(tmp, al256(m * 8) + m * 24, al256(m * 8) + m * 24), "host values");
             uint64_t *dl = (uint64_t *)tmp.ptr;
             double *dv = (double *)((uint8_t *)tmp.ptr + al256(m * 8));
             HIP_TRY(hipMemcpyAsync(dl, hl.data(), m * 8, hipMemcpyHostToDevice, s), "host values");
@@ -213,8 +213,8 @@ owm_status owm_xyz_parse(owm_ctx *ctx, const char *text, uint64_t bytes, owm_clo
             }
             std::sort(bl.begin(), bl.end());
             const uint64_t w_c = al256(std::max<uint64_t>(nlines, 1) * 8);
-            HIP_TRY(ctx->xyz_cloud.reserve(3 * w_c + al256(bl.size() * 8),
-                                           ctx->room_for(ctx->xyz_cloud)),
+            HIP_TRY(ctx->grow(ctx->xyz_cloud, 3 * w_c + al256(bl.size() * 8),
+                              ctx->room_for(ctx->xyz_cloud)),
                     "reader cloud");
             uint8_t *dc = (uint8_t *)ctx->xyz_cloud.ptr;
             uint64_t *dbl = (uint64_t *)(dc + 3 * w_c);

@@ -348,6 +348,8 @@ owm_status owm_autotune_stats(owm_ctx *ctx, const double *x, const double *y, co
  * of parameter re-queries. */
 owm_status owm_tree_build(owm_ctx *ctx, const double *x, const double *y, const double *z,
                           uint64_t n, int device_ptrs, uint32_t leaf_size, owm_tree **out);
+/* The context keeps the device memory of its last freed tree (up to 512 MB) for the
+ * next build, until another of its buffers, or one of its serving slots, finds no room. */
 void owm_tree_free(owm_tree *tree);
 uint64_t owm_tree_points(const owm_tree *tree);
 /* Tree statistics for checks: counts of leaves and internal nodes, the root's
