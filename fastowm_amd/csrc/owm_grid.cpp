@@ -416,8 +416,8 @@ static void plan_key(owm_ctx *ctx, const GridSrc &src, const GridPlan &P, const 
 }
 
 // Runs the planned chain; its results are in io (and qo) when it comes back.  Not
-// taken: it might not fit the budget where the tree chain would, or too many points
-// lie on edges.
+// taken: it might not fit the budget where the tree chain would, there is no memory, or
+// too many points lie on edges.
 static owm_status exec_plan(owm_ctx *ctx, const GridPlan &P, const GridIo &io, const GridSrc &src,
                             uint32_t flags, QueryOut &qo, bool &taken)
 {
@@ -442,6 +442,8 @@ static owm_status exec_plan(owm_ctx *ctx, const GridPlan &P, const GridIo &io, c
         return OWM_OK;
     void *old_arena = ctx->arena.buf.ptr;
     owm_status st = ctx->arena.ensure(ctx, need);
+    if (st == OWM_E_NOMEM)
+        return OWM_OK;  // the tree chain may fit
     if (st != OWM_OK)
         return st;
     if (ctx->arena.buf.ptr != old_arena)

@@ -6,7 +6,8 @@
 // 2 the minima of a resident tree (one tile, its points in reverse); 3 whole runs that
 // may replay, each followed by the tree chain's look at its own key.  poke: 1, every
 // workgroup of k_grid_heavy finds GRID_ERR_POOL set by another one of the launch
-// before its wave 4 first runs; 2, the queue of heavy stretches holds two.
+// before its wave 4 first runs; 2, the queue of heavy stretches holds two; 3, the device
+// has 2 MB.
 // OUT: int64 {status, taken, flags, count, stray marks, barriers passed by launches that
 // began after the flag was raised, by k_grid_part, its workgroups, replays of the chain,
 // calls in which the tree chain's key repeats}, tile ranges (tiles
@@ -110,6 +111,8 @@ int main(int argc, char **argv)
     low.id = 0x7FFFFFF0u;
     low.wx1 = low.wy1 = low.gx1 = low.gy1 = 0xFFFFu;
     hipcpu::stale.assign((const unsigned char *)&low, (const unsigned char *)(&low + 1));
+    if (head[1] == 3)
+        hipcpu::memory_left = 2 << 20;
     owm_ctx *ctx = new owm_ctx;
     uint32_t *err = nullptr;
     int64_t after = 0, part = 0, groups = 0, mark = 0, kind = 0, repeats = 0;

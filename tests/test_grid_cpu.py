@@ -207,3 +207,12 @@ def test_handed_on_calls_replay(exe):
     """A repeated call that the chain hands on: both chains find their last key again."""
     taken, _, _ = chain(exe, [raster(450)], [(5, 20, 0.8)], mode=3, calls=4)
     assert not taken and chain.replays == 3 and chain.repeats == 3
+
+
+def test_no_memory_for_the_chain(exe):
+    """The tree chain's memory is not this chain's: without room for its scratch the
+    call is handed on, not refused."""
+    t = synth.scaled(synth.config_c1(seed=3), 9_001).generate()
+    for mode in (0, 1, 2):
+        taken, _, _ = chain(exe, [t], [(10, 20, 0.8)], mode=mode, poke=3)
+        assert not taken
