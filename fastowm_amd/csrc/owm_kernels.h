@@ -88,6 +88,15 @@ struct BoxArgs {
     uint32_t ntiles;
     uint32_t pt[BOX_TILES + 1], blk[BOX_TILES + 1];
 };
+// Points [c0, c1) of workgroup k of a tile's nb (1 or more), in whole rounds of 2048.
+// n is up to 2^32 - 2: 32-bit sums wrap near that.
+OWM_HD void box_share(uint32_t n, uint32_t nb, uint32_t k, uint32_t &c0, uint32_t &c1)
+{
+    const uint64_t per = (((uint64_t)n + nb - 1) / nb + 2047) / 2048 * 2048;
+    const uint64_t a = k * per, b = a + per;
+    c0 = a < n ? (uint32_t)a : n;
+    c1 = b < n ? (uint32_t)b : n;
+}
 uint64_t box_work_bytes();
 void launch_boxes(hipStream_t s, const BoxArgs &a, const double *x, const double *y, void *work,
                   double *box);

@@ -201,16 +201,19 @@ __global__ __launch_bounds__(TB) void k_boxes(BoxArgs A, const double *__restric
     __syncthreads();
     const uint32_t t = __builtin_amdgcn_readfirstlane(s_t);
     const uint32_t b0 = A.blk[t], nb = A.blk[t + 1] - b0, p0 = A.pt[t], n = A.pt[t + 1] - p0;
-    const uint32_t per = ((n + nb - 1) / nb + 8 * TB - 1) / (8 * TB) * (8 * TB);
-    const uint32_t c0 = min((b - b0) * per, n), c1 = min(c0 + per, n);
+    uint32_t c0, c1;
+    static_assert(8 * TB == 2048, "box_share's rounds");
+    box_share(n, nb, b - b0, c0, c1);
+    const double *px = X + p0 + c0, *py = Y + p0 + c0;
+    const uint32_t m = c1 - c0;  // (far below 2^32: the rounds' indices do not wrap)
     double mnx = INFINITY, mny = INFINITY, mxx = -INFINITY, mxy = -INFINITY;
-    for (uint32_t base = c0 + tid; base < c1; base += 8 * TB) {
+    for (uint32_t base = tid; base < m; base += 8 * TB) {
         double xv[8], yv[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const uint32_t i = base + k * TB;
-            xv[k] = i < c1 ? X[p0 + i] : NAN;
-            yv[k] = i < c1 ? Y[p0 + i] : NAN;
+            xv[k] = i < m ? px[i] : NAN;
+            yv[k] = i < m ? py[i] : NAN;
         }
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
