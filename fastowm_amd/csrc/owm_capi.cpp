@@ -1,5 +1,6 @@
 // C ABI entry points (include/owm.h).  Each catches every C++ exception and
 // returns a status; none exits the process.
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <new>
@@ -650,6 +651,23 @@ owm_status owm_stage1(owm_ctx *ctx, owm_tree *tree, const owm_params *params, ui
     GUARD_END(ctx)
 }
 
+// First of the ids that is neither below n nor OWM_NONE; n_ids: none.  Block by block
+// without branches: with them stage 2 of 125,000 windows took 122 or 148 us, as the loop
+// happened to lie in the library; 96 like this.
+static uint64_t first_bad_id(const uint32_t *ids, uint64_t n_ids, uint32_t n)
+{
+    for (uint64_t b = 0; b < n_ids; b += 4096) {
+        const uint64_t end = std::min<uint64_t>(b + 4096, n_ids);
+        uint32_t bad = 0;
+        for (uint64_t i = b; i < end; ++i)
+            bad |= ids[i] + 1u > n ? 1u : 0u;  // (OWM_NONE + 1 is 0)
+        for (uint64_t i = b; bad && i < end; ++i)
+            if (ids[i] + 1u > n)
+                return i;
+    }
+    return n_ids;
+}
+
 owm_status owm_stage2(owm_ctx *ctx, owm_tree *tree, const owm_params *params,
                       const uint32_t *min_ids, uint64_t n_ids, uint32_t *llp, uint64_t cap,
                       uint64_t *n_llp)
@@ -659,11 +677,11 @@ owm_status owm_stage2(owm_ctx *ctx, owm_tree *tree, const owm_params *params,
         return OWM_E_ARG;
     GUARD_BEGIN
     (void)hipSetDevice(ctx->device);
-    for (uint64_t i = 0; i < n_ids; ++i)
-        if (min_ids[i] != OWM_NONE && min_ids[i] >= tree->n) {
-            set_err(ctx, "min_ids[%llu] = %u is not a point index", (unsigned long long)i, min_ids[i]);
-            return OWM_E_ARG;
-        }
+    const uint64_t bad = first_bad_id(min_ids, n_ids, (uint32_t)tree->n);
+    if (bad < n_ids) {
+        set_err(ctx, "min_ids[%llu] = %u is not a point index", (unsigned long long)bad, min_ids[bad]);
+        return OWM_E_ARG;
+    }
     Prepared P;
     QueryOut qo;
     uint32_t hc[16];

@@ -132,3 +132,19 @@ def test_handed_on_calls_replay(ctx):
         assert np.array_equal(ctx.run_tile(*(d, e)[k], *p), wants[k])
     d[2].copy_(e[2])  # the same memory, other heights
     assert np.array_equal(ctx.run_tile(*d, *p), wants[1])
+
+
+@pytest.mark.parametrize("at", [0, 1, 4095, 4096, 8190, 8191])
+def test_first_bad_id(ctx, at):
+    """Ids that stage 2 refuses, by their place in the list; OWM_NONE is no such id."""
+    say("grid limits, bad id", at)
+    c = synth.scaled(synth.config_c1(seed=3), 5000).generate()
+    tree = ctx.parallel_qtree(*c)
+    ids = np.full(8192, owm.NONE, np.uint32)
+    ids[::3] = np.arange(len(ids[::3]))
+    ids[7] = 4999
+    ids[8191] = 0xFFFFFFFE if at < 8191 else owm.NONE
+    ids[at] = 5000
+    with pytest.raises(owm.OWMError, match=rf"min_ids\[{at}\] = 5000 "):
+        ctx.stage2(tree, ids, 10, 0.8)
+    tree.free()
