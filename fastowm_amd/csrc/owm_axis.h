@@ -231,3 +231,14 @@ inline void grid_axis(GridAxis &A)
     A.ncol = w + g + 1u;
     A.pad = 0;
 }
+
+// An upper bound on the columns under bw neighbouring windows, for axes whose tol is at
+// most 0.125 (rounding moves an edge by far less than a step).
+inline double axis_cols_of(const GridAxis &A, uint32_t bw)
+{
+    const double len = (bw - 1) * A.w.step + 2.0 * A.w.half;
+    double r = (len * A.w.inv + 1.0) * (A.w.pair ? 1.0 : 2.0);
+    if (A.g.n)
+        r += (len * A.g.inv + 1.0) * (A.g.pair ? 1.0 : 2.0);
+    return ceil(r) + 4.0;
+}

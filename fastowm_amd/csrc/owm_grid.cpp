@@ -71,6 +71,10 @@ static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64
         grid_edges(T.ax[a].w, init[a], D.displace, hd, nw[a], false, 64);
         grid_edges(T.ax[a].g, initg[a], P.bsize ? (double)P.bsize : 1.0, hb, ng[a], true, 1);
         grid_axis(T.ax[a]);
+        // coordinates so far from zero, in steps, that the arithmetic decides for few of
+        // the points (and that axis_cols_of would not bound, further out)
+        if (T.ax[a].w.tol > 0.125 || T.ax[a].g.tol > 0.125)
+            return false;
     }
     T.min_num_points = D.min_num_points;
     T.stage2_need = P.overlap != 0.0 ? 2u : 1u;
@@ -101,16 +105,6 @@ static bool plan_tile(GridTile &T, const owm_params &P, const Derived &D, uint64
     T.nb = T.nbx * T.nby;
     sort_tiles(T, lsp);
     return true;
-}
-
-// An upper bound on the columns under bw windows.
-static double cols_of(const GridAxis &A, uint32_t bw)
-{
-    const double len = (bw - 1) * A.w.step + 2.0 * A.w.half;
-    double r = (len * A.w.inv + 1.0) * (A.w.pair ? 1.0 : 2.0);
-    if (A.g.n)
-        r += (len * A.g.inv + 1.0) * (A.g.pair ? 1.0 : 2.0);
-    return std::ceil(r) + 4.0;
 }
 
 // An upper bound on the tree chain's device memory for the same call: a call
@@ -167,7 +161,7 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
         double cells;
         for (;; --T.lbw) {
             const uint32_t bw = 1u << T.lbw;
-            cells = cols_of(T.ax[1], bw) * std::max<double>(cols_of(T.ax[0], bw), bw);
+            cells = axis_cols_of(T.ax[1], bw) * std::max<double>(axis_cols_of(T.ax[0], bw), bw);
             if (cells <= 3072.0 || T.lbw == 3)
                 break;
         }

@@ -216,3 +216,13 @@ def test_no_memory_for_the_chain(exe):
     for mode in (0, 1, 2):
         taken, _, _ = chain(exe, [t], [(10, 20, 0.8)], mode=mode, poke=3)
         assert not taken
+
+
+@pytest.mark.parametrize("origin,ok", [(1e9, True), (1e15, False)])
+def test_far_coordinates(exe, origin, ok):
+    """Coordinates that a window step is lost in: the tree chain's from the start."""
+    rng = np.random.default_rng(2)
+    n = 3000
+    x, y = origin + np.floor(rng.random(n) * 320.0) / 4.0, origin + rng.random(n) * 70.0
+    taken, flags, _ = chain(exe, [(x, y, rng.normal(50.0, 3.0, n))], [(10, 20, 0.8)])
+    assert taken == ok and flags == 0 and (chain.groups > 0) == ok
