@@ -212,6 +212,8 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
         P.axis_off[t + 1] = P.axis_off[t] + T.ax[0].w.n + T.ax[1].w.n;
         P.max_nb = std::max(P.max_nb, T.nb);
     }
+    if (P.nwin >= (1ull << 31))
+        return false;  // the tree chain refuses it
     // heavy stretches: 256 of the whole launch's points, their share of the ends
     // of groups and of segments that are not full
     for (const GridTile &T : P.t) {

@@ -10,8 +10,8 @@
 // has 2 MB.
 // OUT: int64 {status, taken, flags, count, stray marks, barriers passed by launches that
 // began after the flag was raised, by k_grid_part, its workgroups, replays of the chain,
-// calls in which the tree chain's key repeats}, tile ranges (tiles
-// + 1 of them), ids.
+// calls in which the tree chain's key repeats, the largest allocation asked for}, tile
+// ranges (tiles + 1 of them), ids.
 #include "../../fastowm_amd/csrc/owm_host.h"
 #include <math.h>
 
@@ -183,9 +183,9 @@ int main(int argc, char **argv)
         count = 0;
     FILE *o = fopen(argv[2], "wb");
     count_barriers();
-    const int64_t head_out[10] = {status, taken, err ? *err : 0, (int64_t)count, stray, after, part, groups,
-                                  (int64_t)hipcpu::graph_launches, repeats};
-    fwrite(head_out, 8, 10, o);
+    const int64_t head_out[11] = {status, taken, err ? *err : 0, (int64_t)count, stray, after, part, groups,
+                                  (int64_t)hipcpu::graph_launches, repeats, (int64_t)hipcpu::largest};
+    fwrite(head_out, 8, 11, o);
     fwrite(off.data(), 8, T + 1, o);
     fwrite(ids.data(), 4, count, o);
     fclose(o);

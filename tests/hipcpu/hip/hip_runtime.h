@@ -175,6 +175,7 @@ void launch(void (*k)(P...), dim3 g, dim3 b, A... a)
 
 // bytes that further allocations may take (freed ones come back)
 inline uint64_t memory_left = ~0ull;
+inline uint64_t largest = 0;  // allocation asked for
 inline std::map<void *, uint64_t> sizes;
 // what device memory holds before it is written
 inline std::vector<unsigned char> stale{0xA5};
@@ -274,6 +275,7 @@ typedef hipcpu::Graph *hipGraphExec_t;
 inline hipError_t hipMalloc(void **p, uint64_t n)
 {
     *p = nullptr;
+    hipcpu::largest = n > hipcpu::largest ? n : hipcpu::largest;
     if (n > hipcpu::memory_left)
         return hipErrorOutOfMemory;
     *p = malloc(n);

@@ -48,11 +48,11 @@ def chain(exe, clouds, params, mode=0, poke=0, calls=1, boxes=None):
     r = subprocess.run([exe, *paths], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, (r.returncode, r.stderr)
     with open(paths[1], "rb") as f:
-        status, taken, flags, count, stray, *work = np.fromfile(f, np.int64, 10)
+        status, taken, flags, count, stray, *work = np.fromfile(f, np.int64, 11)
         off = np.fromfile(f, np.int64, len(clouds) + 1)
         ids = np.fromfile(f, np.uint32, count)
     assert status == 0 and stray == 0
-    chain.after, chain.part, chain.groups, chain.replays, chain.repeats = work
+    chain.after, chain.part, chain.groups, chain.replays, chain.repeats, chain.largest = work
     return bool(taken), int(flags), [ids[a:b] for a, b in zip(off, off[1:])] if taken else None
 
 
@@ -226,3 +226,13 @@ def test_far_coordinates(exe, origin, ok):
     x, y = origin + np.floor(rng.random(n) * 320.0) / 4.0, origin + rng.random(n) * 70.0
     taken, flags, _ = chain(exe, [(x, y, rng.normal(50.0, 3.0, n))], [(10, 20, 0.8)])
     assert taken == ok and flags == 0 and (chain.groups > 0) == ok
+
+
+@pytest.mark.parametrize("tiles,planned", [(31, True), (33, False)])
+def test_too_many_windows(exe, tiles, planned):
+    """A batch of 2^31 windows and more, which the tree chain refuses, is not this
+    chain's either (seen by the scratch it asks for; the device has 2 MB)."""
+    c = np.array([1.0, 40_000.0]), np.array([1.0, 40_000.0]), np.array([1.0, 2.0])
+    boxes = [(0.0, 40_900.0, 0.0, 40_900.0)] * tiles  # 8181 x 8181 windows
+    taken, _, _ = chain(exe, [c] * tiles, [(10, 0, 0.5)] * tiles, poke=3, boxes=boxes)
+    assert not taken and (chain.largest > 1 << 30) == planned
