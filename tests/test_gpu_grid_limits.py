@@ -148,3 +148,53 @@ def test_first_bad_id(ctx, at):
     with pytest.raises(owm.OWMError, match=rf"min_ids\[{at}\] = 5000 "):
         ctx.stage2(tree, ids, 10, 0.8)
     tree.free()
+
+
+def _clouds():
+    rng = np.random.default_rng(11)
+    plain = synth.scaled(synth.config_c2(seed=5), 150_000).generate()
+    yield "plain", plain, (10, 20, 0.8)
+    yield "cm", tuple(np.round(a, 2) for a in plain), (7, 13, 0.5)
+    yield "unpaired", plain, (12, 20, 0.7)
+    yield "no cells", plain, (8, 0, 0.0)
+    yield "one sort tile", tuple(a[:1023] for a in plain), (10, 20, 0.8)
+    x, y, z = (a.copy() for a in synth.scaled(synth.config_c2(seed=6), 700_000).generate())
+    yield "large sort tiles", (x, y, z), (10, 20, 0.8)
+    h = 400.0 * rng.random((2, 300_000))
+    h[:, :270_000] = 50.0 + 6.0 * rng.random((2, 270_000))
+    h[0, :5000] = np.round(h[0, :5000])
+    yield "heavy", (h[0], h[1], np.round(rng.normal(50.0, 2.0, 300_000), 1)), (10, 20, 0.8)
+
+
+@pytest.mark.parametrize("name,c,p", [pytest.param(*v, id=v[0]) for v in _clouds()])
+def test_grid_alone_answers(ctx, name, c, p):
+    """The column grid's own answer: nothing of the tree chain runs behind it, neither for
+    a whole run nor for a resident tree's queries."""
+    say("grid limits, grid alone", name)
+    want = O.run(*c, *p, 32)[0]
+    got, calls = profiled(ctx, lambda: ctx.run_tile(*c, *p))
+    assert calls["grid_partition"] == 1 and not calls["sort_tree_pass"] and not calls["stage1"]
+    assert np.array_equal(got, want)
+    tree = ctx.parallel_qtree(*c)
+    (minima, _), calls = profiled(ctx, lambda: ctx.stage1(tree, p[0], p[2], p[1]))
+    assert calls["grid_partition"] == 1 and not calls["stage1"] and not calls["stage1_join"]
+    assert np.array_equal(minima, O.Tree(*c, O.params(*p, synth.bbox(c[0], c[1]), len(c[0]), 32)).stage1())
+    got, calls = profiled(ctx, lambda: ctx.tree_run(tree, *p))
+    assert calls["grid_partition"] == 1 and not calls["stage1"] and np.array_equal(got, want)
+    tree.free()
+
+
+@pytest.mark.parametrize("shift,grid", [(0.0, False), (0.25, True)])
+def test_lattice_and_its_box(ctx, shift, grid):
+    """Points on a lattice of the windows' step: all on edges where the box starts on the
+    lattice, none where the points are shifted in the same box."""
+    say("grid limits, lattice", shift)
+    rng = np.random.default_rng(9)
+    n = 400_000
+    x, y = (rng.integers(1, 800, n) + shift for _ in range(2))
+    z = np.round(rng.normal(50.0, 3.0, n), 1)
+    box = (0.0, 801.0, 0.0, 801.0)
+    want = O.run(x, y, z, 5, 20, 0.8, 32, box)[0]
+    got, calls = profiled(ctx, lambda: ctx.run_tile(x, y, z, 5, 20, 0.8, bbox=box))
+    assert calls["grid_partition"] == 1 and (calls["sort_tree_pass"] == 0) == grid
+    assert np.array_equal(got, want) and len(want) > 1000
