@@ -7,7 +7,7 @@
 // may replay, each followed by the tree chain's look at its own key.  poke: 1, every
 // workgroup of k_grid_heavy finds GRID_ERR_POOL set by another one of the launch
 // before its wave 4 first runs; 2, the queue of heavy stretches holds two; 3, the device
-// has 2 MB.
+// has 2 MB; 4 and 5, a share of the lists holds 600 words (5: from k_grid_heavy on).
 // OUT: int64 {status, taken, flags, count, stray marks, barriers passed by launches that
 // began after the flag was raised, by k_grid_part, its workgroups, replays of the chain,
 // calls in which the tree chain's key repeats, the largest allocation asked for}, tile
@@ -134,6 +134,9 @@ int main(int argc, char **argv)
             }
         if (!kind && k != (const void *)&k_grid_prep && k != (const void *)&k_flags_out && *err)
             kind = 1;
+        const bool heavy = k == (const void *)&k_grid_heavy<512, false>;
+        if ((head[1] == 4 && k == (const void *)&k_grid_bin<512, 1, false>) || (head[1] >= 4 && heavy))
+            const_cast<GridDev *>((const GridDev *)arg)->list_cap = 600;
         if (head[1] == 2 && k == (const void *)&k_grid_bin<512, 1, false>)
             for (uint32_t t = 0; t < T; ++t)
                 const_cast<GridTile *>(((const GridDev *)arg)->tiles)[t].heavy_cap = 2;

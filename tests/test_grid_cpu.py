@@ -107,13 +107,15 @@ def test_raster_beside_a_plain_tile(exe, side, ok):
 
 
 def heavy_cloud(n=160_000, seed=5, on_edges=0):
-    """Most points in a few square metres."""
+    """Most points in a few square metres; about half of the first `on_edges` on the
+    edges of windows (the corner points place the box)."""
     rng = np.random.default_rng(seed)
     x, y = rng.random(n) * 400.0, rng.random(n) * 400.0
     k = int(n * 0.95)
     x[:k], y[:k] = 101.0 + rng.random(k) * 6.0, 203.0 + rng.random(k) * 6.0
     m = on_edges
     x[:m], y[:m] = np.round(x[:m]), np.round(y[:m])
+    x[-2:], y[-2:] = (0.0, 400.0), (0.0, 400.0)
     s = rng.permutation(n)
     return x[s], y[s], np.round(rng.normal(50.0, 2.0, n), 1)
 
@@ -236,3 +238,12 @@ def test_too_many_windows(exe, tiles, planned):
     boxes = [(0.0, 40_900.0, 0.0, 40_900.0)] * tiles  # 8181 x 8181 windows
     taken, _, _ = chain(exe, [c] * tiles, [(10, 0, 0.5)] * tiles, poke=3, boxes=boxes)
     assert not taken and (chain.largest > 1 << 30) == planned
+
+
+@pytest.mark.parametrize("poke", [4, 5])
+def test_full_lists(exe, poke):
+    """Shares of the lists that one block nearly fills, for the bins and for the heavy
+    stretches alone: handed on, and the launches behind do nothing."""
+    c, p = heavy_cloud(on_edges=100_000), (10, 20, 0.8)
+    taken, flags, _ = chain(exe, [c], [p], poke=poke)
+    assert not taken and flags & 32 and chain.after == 0
