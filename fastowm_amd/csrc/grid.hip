@@ -45,33 +45,6 @@ __device__ __forceinline__ uint32_t find_entry(const uint32_t *__restrict__ off,
     return __builtin_amdgcn_readfirstlane(*s_t);
 }
 
-// Exclusive scan over the workgroup (NT threads); total of all.
-template <int NT>
-__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t *s_w, uint32_t &total)
-{
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t inc = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(inc, o, 64);
-        if (lane >= (uint32_t)o)
-            inc += u;
-    }
-    if (lane == 63)
-        s_w[w] = inc;
-    __syncthreads();
-    uint32_t add = 0, tot = 0;
-#pragma unroll
-    for (int k = 0; k < NT / 64; ++k) {
-        const uint32_t u = s_w[k];
-        add += (uint32_t)k < w ? u : 0u;
-        tot += u;
-    }
-    __syncthreads();
-    total = tot;
-    return add + inc - v;
-}
-
 // Bucket and cell within it of a column and row.
 __device__ __forceinline__ uint32_t grid_key(const GridTile &T, uint32_t cx, uint32_t cy)
 {
@@ -302,7 +275,7 @@ __global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_par
     for (uint32_t b = b0; b < b1; ++b)
         sum += hist[b];
     uint32_t total;
-    uint32_t run = block_scan<GP_NT>(sum, s_w, total);
+    uint32_t run = owm_block_scan<GP_NT>(sum, s_w, total);
     uint16_t *tab = G.tab + T.tab_off + (uint64_t)st * (nb + 1);
     for (uint32_t b = b0; b < b1; ++b) {
         const uint32_t h = hist[b];
@@ -477,7 +450,7 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
         }
         const uint32_t nseg = (o1 - o0 + seg_pts - 1) / seg_pts;
         uint32_t total;
-        const uint32_t at0 = block_scan<NT>(nseg, s_w, total);
+        const uint32_t at0 = owm_block_scan<NT>(nseg, s_w, total);
         if (!SUB) {
             const uint32_t pts = __builtin_amdgcn_readfirstlane(total) * seg_pts;
             if (__builtin_expect(pts > left, 0)) {

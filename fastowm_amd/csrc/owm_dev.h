@@ -136,6 +136,34 @@ __device__ __forceinline__ uint32_t owm_find_tile(const uint32_t *off, uint32_t 
     return lo;
 }
 
+// Exclusive scan over the workgroup (NT threads, all of which call it; s_w: NT / 64 shared
+// words); total of all.
+template <int NT>
+__device__ __forceinline__ uint32_t owm_block_scan(uint32_t v, uint32_t *s_w, uint32_t &total)
+{
+    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(inc, o, 64);
+        if (lane >= (uint32_t)o)
+            inc += u;
+    }
+    if (lane == 63)
+        s_w[w] = inc;
+    __syncthreads();
+    uint32_t add = 0, tot = 0;
+#pragma unroll
+    for (int k = 0; k < NT / 64; ++k) {
+        const uint32_t u = s_w[k];
+        add += (uint32_t)k < w ? u : 0u;
+        tot += u;
+    }
+    __syncthreads();
+    total = tot;
+    return add + inc - v;
+}
+
 // Order-preserving 64-bit key of an eligible z (z < DBL_MAX): equal doubles
 // give equal keys (-0.0 is folded onto +0.0), so (key, index) order is the
 // reference's "lowest z, then lowest index" order.

@@ -386,30 +386,6 @@ __device__ __forceinline__ uint32_t qf_path(const QsPath &P, double x, double y)
     return k;
 }
 
-template <int NT>
-__device__ __forceinline__ uint32_t qf_scan(uint32_t v, uint32_t *s_w, uint32_t &total)
-{
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t inc = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(inc, o, 64);
-        if (lane >= (uint32_t)o)
-            inc += u;
-    }
-    if (lane == 63)
-        s_w[w] = inc;
-    __syncthreads();
-    uint32_t add = 0, tot = 0;
-    for (int k = 0; k < NT / 64; ++k) {
-        add += (uint32_t)k < w ? s_w[k] : 0u;
-        tot += s_w[k];
-    }
-    __syncthreads();
-    total = tot;
-    return add + inc - v;
-}
-
 __global__ __launch_bounds__(QP_NT) void k_qs_part(QsFast F)
 {
     extern __shared__ uint4 s_qp[];
@@ -461,7 +437,7 @@ __global__ __launch_bounds__(QP_NT) void k_qs_part(QsFast F)
         h[j] = hist[tid * PER + j];
         sum += h[j];
     }
-    uint32_t run = qf_scan<QP_NT>(sum, s_w, total);
+    uint32_t run = owm_block_scan<QP_NT>(sum, s_w, total);
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         hist[tid * PER + j] = run;
@@ -612,7 +588,7 @@ __global__ __launch_bounds__(QB_NT, 8) void k_qs_bins(QsFast F)
         s_hist[k] = 0;
     if (tid == 0)
         s_open = s_pts = s_nodes = 0;
-    qf_scan<QB_NT>(sum, s_w, total);
+    owm_block_scan<QB_NT>(sum, s_w, total);
     if (tid == 0)
         F.tot[bucket] = total;
     if (total > F.bucket_cap) {  // one workgroup would hold the call up

@@ -33,30 +33,6 @@ constexpr int CP_ITEMS = 16;
 constexpr int CP_TILE = CP_BLOCK * CP_ITEMS;
 constexpr uint32_t LB_AGG = 1u << 30, LB_INC = 2u << 30, LB_CNT = (1u << 30) - 1;
 
-__device__ __forceinline__ uint32_t block_excl_scan_cp(uint32_t v, uint32_t *s_tmp, uint32_t &total)
-{
-    uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    uint32_t inc = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        uint32_t u = __shfl_up(inc, o, 64);
-        if (lane >= (uint32_t)o)
-            inc += u;
-    }
-    if (lane == 63)
-        s_tmp[w] = inc;
-    __syncthreads();
-    uint32_t add = 0, tot = 0;
-    for (uint32_t k = 0; k < CP_BLOCK / 64; ++k) {
-        if (k < w)
-            add += s_tmp[k];
-        tot += s_tmp[k];
-    }
-    __syncthreads();
-    total = tot;
-    return add + inc - v;
-}
-
 // Decoupled look-back over compaction tiles taken in order (a tile's
 // predecessors are all held by running workgroups): publish this tile's
 // count, add the predecessors' counts back to the first inclusive prefix,
@@ -120,7 +96,7 @@ __global__ __launch_bounds__(CP_BLOCK) void k_compact_valid(const uint32_t *__re
             cnt += f;
         }
         uint32_t total;
-        uint32_t excl = block_excl_scan_cp(cnt, s_tmp, total);
+        uint32_t excl = owm_block_scan<CP_BLOCK>(cnt, s_tmp, total);
         if (threadIdx.x == 0) {
             const uint32_t prefix = tile_prefix(lookback, tile, total);
             s_prefix = prefix;
@@ -251,7 +227,7 @@ __global__ __launch_bounds__(CP_BLOCK) void k_bits_compact(const uint32_t *__res
             cnt += __popc(wv[k].x) + __popc(wv[k].y) + __popc(wv[k].z) + __popc(wv[k].w);
         }
         uint32_t total;
-        const uint32_t excl = block_excl_scan_cp(cnt, s_tmp, total);
+        const uint32_t excl = owm_block_scan<CP_BLOCK>(cnt, s_tmp, total);
         // the tiles of the batch whose points this tile of words holds, found while
         // the prefix is on its way
         const uint32_t p0 = tile * BC_TILE << 5, p1 = (tile + 1) * BC_TILE << 5;
