@@ -15,7 +15,7 @@
 //                   then y; windows' minima mark the point bitmaps of stage 2
 //   k_grid_cells    stage 3: the rectangle of each cell without an LLP
 // Against the tree chain (56 B a point moved by each sort pass, 32 B by the leaf
-// aggregates, about 35 B by stage 1 on window columns) a point moves 52 B after
+// aggregates, about 35 B by stage 1 on window columns) a point moves 48 B after
 // its box is known.  Measured on MI355X: 512 uneven tiles (329M points) 14.6 ->
 // 5.3 ms (partition 2.3, bins 1.0, windows 0.3 ms), a 120M-point tile 6.6 ->
 // 1.9 ms, 20M points with clusters 1.38 -> 0.43 ms, 1M points 0.32 -> 0.10 ms,
@@ -386,7 +386,7 @@ __device__ __forceinline__ void queue_rest(const GridDev &G, const GridTile &T, 
 
 // One workgroup per item: a bucket's runs in one share of the tile's sort tiles.
 // Cells keep the count, the lowest z key and the lowest index at that key.  A
-// round takes GB_SEG * TWO points per lane, without branches (a lane without a
+// round takes GB_SEG points per lane, without branches (a lane without a
 // point, or whose point has no column, works on one spare cell), so that the
 // round's LDS operations are in flight together: counts and key minima; after a
 // barrier the points that still hold their cell's minimum, of which those that
@@ -405,11 +405,10 @@ __device__ __forceinline__ void queue_rest(const GridDev &G, const GridTile &T, 
 // 5 m x 5 m: 64 -> 0.48 ms; density falling with the distance from a scanner:
 // 0.66 -> 0.29 ms; clouds without such shares pay the empty launch and the test
 // (20M points 100 -> 105 us, 120M 0.61 -> 0.64 ms).
-template <int NT, int TWO, bool TREE, bool SUB>
+template <int NT, bool TREE, bool SUB>
 __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t item,
                                           uint32_t cells, uint32_t st0, uint32_t st1, uint4 *out)
 {
-    constexpr int KK = GB_SEG * TWO;
     extern __shared__ unsigned long long s_bin[];
     unsigned long long *sZ = s_bin;                 // [cells + 64]
     uint32_t *sId = (uint32_t *)(sZ + cells + 64);  // [cells + 64]
@@ -467,42 +466,38 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
             }
             __syncthreads();
             const uint32_t here = min((uint32_t)GB_RUNS, total - p0);
-            for (uint32_t r0 = 0; r0 < here; r0 += ngrp * TWO) {
-                unsigned long long zk[KK], cur[KK];
-                uint32_t cw[KK], cell[KK], id0[TWO], all = 0;
+            for (uint32_t r0 = 0; r0 < here; r0 += ngrp) {
+                unsigned long long zk[GB_SEG], cur[GB_SEG];
+                uint32_t cw[GB_SEG], cell[GB_SEG], all = 0;
+                const uint2 run = r0 + grp < here ? sRun[r0 + grp] : make_uint2(0u, 0u);
+                const uint32_t id0 = pt_off + (run.x >> lsp << lsp);
+                RecWord w[3] = {};
+                if (first < run.y) {
+                    // four records in three loads (the last may hold the next
+                    // run's, or the padding behind the tile's)
+                    const RecWord *p =
+                        (const RecWord *)(G.rec + ((uint64_t)rec_off + run.x + first) * 3);
+                    w[0] = p[0];
+                    w[1] = p[1];
+                    w[2] = p[2];
+                }
+                const uint32_t v[12] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y,
+                                        w[1].z, w[1].w, w[2].x, w[2].y, w[2].z, w[2].w};
 #pragma unroll
-                for (int h = 0; h < TWO; ++h) {
-                    const uint32_t e = r0 + h * ngrp + grp;
-                    const uint2 run = e < here ? sRun[e] : make_uint2(0u, 0u);
-                    id0[h] = pt_off + (run.x >> lsp << lsp);
-                    RecWord w[3] = {};
-                    if (first < run.y) {
-                        // four records in three loads (the last may hold the next
-                        // run's, or the padding behind the tile's)
-                        const RecWord *p =
-                            (const RecWord *)(G.rec + ((uint64_t)rec_off + run.x + first) * 3);
-                        w[0] = p[0];
-                        w[1] = p[1];
-                        w[2] = p[2];
-                    }
-                    const uint32_t v[12] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y,
-                                            w[1].z, w[1].w, w[2].x, w[2].y, w[2].z, w[2].w};
-#pragma unroll
-                    for (int k = 0; k < GB_SEG; ++k) {
-                        zk[h * GB_SEG + k] = (unsigned long long)v[3 * k + 1] << 32 | v[3 * k];
-                        cw[h * GB_SEG + k] = first + k < run.y ? v[3 * k + 2] : KEY_NONE;
-                    }
+                for (int k = 0; k < GB_SEG; ++k) {
+                    zk[k] = (unsigned long long)v[3 * k + 1] << 32 | v[3 * k];
+                    cw[k] = first + k < run.y ? v[3 * k + 2] : KEY_NONE;
                 }
 #pragma unroll
-                for (int k = 0; k < KK; ++k) {
+                for (int k = 0; k < GB_SEG; ++k) {
                     cell[k] = min(cw[k] >> GRID_SLOT_BITS, spare);
                     all |= cw[k];
                     atomicAdd(&sCnt[cell[k]], 1u);
                     cur[k] = sZ[cell[k]];
                 }
-                bool low[KK], eq[KK];
+                bool low[GB_SEG], eq[GB_SEG];
 #pragma unroll
-                for (int k = 0; k < KK; ++k) {
+                for (int k = 0; k < GB_SEG; ++k) {
                     low[k] = zk[k] < cur[k];
                     if (low[k])
                         atomicMin(&sZ[cell[k]], zk[k]);
@@ -510,7 +505,7 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
                 uint32_t pend = 0;  // points without a column not listed: the list was full
                 if ((int32_t)all < 0) {
 #pragma unroll
-                    for (int k = 0; k < KK; ++k)
+                    for (int k = 0; k < GB_SEG; ++k)
                         if ((int32_t)cw[k] < 0) {
                             const uint32_t e = atomicAdd(&s_nr, 1u);
                             if (e < GB_RARE)
@@ -528,7 +523,7 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
                             s_nr = 0;
                         __syncthreads();
 #pragma unroll
-                        for (int k = 0; k < KK; ++k)
+                        for (int k = 0; k < GB_SEG; ++k)
                             if ((pend >> k) & 1u) {
                                 const uint32_t e = atomicAdd(&s_nr, 1u);
                                 if (e < GB_RARE) {
@@ -539,19 +534,19 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
                     } while (__syncthreads_or(pend != 0));
                 }
 #pragma unroll
-                for (int k = 0; k < KK; ++k)
+                for (int k = 0; k < GB_SEG; ++k)
                     cur[k] = sZ[cell[k]];
 #pragma unroll
-                for (int k = 0; k < KK; ++k) {
+                for (int k = 0; k < GB_SEG; ++k) {
                     eq[k] = zk[k] == cur[k];
                     if (eq[k] && low[k])
                         sId[cell[k]] = OWM_NONE;
                 }
                 __syncthreads();
 #pragma unroll
-                for (int k = 0; k < KK; ++k)
+                for (int k = 0; k < GB_SEG; ++k)
                     if (eq[k]) {
-                        const uint32_t i = id0[k / GB_SEG] + (cw[k] & GRID_SLOT_MASK);
+                        const uint32_t i = id0 + (cw[k] & GRID_SLOT_MASK);
                         // (idle lanes may point anywhere: theirs is the spare cell)
                         if (!TREE)
                             atomicMin(&sId[cell[k]], i);
@@ -579,7 +574,7 @@ __device__ __forceinline__ void bin_range(const GridDev &G, uint32_t t, uint32_t
     }
 }
 
-template <int NT, int TWO, bool TREE>
+template <int NT, bool TREE>
 __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_t t1,
                                                  uint32_t item0, uint32_t items, uint32_t cells)
 {
@@ -596,7 +591,7 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
     const uint32_t t = find_entry(G.item_off, t0, t1, item, &s_t);
     const GridTile &T = G.tiles[t];
     const uint32_t q = item - T.item_off, part = q % T.split;
-    bin_range<NT, TWO, TREE, false>(G, t, item, cells, (uint32_t)((uint64_t)T.nst * part / T.split),
+    bin_range<NT, TREE, false>(G, t, item, cells, (uint32_t)((uint64_t)T.nst * part / T.split),
                                     (uint32_t)((uint64_t)T.nst * (part + 1) / T.split), nullptr);
 }
 
@@ -632,7 +627,7 @@ __global__ __launch_bounds__(NT) void k_grid_heavy(GridDev G, uint32_t cap,
         const uint4 v = H.q[e];
         uint32_t *own = H.own + 4 * v.w;
         const uint32_t t = own[3];
-        bin_range<NT, 1, TREE, true>(G, t, v.x, cells, v.y, v.z,
+        bin_range<NT, TREE, true>(G, t, v.x, cells, v.y, v.z,
                                      H.cells + (uint64_t)e * cells);
         // the last of the item's adds them up: every wave's stores have reached
         // the L2, the fence makes them visible beyond this XCD
@@ -1059,16 +1054,16 @@ void launch_grid_bin(hipStream_t s, const GridDev &G, uint32_t t0, uint32_t t1, 
     const bool wide = cells > 1024 || items <= 1024;
     const dim3 grid(g), block(wide ? 512 : 256);
     if (G.zi && wide)
-        hipLaunchKernelGGL((k_grid_bin<512, 1, true>), grid, block, BIN_LDS(cells), s, G, t0, t1,
+        hipLaunchKernelGGL((k_grid_bin<512, true>), grid, block, BIN_LDS(cells), s, G, t0, t1,
                            item0, items, cells);
     else if (G.zi)
-        hipLaunchKernelGGL((k_grid_bin<256, 1, true>), grid, block, BIN_LDS(cells), s, G, t0, t1,
+        hipLaunchKernelGGL((k_grid_bin<256, true>), grid, block, BIN_LDS(cells), s, G, t0, t1,
                            item0, items, cells);
     else if (wide)
-        hipLaunchKernelGGL((k_grid_bin<512, 1, false>), grid, block, BIN_LDS(cells), s, G, t0, t1,
+        hipLaunchKernelGGL((k_grid_bin<512, false>), grid, block, BIN_LDS(cells), s, G, t0, t1,
                            item0, items, cells);
     else
-        hipLaunchKernelGGL((k_grid_bin<256, 1, false>), grid, block, BIN_LDS(cells), s, G, t0, t1,
+        hipLaunchKernelGGL((k_grid_bin<256, false>), grid, block, BIN_LDS(cells), s, G, t0, t1,
                            item0, items, cells);
 }
 
@@ -1116,10 +1111,10 @@ hipError_t grid_kernels_init()
         {(const void *)k_grid_part<false, 12>, (12 << 12) + (GRID_MAX_BUCKETS + 1) * 4},
         {(const void *)k_grid_part<true, 12>, (12 << 12) + (GRID_MAX_BUCKETS + 1) * 4},
         {(const void *)k_grid_part<false, 13>, (12 << 13) + (GRID_MAX_BUCKETS + 1) * 4},
-        {(const void *)k_grid_bin<256, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
-        {(const void *)k_grid_bin<512, 1, false>, BIN_LDS(GRID_MAX_CELLS)},
-        {(const void *)k_grid_bin<256, 1, true>, BIN_LDS(GRID_MAX_CELLS)},
-        {(const void *)k_grid_bin<512, 1, true>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_bin<256, false>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_bin<512, false>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_bin<256, true>, BIN_LDS(GRID_MAX_CELLS)},
+        {(const void *)k_grid_bin<512, true>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_heavy<512, false>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_heavy<512, true>, BIN_LDS(GRID_MAX_CELLS)},
         {(const void *)k_grid_windows, GRID_MAX_WIN_CELLS * 16}};

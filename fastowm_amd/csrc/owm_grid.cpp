@@ -143,7 +143,9 @@ static bool make_plan(owm_ctx *ctx, const owm_tile *tiles, uint32_t n_tiles,
     // the device often (a workgroup has a CU to itself): partition and bins, 100M
     // points in runs of three 654 + 882 us with 4096, 733 + 595 with 8192; 120M in
     // runs of eight 805 + 637 and 869 + 492; 40M in runs of six 252 + 251 and 308 +
-    // 199; 20M in runs of twenty 123 + 85 and 173 + 70.
+    // 199; 20M in runs of twenty 123 + 85 and 173 + 70.  341 buckets and more share a
+    // sort tile of 4096 in runs of twelve and less, between the eight where the larger
+    // tiles win and the twenty where they lose.
     bool brief = launch_points >= (48u << 20);
     for (const GridTile &T : raw)
         brief = brief && (T.n == 0 || T.nb > 341);

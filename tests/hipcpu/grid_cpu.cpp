@@ -135,9 +135,9 @@ int main(int argc, char **argv)
         if (!kind && k != (const void *)&k_grid_prep && k != (const void *)&k_flags_out && *err)
             kind = 1;
         const bool heavy = k == (const void *)&k_grid_heavy<512, false>;
-        if ((head[1] == 4 && k == (const void *)&k_grid_bin<512, 1, false>) || (head[1] >= 4 && heavy))
+        if ((head[1] == 4 && k == (const void *)&k_grid_bin<512, false>) || (head[1] >= 4 && heavy))
             const_cast<GridDev *>((const GridDev *)arg)->list_cap = 600;
-        if (head[1] == 2 && k == (const void *)&k_grid_bin<512, 1, false>)
+        if (head[1] == 2 && k == (const void *)&k_grid_bin<512, false>)
             for (uint32_t t = 0; t < T; ++t)
                 const_cast<GridTile *>(((const GridDev *)arg)->tiles)[t].heavy_cap = 2;
     };
