@@ -34,13 +34,18 @@ constexpr int gp_threads(int lsp) { return lsp == 13 ? 1024 : 512; }
 constexpr uint32_t KEY_NONE = 0x7FFFFFFFu, KEY_RARE = 0x80000000u;
 
 // Table entry whose range of off[] holds v, found by the whole workgroup at
-// once (off[t] <= v < off[t + 1]; s_t: one shared word).
-__device__ __forceinline__ uint32_t find_entry(const uint32_t *__restrict__ off, uint32_t t0,
+// once (off[t] <= v < off[t + 1]; s_t: one shared word): each thread's look, then what
+// one of them found.
+__device__ __forceinline__ void look_for_entry(const uint32_t *__restrict__ off, uint32_t t0,
                                                uint32_t t1, uint32_t v, uint32_t *s_t)
 {
     for (uint32_t t = t0 + threadIdx.x; t < t1; t += blockDim.x)
         if (off[t] <= v && v < off[t + 1])
             *s_t = t;
+}
+
+__device__ __forceinline__ uint32_t entry_found(const uint32_t *s_t)
+{
     __syncthreads();
     return __builtin_amdgcn_readfirstlane(*s_t);
 }
@@ -143,7 +148,8 @@ __global__ __launch_bounds__(gp_threads(LSP), LSP == 13 ? 4 : 6) void k_grid_par
     // which has no part in finding the tile of most launches)
     if (tid == GP_NT - 1)
         s_stop = load_past_caches(G.err, GRID_STOP_PART);
-    const uint32_t t = find_entry(G.st_off, 0, G.ntiles, u, &s_t);
+    look_for_entry(G.st_off, 0, G.ntiles, u, &s_t);
+    const uint32_t t = entry_found(&s_t);
     if (s_stop)
         return;
     const GridTile &T = G.tiles[t];
@@ -579,8 +585,7 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
                                                  uint32_t item0, uint32_t items, uint32_t cells)
 {
     __shared__ uint32_t s_t;
-    if (G.err[GRID_STOP_PART])
-        return;
+    const uint32_t stop = G.err[GRID_STOP_PART];
     // consecutive items (neighbouring buckets, whose runs share cache lines)
     // on one XCD: workgroups go round the eight XCDs
     const uint32_t per = (items + 7u) / 8u;
@@ -588,7 +593,10 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
     if (rel >= items)
         return;
     const uint32_t item = item0 + rel;
-    const uint32_t t = find_entry(G.item_off, t0, t1, item, &s_t);
+    look_for_entry(G.item_off, t0, t1, item, &s_t);
+    if (stop)  // (its load went beside the table's)
+        return;
+    const uint32_t t = entry_found(&s_t);
     const GridTile &T = G.tiles[t];
     const uint32_t q = item - T.item_off, part = q % T.split;
     bin_range<NT, TREE, false>(G, t, item, cells, (uint32_t)((uint64_t)T.nst * part / T.split),
@@ -726,11 +734,13 @@ __global__ __launch_bounds__(GW_NT) void k_grid_windows(GridDev G, const double 
     __shared__ int sx0[32], sx1[32], sy0[32], sy1[32];
     __shared__ uint2 sSeg[GW_SEGS];
     const uint32_t tid = threadIdx.x;
-    if (G.err[GRID_STOP_PART] | G.err[GRID_STOP_BIN] | G.err[GRID_STOP_HEAVY])
-        return;
+    const uint32_t stop = G.err[GRID_STOP_PART] | G.err[GRID_STOP_BIN] | G.err[GRID_STOP_HEAVY];
     if (tid == 0)
         s_nseg = 0;
-    const uint32_t t = find_entry(G.blk_off, 0, G.ntiles, blockIdx.x, &s_t);
+    look_for_entry(G.blk_off, 0, G.ntiles, blockIdx.x, &s_t);
+    if (stop)
+        return;
+    const uint32_t t = entry_found(&s_t);
     const GridTile &T = G.tiles[t];
     const uint32_t lb = T.lbw, bw = 1u << lb;
     const uint32_t q0 = blockIdx.x - T.blk_off, bj = q0 / T.nblkx, bi = q0 - bj * T.nblkx;
@@ -949,10 +959,9 @@ __global__ __launch_bounds__(256) void k_grid_cells(GridDev G)
 {
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (*G.err)  // (this launch sets none)
-        return;
+    const uint32_t stop = *G.err;  // (this launch sets none)
     for (uint32_t c = blockIdx.x * 4 + w; c < G.ngcell; c += gridDim.x * 4) {
-        if (G.cell_flag[c])
+        if (G.cell_flag[c] | stop)
             continue;
         const uint32_t t = owm_find_tile(G.gcell_off, G.ntiles, c);
         const GridTile &T = G.tiles[t];
