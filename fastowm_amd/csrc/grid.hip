@@ -600,7 +600,7 @@ __global__ __launch_bounds__(NT) void k_grid_bin(GridDev G, uint32_t t0, uint32_
     const GridTile &T = G.tiles[t];
     const uint32_t q = item - T.item_off, part = q % T.split;
     bin_range<NT, TREE, false>(G, t, item, cells, (uint32_t)((uint64_t)T.nst * part / T.split),
-                                    (uint32_t)((uint64_t)T.nst * (part + 1) / T.split), nullptr);
+                               (uint32_t)((uint64_t)T.nst * (part + 1) / T.split), nullptr);
 }
 
 struct CellAgg {
@@ -635,8 +635,7 @@ __global__ __launch_bounds__(NT) void k_grid_heavy(GridDev G, uint32_t cap,
         const uint4 v = H.q[e];
         uint32_t *own = H.own + 4 * v.w;
         const uint32_t t = own[3];
-        bin_range<NT, TREE, true>(G, t, v.x, cells, v.y, v.z,
-                                     H.cells + (uint64_t)e * cells);
+        bin_range<NT, TREE, true>(G, t, v.x, cells, v.y, v.z, H.cells + (uint64_t)e * cells);
         // the last of the item's adds them up: every wave's stores have reached
         // the L2, the fence makes them visible beyond this XCD
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
